@@ -332,6 +332,23 @@ static uint64_t morton3(int x, int y, int z) {
     return spread((uint64_t)x) | spread((uint64_t)y) << 1 | spread((uint64_t)z) << 2;
 }
 
+// Bound on the distance between points of two tets of the near zone: their
+// centroids lie in cubes at most one apart per axis, i.e. within two cube
+// edges per axis.
+static double near_reach(const HostGeometry &g) {
+    double r2 = 0.0;  // largest centroid-to-vertex distance of a tet, squared
+    for (int t = 0; t < g.N; ++t) {
+        const double *p = &g.tcoord[12 * (size_t)t];
+        double c[3];
+        for (int i = 0; i < 3; ++i) c[i] = (p[i] + p[3 + i] + p[6 + i] + p[9 + i]) / 4;
+        for (int a = 0; a < 4; ++a) {
+            const double dx = p[3 * a] - c[0], dy = p[3 * a + 1] - c[1], dz = p[3 * a + 2] - c[2];
+            r2 = std::max(r2, dx * dx + dy * dy + dz * dz);
+        }
+    }
+    return 2.0 * std::sqrt(3.0) * g.box_delta + 2.0 * std::sqrt(r2);
+}
+
 static void create_operator(scadyn_operator *op, const scadyn_mesh &mesh, const scadyn_opts &opts, double k) {
     if (!(k > 0.0)) fail(SCADYN_ERR_ARG, "wavenumber must be positive");
     op->opts = opts;
@@ -443,14 +460,14 @@ static void create_operator(scadyn_operator *op, const scadyn_mesh &mesh, const 
     }
     // ---- near zone
     {
-        cd *d_G = M.alloc<cd>(27 * 27 * 27);
+        cd *d_G = M.alloc<cd>(27 * 125);
         launch_pg_table(d_G, gd, k, s);
         int *d_PT = M.upload(op->np.T, s);
         int *d_PB = M.upload(op->np.B, s);
         uint8_t *d_PO = M.upload(op->np.off, s);
         op->d_blocks = M.alloc<cf>((size_t)op->nblocks * 9);
         launch_near_blocks(d_PT, d_PB, d_PO, op->nblocks, op->d_tcoord, op->d_vol, op->d_param, op->d_S4, d_G, k,
-                           op->d_blocks, s);
+                           near_reach(g), op->d_blocks, s);
         op->d_row_start = M.upload(op->np.row_start, s);
         op->d_ent_col = M.upload(op->np.ent_col, s);
         op->d_ent_blk = M.upload(op->np.ent_blk, s);

@@ -119,6 +119,11 @@ __device__ inline void tet_face(const double *tc, int f, v3 &p0, v3 &p1, v3 &p2)
         default: p0 = tet_vertex(tc, 0); p1 = tet_vertex(tc, 2); p2 = tet_vertex(tc, 1); break;
     }
 }
+// corner c of face f by the same table, for an f and c that differ by lane: two
+// bits a corner
+__device__ inline v3 face_corner(const double *tc, int f, int c) {
+    return tet_vertex(tc, (0x634b39 >> (2 * (3 * f + c))) & 3);
+}
 // tri_n_vectors (src/common.f90:326-339)
 __device__ inline v3 tri_normal(v3 p0, v3 p1, v3 p2) {
     v3 n = cross3(sub3(p1, p0), sub3(p2, p0));
@@ -146,84 +151,167 @@ __device__ inline v3 tet_point(const double *tc, double x1, double x2, double x3
     return p;
 }
 
-// ---- analytical integrals of 1/R and R over a flat triangle -----------------
-// (src/singularity_subtraction.f90:15-108), returns K1 = int 1/R dS, K2 = int R dS
-__device__ void analytic_tri(v3 p0, v3 p1, v3 p2, v3 n, v3 r, double &K1, double &K2) {
-    v3 p[3] = {p0, p1, p2};
-    const double w0 = dot3(sub3(r, p0), n);
-    const double aw0 = fabs(w0);
-    double k1 = 0.0;
-    double tl[3], I1[3];
-    const int e1[3] = {1, 2, 0}, e2[3] = {2, 0, 1};
+// ---- near-zone kernels -------------------------------------------------------
+// The elementary functions of these kernels, each within about an ulp: seeds
+// from the hardware reciprocals, refined; logarithm and arctangent as series in
+// the square of a reduced argument (economised on Chebyshev nodes, relative
+// error below 3e-18).  The library's versions cost two to four times the
+// instructions for ranges and special cases that do not occur here.
+__device__ inline double fast_div(double n, double d) {
+    double r = __builtin_amdgcn_rcp(d);
+    r = fma(r, fma(-d, r, 1.0), r);
+    r = fma(r, fma(-d, r, 1.0), r);
+    const double q = n * r;
+    return fma(fma(-d, q, n), r, q);
+}
+__device__ inline double fast_sqrt(double x) {
+    x = fmax(x, 1.0e-290);  // 0 counts as 1e-145
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    const double r = fma(-h, g, 0.5);
+    g = fma(g, r, g);
+    h = fma(h, r, h);
+    return fma(fma(-g, g, x), h, g);
+}
+__device__ inline double fast_rsqrt(double x) {
+    double y = __builtin_amdgcn_rsq(x);
+    y = fma(0.5 * y, fma(-x * y, y, 1.0), y);
+    return fma(0.5 * y, fma(-x * y, y, 1.0), y);
+}
+// log(n / d), n, d > 0: 2 atanh((n' - d')/(n' + d')) of the mantissas, their
+// ratio brought into [1/sqrt 2, sqrt 2]
+__device__ inline double log_ratio(double n, double d) {
+    const double C[9] = {1.0,
+                         0.3333333333333333,
+                         0.20000000000003748,
+                         0.1428571428440936,
+                         0.11111111338494353,
+                         0.09090886866684009,
+                         0.07693580563610432,
+                         0.06624379288610822,
+                         0.06631072256545831};
+    double mn = __builtin_amdgcn_frexp_mant(n);
+    const double md = __builtin_amdgcn_frexp_mant(d);
+    int e = __builtin_amdgcn_frexp_exp(n) - __builtin_amdgcn_frexp_exp(d);
+    const bool up = mn > 1.4142135623730951 * md, dn = 1.4142135623730951 * mn < md;
+    mn *= up ? 0.5 : (dn ? 2.0 : 1.0);
+    e += up ? 1 : (dn ? -1 : 0);
+    const double t = fast_div(mn - md, mn + md), z = t * t;
+    double q = C[8];
+#pragma unroll
+    for (int i = 7; i >= 0; --i) q = fma(q, z, C[i]);
+    const double ed = (double)e;
+    // ln 2 in two parts, the first exact in 33 bits
+    return fma(ed, 0.693147180369123816490, fma(ed, 1.90821492927058770002e-10, 2.0 * t * q));
+}
+// atan2(y, x) for y >= 0
+__device__ inline double atan2_pos(double y, double x) {
+    const double C[13] = {1.0,
+                          -0.33333333333333326,
+                          0.19999999999997015,
+                          -0.14285714285329706,
+                          0.11111111085321958,
+                          -0.09090908059025865,
+                          0.07692281099819559,
+                          -0.06666205258255166,
+                          0.0587683398793194,
+                          -0.05217312467523656,
+                          0.04499500298415364,
+                          -0.03338781452398182,
+                          0.015113754999461897};
+    const double ax = fabs(x);
+    const double lo = fmin(y, ax), hi = fmax(y, ax);
+    const bool mid = lo > 0.41421356237309503 * hi;  // beyond pi/8: from pi/4
+    const double t = fast_div(mid ? lo - hi : lo, mid ? hi + lo : hi), z = t * t;
+    double q = C[12];
+#pragma unroll
+    for (int i = 11; i >= 0; --i) q = fma(q, z, C[i]);
+    q = fma(t, q, mid ? 0.25 * PI_D : 0.0);
+    q = y > ax ? 0.5 * PI_D - q : q;
+    return x < 0.0 ? PI_D - q : q;
+}
+
+// exp(ikR)/(4 pi R) - (1/R - k^2 R / 2)/(4 pi), the smooth remainder of the
+// singularity subtraction (src/singularity_subtraction.f90:146-152), from
+// d2 = R^2.  With x = kR the remainder is
+//   k/(4 pi) [ (cos x - 1 + x^2/2)/x  +  i sin(x)/x ],
+// two power series in x^2 (the real one times x).  Summed as series they have
+// neither the cancellation of the closed form nor its sincos and divisions
+// (about 45 instructions instead of 150), and their value at R = 0 is the
+// limit ik/(4 pi) that the reference takes below its cut-off distance.
+// SER terms are exact to double rounding for x up to SERIES_X (11 terms: the
+// first one left out is 1.5^22/23! = 3e-19; 17 terms: 4^34/35! = 3e-20); the
+// general variant takes sincos beyond.
+constexpr double SERIES_X_SHORT = 1.5, SERIES_X_LONG = 4.0;
+constexpr int SERIES_SHORT = 11, SERIES_LONG = 17;
+constexpr double inv_factorial(int n) {
+    double f = 1.0;
+    for (int i = 2; i <= n; ++i) f *= (double)i;
+    return 1.0 / f;
+}
+template <int SER, bool GENERAL>
+__device__ inline cd smooth_green(double d2, double k, double k4pi) {
+    const double z = k * k * d2;
+    const double x = fast_sqrt(z);
+    if (GENERAL && x > SERIES_X_LONG) {
+        double s, c;
+        sincos(x, &s, &c);
+        const double w = k4pi / x;
+        return cmk(w * (c - 1.0 + 0.5 * z), w * s);
+    }
+    double re = 0.0, im = 0.0;
+#pragma unroll
+    for (int q = SER - 1; q >= 0; --q) im = fma(im, -z, inv_factorial(2 * q + 1));
+#pragma unroll
+    for (int q = SER - 3; q >= 0; --q) re = fma(re, -z, inv_factorial(2 * q + 4));
+    return cmk(k4pi * (x * z * re), k4pi * im);
+}
+
+// One edge of a face as the integrals over the face see it: unit direction s,
+// in-plane outward normal m = s x n, length.
+struct EdgeGeom {
+    v3 s, m;
+    double len;
+};
+// A face opposite a vertex: corners, unit normal, twice its area, edges in the
+// order (1,2), (2,0), (0,1) of its corners.
+struct FaceGeom {
+    v3 p[3], n;
+    double area2;
+    EdgeGeom e[3];
+};
+
+// int 1/R dS (K1) and int R dS (K2) over a flat triangle seen from r: the
+// closed forms of src/singularity_subtraction.f90:15-108 (Wilton et al. 1984).
+// The sum over the edges of the arctangent terms is the solid angle of the
+// triangle, taken with one atan2 (Van Oosterom and Strackee 1983) instead of
+// six atan; it multiplies the height |w0| and is left out below the
+// reference's height threshold.
+__device__ inline void tri_integrals(const FaceGeom &f, v3 r, double &K1, double &K2) {
+    const v3 d0 = sub3(f.p[0], r), d1 = sub3(f.p[1], r), d2 = sub3(f.p[2], r);
+    const v3 d[3] = {d0, d1, d2};
+    const double R[3] = {fast_sqrt(dot3(d0, d0)), fast_sqrt(dot3(d1, d1)), fast_sqrt(dot3(d2, d2))};
+    const double w0 = -dot3(d0, f.n);
+    const double aw0 = fabs(w0), w02 = w0 * w0;
+    double k1 = 0.0, k2 = 0.0;
 #pragma unroll
     for (int l = 0; l < 3; ++l) {
-        v3 pl1 = p[e1[l]], pl2 = p[e2[l]];
-        v3 slv = sub3(pl2, pl1);
-        double nsl = sqrt(dot3(slv, slv));
-        v3 sl = mk3(slv.x / nsl, slv.y / nsl, slv.z / nsl);
-        v3 ml = cross3(sl, n);
-        v3 pl1mr = sub3(pl1, r);
-        double tl0 = dot3(pl1mr, ml);
-        v3 pl2mpl1 = sub3(pl2, pl1);
-        double ll = sqrt(dot3(pl2mpl1, pl2mpl1));
-        double sml = dot3(pl1mr, sl);
-        double spl = sml + ll;
-        v3 rmplm1 = sub3(r, pl2);
-        double Rpl = sqrt(dot3(rmplm1, rmplm1));
-        double Rml = sqrt(dot3(pl1mr, pl1mr));
-        double R0l = sqrt(tl0 * tl0 + w0 * w0);
-        double Km3 = 0.0;
-        if (aw0 > 1.0e-10) {
-            double Bl = atan((tl0 * spl) / (R0l * R0l + aw0 * Rpl)) -
-                        atan((tl0 * sml) / (R0l * R0l + aw0 * Rml));
-            Km3 = 1.0 / aw0 * Bl;
-        }
-        double Il;
-        if ((Rml + sml) > (Rpl - spl))
-            Il = log(fabs((Rpl + spl) / (Rml + sml)));
-        else
-            Il = log(fabs((Rml - sml) / (Rpl - spl)));
-        k1 = k1 + 1.0 / (-1.0 + 2.0) * (-1.0 * w0 * w0 * Km3 + tl0 * Il);
-        tl[l] = tl0;
-        I1[l] = 1.0 / (1.0 + 1.0) * (spl * Rpl - sml * Rml + 1.0 * R0l * R0l * Il);
+        const int a = (l + 1) % 3, b = (l + 2) % 3;
+        const EdgeGeom &e = f.e[l];
+        const double t0 = dot3(d[a], e.m), sm = dot3(d[a], e.s), sp = sm + e.len;
+        const double Rm = R[a], Rp = R[b];
+        // of the two equal forms of the logarithm, the one without cancellation
+        const bool fwd = (Rm + sm) > (Rp - sp);
+        const double I = log_ratio(fabs(fwd ? Rp + sp : Rm - sm), fabs(fwd ? Rm + sm : Rp - sp));
+        k1 = fma(t0, I, k1);
+        k2 = fma(t0, 0.5 * (sp * Rp - sm * Rm + (t0 * t0 + w02) * I), k2);
+    }
+    if (aw0 > 1.0e-10) {
+        const double D = R[0] * R[1] * R[2] + dot3(d0, d1) * R[2] + dot3(d1, d2) * R[0] + dot3(d2, d0) * R[1];
+        k1 -= aw0 * 2.0 * atan2_pos(aw0 * f.area2, D);
     }
     K1 = k1;
-    K2 = 1.0 / (1.0 + 2.0) * (1.0 * w0 * w0 * k1 + (tl[0] * I1[0] + tl[1] * I1[1] + tl[2] * I1[2]));
-}
-
-// G - (1/R - k^2 R / 2)/(4 pi), the smooth remainder (singularity_subtraction.f90:146-152)
-__device__ inline cd green_remainder(double R, double k) {
-    double f = 1.0 / (4 * PI_D) * 1.0 * 1.0 * (1.0 / R);
-    f = f + 1.0 / (4 * PI_D) * (k * k) * (-0.5) * R;
-    cd G0 = green(R, k);
-    return cmk(G0.x - f, G0.y);
-}
-
-// int_V G(rf, r') dV' over tet B (singularity_subtraction_int_V_G), 24-point rule
-__device__ cd int_V_G(v3 rf, double k, const double *tcB, double vB, double cut) {
-    cd intR = cmk(0, 0);
-    for (int i = 0; i < 24; ++i) {
-        v3 pb = tet_point(tcB, c_tet24_p[3 * i], c_tet24_p[3 * i + 1], c_tet24_p[3 * i + 2]);
-        double wb = c_tet24_w[i] * 6.0 * vB;
-        double RR = dist3(pb, rf);
-        cd II = (RR < cut) ? cmk(0.0, k / (4.0 * PI_D)) : green_remainder(RR, k);
-        intR = cadd(intR, cscale(II, wb));
-    }
-    double r4a = 0.0, r4b = 0.0;
-#pragma unroll
-    for (int f = 0; f < 4; ++f) {
-        v3 p0, p1, p2;
-        tet_face(tcB, f, p0, p1, p2);
-        v3 n = tri_normal(p0, p1, p2);
-        double K1, K2;
-        analytic_tri(p0, p1, p2, n, rf, K1, K2);
-        double a1 = dot3(n, sub3(p0, rf));
-        r4a = r4a + a1 * K1 * 0.5;
-        r4b = r4b + a1 * K2 * 0.25;
-    }
-    double f2 = 1.0 / (4 * PI_D) * 1.0 * 1.0 * r4a;
-    f2 = f2 + 1.0 / (4 * PI_D) * (k * k) * (-0.5) * r4b;
-    return cmk(intR.x + f2, intR.y);
+    K2 = (w02 * k1 + k2) * (1.0 / 3.0);
 }
 
 // ---- projection coefficients ----------------------------------------------
@@ -311,27 +399,29 @@ __global__ void k_fg_octant(const cd *__restrict__ F, cd *__restrict__ fg, int L
 }
 
 // ---- near-zone G between box nodes for the 27 cube offsets ---------------------
-// Gtab[off][i][j] = G(node_i of test box, node_j of basis box), 0 when the
-// nodes coincide (compute_pG, src/precorrection.f90:21-46)
+// Gtab[off][t] = G(node of the test box, node of the basis box) for the node
+// difference (tx, ty, tz) - 2, t = tx + 5 ty + 25 tz, plus the offset between
+// the boxes; 0 when the nodes coincide (compute_pG, src/precorrection.f90:21-46;
+// the 27 x 27 matrix of an offset has these 125 values)
 __global__ void k_pg_table(cd *__restrict__ Gtab, GridDesc gd, double k) {
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= 27 * 27 * 27) return;
-    const int j = e % 27, i = (e / 27) % 27, off = e / 729;
-    const int ox = off % 3 - 1, oy = (off / 3) % 3 - 1, oz = off / 9 - 1;
+    if (e >= 27 * 125) return;
+    const int t = e % 125, off = e / 125;
     // test box based at node (0,0,0) of a reference cube (2,2,2), basis box at
     // (2+2ox, 2+2oy, 2+2oz); coordinates as min + delta*index
-    int ti[3] = {2 + i % 3, 2 + (i / 3) % 3, 2 + i / 9};
-    int bi[3] = {2 + 2 * ox + j % 3, 2 + 2 * oy + (j / 3) % 3, 2 + 2 * oz + j / 9};
-    cd v = cmk(0, 0);
-    if (!(ti[0] == bi[0] && ti[1] == bi[1] && ti[2] == bi[2])) {
-        double d2 = 0;
-        for (int c = 0; c < 3; ++c) {
-            double a = (gd.min[c] + gd.delta * ti[c]) - (gd.min[c] + gd.delta * bi[c]);
-            d2 += a * a;
-        }
-        v = green(sqrt(d2), k);
+    const int dt[3] = {t % 5 - 2, (t / 5) % 5 - 2, t / 25 - 2};
+    const int o[3] = {off % 3 - 1, (off / 3) % 3 - 1, off / 9 - 1};
+    bool same = true;
+    double d2 = 0;
+    for (int c = 0; c < 3; ++c) {
+        // a pair of nodes with this difference: test node i, basis node i - dt
+        const int i = dt[c] > 0 ? dt[c] : 0, j = i - dt[c];
+        const int ti = 2 + i, bi = 2 + 2 * o[c] + j;
+        same = same && ti == bi;
+        const double a = (gd.min[c] + gd.delta * ti) - (gd.min[c] + gd.delta * bi);
+        d2 += a * a;
     }
-    Gtab[e] = v;
+    Gtab[e] = same ? cmk(0, 0) : green(sqrt(d2), k);
 }
 
 __device__ inline double wave_sum(double v) {
@@ -339,126 +429,225 @@ __device__ inline double wave_sum(double v) {
     return v;
 }
 
-// One wave64 per stored block; 4 blocks per workgroup.
-__global__ __launch_bounds__(256) void k_near_blocks(
+// quadrature point and rule weight
+struct __attribute__((aligned(16))) RulePoint {
+    double x, y, z, w;
+};
+// Operands of one near-zone block in LDS.
+struct NearLds {
+    FaceGeom fb[4];             // faces of the basis tet
+    double tn[4][3], bn[4][3];  // face normals of the test and basis tet
+    double ta2[4];              // twice the areas of the test tet's faces
+    RulePoint tq[24], bq[24];   // volume rule points of both tets
+    RulePoint ts[28], bs[28];   // surface rule points, 7 per face
+    cd SB[108], u[108];         // projection of the basis tet; G S_B
+    cd s[16], form[10];         // face-pair integrals; bilinear forms of the correction
+};
+
+// One block of the near-zone matrix per wave (workgroups of one wave): the
+// 3 x 3 Galerkin block of test tet T and basis tet B with the singularity
+// subtracted, minus what the grid already gives (src/precorrection.f90:182-258,
+// :729-806).  The kernel is bound by FP64 vector instructions: 1,360 smooth
+// kernel values and 208 triangle integrals per block.  So the work is laid out
+// flat over the lanes: 24 x 24 volume pairs in 9 rounds, the 16 face pairs of
+// 7 x 7 points on 4 lanes each, and all 208 triangle integrals together in 4
+// rounds; points, normals and edges are computed once per block into LDS.
+// Measured at 43,248 tets (3.22 M blocks, ka 2): 23.2 ms, 3,350 vector
+// instructions per block at 83% of the issue rate.  With one quadrature point or
+// face pair per lane (24 and 112 of 64 and 128 lanes busy), closed-form
+// remainders and six atan per triangle it took 136.2 ms, with the flat layout and
+// the library's elementary functions 33.2 ms.
+template <int SER, bool GENERAL>
+__global__ __launch_bounds__(64, 4) void k_near_blocks(
     const int *__restrict__ PT, const int *__restrict__ PB, const uint8_t *__restrict__ POFF,
-    long long P, const double *__restrict__ tcoord, const double *__restrict__ vol,
+    const double *__restrict__ tcoord, const double *__restrict__ vol,
     const cd *__restrict__ param, const cd *__restrict__ S4, const cd *__restrict__ Gtab, double k,
     cf *__restrict__ blocks) {
-    __shared__ cd u_s[4][4][27];  // per wave: G * S_B channels
-    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const long long p0 = (long long)blockIdx.x * 4 + wv;
-    const bool valid = p0 < P;
-    const long long p = valid ? p0 : P - 1;  // idle waves recompute the last block, never store
+    __shared__ NearLds L;
+    const int lane = threadIdx.x;
+    const size_t p = blockIdx.x;
     const int T = PT[p], B = PB[p], off = POFF[p];
     const double *tcT = tcoord + 12 * (size_t)T;
     const double *tcB = tcoord + 12 * (size_t)B;
     const double vT = vol[T], vB = vol[B];
-    const cd *ST = S4 + (size_t)T * 108, *SB = S4 + (size_t)B * 108;
-    const cd *G = Gtab + (size_t)off * 729;
+    const cd *ST = S4 + (size_t)T * 108;
+    const cd *G = Gtab + off * 125;
+    const double k4pi = k / (4.0 * PI_D), i4pi = 1.0 / (4.0 * PI_D), k2 = k * k;
 
-    // --- correction: u_c = G S_B[c]  (precorrect_const, src/precorrection.f90:50-82)
-    for (int e = lane; e < 108; e += 64) {
-        const int i = e % 27, ch = e / 27;
-        cd acc = cmk(0, 0);
-        for (int j = 0; j < 27; ++j) cfma(acc, G[i * 27 + j], SB[j * 4 + ch]);
-        u_s[wv][ch][i] = acc;
+    // --- points, normals, edges, S_B
+    for (int e = lane; e < 108; e += 64) L.SB[e] = S4[(size_t)B * 108 + e];
+    if (lane < 48) {
+        const int q = lane % 24;
+        const v3 r = tet_point(lane < 24 ? tcT : tcB, c_tet24_p[3 * q], c_tet24_p[3 * q + 1], c_tet24_p[3 * q + 2]);
+        (lane < 24 ? L.tq : L.bq)[q] = {r.x, r.y, r.z, c_tet24_w[q]};
+    }
+    if (lane < 56) {
+        const int q = lane % 28, f = q / 7, i = q % 7;
+        const double *tc = lane < 28 ? tcT : tcB;
+        const v3 r = tri_point(face_corner(tc, f, 0), face_corner(tc, f, 1), face_corner(tc, f, 2), c_tri7_p[2 * i],
+                               c_tri7_p[2 * i + 1]);
+        (lane < 28 ? L.ts : L.bs)[q] = {r.x, r.y, r.z, c_tri7_w[i]};
+    }
+    if (lane < 16) {
+        // lanes 0-3 the test tet's faces, 4-15 the edges of the basis tet's
+        // (edge l from corner l + 1 to corner l + 2 of its face)
+        const int f = lane < 4 ? lane : (lane - 4) / 3, l = (lane + 2) % 3;
+        const double *tc = lane < 4 ? tcT : tcB;
+        const v3 q0 = face_corner(tc, f, 0), q1 = face_corner(tc, f, 1), q2 = face_corner(tc, f, 2);
+        const v3 cr = cross3(sub3(q1, q0), sub3(q2, q0));
+        const double cc = dot3(cr, cr), ci = fast_rsqrt(cc);
+        const v3 n = mul3(cr, ci);
+        const double a2 = cc * ci;  // twice the area
+        if (lane < 4) {
+            L.tn[f][0] = n.x, L.tn[f][1] = n.y, L.tn[f][2] = n.z;
+            L.ta2[f] = a2;
+        } else {
+            const v3 ev = sub3(face_corner(tc, f, l == 0 ? 2 : l - 1), face_corner(tc, f, l == 2 ? 0 : l + 1));
+            const double ee = dot3(ev, ev), ei = fast_rsqrt(ee);
+            EdgeGeom &e = L.fb[f].e[l];
+            e.s = mul3(ev, ei);
+            e.m = cross3(e.s, n);
+            e.len = ee * ei;
+            L.fb[f].p[l] = face_corner(tc, f, l);
+            if (l == 0) {
+                L.fb[f].n = n;
+                L.bn[f][0] = n.x, L.bn[f][1] = n.y, L.bn[f][2] = n.z;
+                L.fb[f].area2 = a2;
+            }
+        }
     }
     __syncthreads();
-    // 10 bilinear forms: a = S_T . u_0 ; corr2(a,b) = D_a,T . u_{1+b}
-    cd cform = cmk(0, 0);
-    if (lane < 10) {
-        const int ca = lane == 0 ? 0 : 1 + (lane - 1) / 3;
-        const int cb = lane == 0 ? 0 : 1 + (lane - 1) % 3;
-        for (int i = 0; i < 27; ++i) cfma(cform, ST[i * 4 + ca], u_s[wv][cb][i]);
+
+    // --- correction: u_c = G S_B[c]  (precorrect_const, src/precorrection.f90:50-82);
+    // lane (i, half): box node i, channels 2 half and 2 half + 1
+    if (lane < 54) {
+        const int i = lane % 27, c = 2 * (lane / 27);
+        const int bi = i % 3 + 5 * ((i / 3) % 3) + 25 * (i / 9);
+        cd a0 = cmk(0, 0), a1 = a0;
+#pragma unroll 3
+        for (int j = 0; j < 27; ++j) {
+            const cd g = G[62 + bi - (j % 3 + 5 * ((j / 3) % 3) + 25 * (j / 9))];
+            cfma(a0, g, L.SB[4 * j + c]);
+            cfma(a1, g, L.SB[4 * j + c + 1]);
+        }
+        L.u[c * 27 + i] = a0;
+        L.u[(c + 1) * 27 + i] = a1;
+    }
+    __syncthreads();
+    // 10 bilinear forms on 4 lanes each: S_T . u_0 ; corr2(a,b) = D_a,T . u_{1+b}
+    {
+        cd c = cmk(0, 0);
+        const int q = lane >> 2;
+        if (q < 10) {
+            const int ca = q == 0 ? 0 : 1 + (q - 1) / 3;
+            const int cb = q == 0 ? 0 : 1 + (q - 1) % 3;
+            for (int i = lane & 3; i < 27; i += 4) cfma(c, ST[i * 4 + ca], L.u[cb * 27 + i]);
+        }
+        for (int o = 1; o < 4; o <<= 1) {
+            c.x += __shfl_xor(c.x, o, 64);
+            c.y += __shfl_xor(c.y, o, 64);
+        }
+        if (q < 10 && (lane & 3) == 0) L.form[q] = c;
     }
 
     // --- V_V: 24-point rule on both tets (integrate_V_V_G, src/precorrection.f90:729-760)
     cd vv = cmk(0, 0);
-    if (lane < 24) {
-        double wsum = 0.0;
-        for (int i = 0; i < 24; ++i) wsum += c_tet24_w[i] * 6.0 * vB;
-        const double cut = 1.0e-10 * pow(wsum, (double)(1.0f / 3.0f));
-        v3 rf = tet_point(tcT, c_tet24_p[3 * lane], c_tet24_p[3 * lane + 1], c_tet24_p[3 * lane + 2]);
-        double wt = c_tet24_w[lane] * 6.0 * vT;
-        vv = cscale(int_V_G(rf, k, tcB, vB, cut), wt);
-    }
-
-    // --- dV_dV: face pairs x 7-point rules (integrate_dV_dV_G, :764-806)
-    cd dd[9];
-#pragma unroll
-    for (int q = 0; q < 9; ++q) dd[q] = cmk(0, 0);
-    for (int item = lane; item < 112; item += 64) {
-        const int ft = item / 28, fb = (item / 7) % 4, i = item % 7;
-        v3 t0, t1, t2, b0, b1, b2;
-        tet_face(tcT, ft, t0, t1, t2);
-        tet_face(tcB, fb, b0, b1, b2);
-        v3 Tn = tri_normal(t0, t1, t2);
-        v3 Bn = tri_normal(b0, b1, b2);
-        double tww = tri_ww1(t0, t1, t2);
-        double bww = tri_ww1(b0, b1, b2);
-        v3 rf = tri_point(t0, t1, t2, c_tri7_p[2 * i], c_tri7_p[2 * i + 1]);
-        double wt = c_tri7_w[i] * tww;
-        double wsum = 0.0;
-        for (int j = 0; j < 7; ++j) wsum += c_tri7_w[j] * bww;
-        const double cut = 1.0e-10 * sqrt(wsum);
-        cd intR = cmk(0, 0);
-        for (int j = 0; j < 7; ++j) {
-            v3 pb = tri_point(b0, b1, b2, c_tri7_p[2 * j], c_tri7_p[2 * j + 1]);
-            double R = dist3(pb, rf);
-            cd II = (R < cut) ? cmk(0.0, k / (4.0 * PI_D)) : green_remainder(R, k);
-            intR = cadd(intR, cscale(II, c_tri7_w[j] * bww));
+    {
+        int i = lane / 24, j = lane % 24;
+#pragma unroll 1
+        for (int r = 0; r < 9; ++r) {
+            const RulePoint a = L.tq[i], b = L.bq[j];
+            const double dx = a.x - b.x, dy = a.y - b.y, dz = a.z - b.z, w = a.w * b.w;
+            const cd g = smooth_green<SER, GENERAL>(dx * dx + dy * dy + dz * dz, k, k4pi);
+            vv.x = fma(w, g.x, vv.x);
+            vv.y = fma(w, g.y, vv.y);
+            i += 2, j += 16;  // 64 = 2 * 24 + 16
+            if (j >= 24) j -= 24, ++i;
         }
-        double K1, K2;
-        analytic_tri(b0, b1, b2, Bn, rf, K1, K2);
-        double f2 = 1.0 / (4 * PI_D) * 1.0 * 1.0 * K1;
-        f2 = f2 + 1.0 / (4 * PI_D) * (k * k) * (-0.5) * K2;
-        cd s = cscale(cmk(intR.x + f2, intR.y), wt);
-        const double tn[3] = {Tn.x, Tn.y, Tn.z}, bn[3] = {Bn.x, Bn.y, Bn.z};
-#pragma unroll
-        for (int a = 0; a < 3; ++a)
-#pragma unroll
-            for (int b = 0; b < 3; ++b) dd[a + 3 * b] = cadd(dd[a + 3 * b], cscale(s, tn[a] * bn[b]));
+        const double sc = 36.0 * vT * vB;
+        vv.x *= sc;
+        vv.y *= sc;
     }
-
-    // --- reductions over the wave
-    double vvr = wave_sum(vv.x), vvi = wave_sum(vv.y);
-    double ddr[9], ddi[9];
-#pragma unroll
-    for (int q = 0; q < 9; ++q) {
-        ddr[q] = wave_sum(dd[q].x);
-        ddi[q] = wave_sum(dd[q].y);
+    // --- dV_dV: face pairs x 7-point rules (integrate_dV_dV_G, :764-806); lanes
+    // 4 q .. 4 q + 3 hold face pair q = 4 ft + fb
+    const int fp = lane >> 2, ft = fp >> 2, fb = fp & 3;
+    cd s = cmk(0, 0);
+#pragma unroll 1
+    for (int e = lane & 3; e < 49; e += 4) {
+        const int i = (37 * e) >> 8, j = e - 7 * i;  // e / 7 for e < 49
+        const RulePoint a = L.ts[7 * ft + i], b = L.bs[7 * fb + j];
+        const double dx = a.x - b.x, dy = a.y - b.y, dz = a.z - b.z, w = a.w * b.w;
+        const cd g = smooth_green<SER, GENERAL>(dx * dx + dy * dy + dz * dz, k, k4pi);
+        s.x = fma(w, g.x, s.x);
+        s.y = fma(w, g.y, s.y);
     }
-    double cfr[10], cfi[10];
-#pragma unroll
-    for (int q = 0; q < 10; ++q) {
-        cfr[q] = __shfl(cform.x, q, 64);
-        cfi[q] = __shfl(cform.y, q, 64);
+    {
+        const double bw = L.fb[fb].area2;
+        s.x *= bw;
+        s.y *= bw;
     }
-    if (lane == 0 && valid) {
+    // --- triangle integrals over the basis tet's faces: rounds 0 and 1 the 7
+    // surface points of the lane's own face pair, then the 96 (volume point,
+    // face) pairs on what lanes those leave idle and in two rounds more
+#pragma unroll 1
+    for (int r = 0; r < 4; ++r) {
+        int f = fb, surf = -1, volp = -1;
+        if (r < 2) {
+            const int i = (lane & 3) + 4 * r;
+            if (i < 7)
+                surf = i;
+            else  // the fourth lane of each face pair in round 1: pairs 80 .. 95
+                volp = 80 + fp;
+        } else {
+            const int e = lane + 64 * (r - 2);
+            if (e < 80) volp = e;
+        }
+        if (volp >= 0) f = volp & 3;
+        if (surf >= 0 || volp >= 0) {
+            const RulePoint &q = surf >= 0 ? L.ts[7 * ft + surf] : L.tq[volp >> 2];
+            const v3 pt = mk3(q.x, q.y, q.z);
+            double K1, K2;
+            tri_integrals(L.fb[f], pt, K1, K2);
+            if (surf >= 0) {
+                s.x = fma(q.w, i4pi * (K1 - 0.5 * k2 * K2), s.x);
+            } else {
+                // int over the tet of 1/R and R as face integrals times the height
+                const double h = dot3(L.fb[f].n, sub3(L.fb[f].p[0], pt));
+                vv.x = fma(6.0 * vT * q.w, i4pi * h * (0.5 * K1 - 0.125 * k2 * K2), vv.x);
+            }
+        }
+    }
+    for (int o = 1; o < 4; o <<= 1) {
+        s.x += __shfl_xor(s.x, o, 64);
+        s.y += __shfl_xor(s.y, o, 64);
+    }
+    if ((lane & 3) == 0) L.s[fp] = cscale(s, L.ta2[ft]);
+    const double vvr = wave_sum(vv.x), vvi = wave_sum(vv.y);
+    __syncthreads();
+    if (lane < 9) {
+        const int a = lane % 3, b = lane / 3;
+        cd dd = cmk(0, 0);
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            const double w = L.tn[q >> 2][a] * L.bn[q & 3][b];
+            const cd v = L.s[q];
+            dd.x = fma(w, v.x, dd.x);
+            dd.y = fma(w, v.y, dd.y);
+        }
         const double sc = sqrt(vT * vB);
         const double inv = 1.0 / sqrt(vB * vT);
-        const double k2 = k * k;
-        cd epsm1 = cmk(0, 0);
-        const bool self = (T == B);
-        if (self) {
-            cd e = param[T];
-            epsm1 = cdiv(cmk(1.0, 0.0), cmk(e.x - 1.0, e.y));
-        }
-#pragma unroll
-        for (int a = 0; a < 3; ++a)
-#pragma unroll
-            for (int b = 0; b < 3; ++b) {
-                cd corr = (a == b) ? cmk(cfr[0] * sc, cfi[0] * sc) : cmk(0, 0);
-                cd corr2 = cmk(cfr[1 + 3 * a + b] * sc, cfi[1 + 3 * a + b] * sc);
-                cd alok1 = (a == b) ? cmk(vvr, vvi) : cmk(0, 0);
-                cd t1 = csub(alok1, corr);
-                cd t2 = csub(cmk(ddr[a + 3 * b], ddi[a + 3 * b]), corr2);
-                cd inner = cadd(cmk(-k2 * t1.x, -k2 * t1.y), t2);
-                cd alok = (self && a == b) ? epsm1 : cmk(0, 0);
-                cd val = cadd(alok, cmk(inv * inner.x, inv * inner.y));
-                blocks[p * 9 + a + 3 * b] = make_float2((float)val.x, (float)val.y);
+        const cd c1 = cscale(L.form[0], sc), c2 = cscale(L.form[1 + 3 * a + b], sc);
+        cd inner = csub(dd, c2);
+        cd val = cmk(0, 0);
+        if (a == b) {
+            inner = cadd(inner, cmk(-k2 * (vvr - c1.x), -k2 * (vvi - c1.y)));
+            if (T == B) {
+                const cd e = param[T];
+                val = cdiv(cmk(1.0, 0.0), cmk(e.x - 1.0, e.y));
             }
+        }
+        val = cadd(val, cscale(inner, inv));
+        blocks[p * 9 + lane] = make_float2((float)val.x, (float)val.y);
     }
 }
 
@@ -588,20 +777,25 @@ void launch_fg_octant(const cd *F, cd *fg, int Lx, int Ly, int Lz, hipStream_t s
     HIP_CHECK(hipGetLastError());
 }
 void launch_pg_table(cd *Gtab, const GridDesc &gd, double k, hipStream_t s) {
-    hipLaunchKernelGGL(k_pg_table, dim3((27 * 27 * 27 + 255) / 256), dim3(256), 0, s, Gtab, gd, k);
+    hipLaunchKernelGGL(k_pg_table, dim3((27 * 125 + 255) / 256), dim3(256), 0, s, Gtab, gd, k);
     HIP_CHECK(hipGetLastError());
 }
 void launch_near_blocks(const int *PT, const int *PB, const uint8_t *POFF, long long P, const double *tcoord,
-                        const double *vol, const cd *param, const cd *S4, const cd *Gtab, double k, cf *blocks,
-                        hipStream_t s) {
-    if (P == 0) return;
-    long long nb = (P + 3) / 4;
+                        const double *vol, const cd *param, const cd *S4, const cd *Gtab, double k, double reach,
+                        cf *blocks, hipStream_t s) {
+    // the shortest series that covers every pair of points of the near zone
+    // (k reach bounds kR): at 43,248 tets 11 terms take 23.2 ms, 17 terms 24.9 ms
+    // and the general variant 31.8 ms (at ka 25, where part of the pairs take
+    // sincos)
+    const double x = k * reach;
+    auto kern = x <= SERIES_X_SHORT ? &k_near_blocks<SERIES_SHORT, false>
+                                    : (x <= SERIES_X_LONG ? &k_near_blocks<SERIES_LONG, false>
+                                                          : &k_near_blocks<SERIES_LONG, true>);
     const long long maxb = 1LL << 30;
-    for (long long b0 = 0; b0 < nb; b0 += maxb) {
-        long long cnt = std::min(maxb, nb - b0);
-        long long p0 = b0 * 4;
-        hipLaunchKernelGGL(k_near_blocks, dim3((unsigned)cnt), dim3(256), 0, s, PT + p0, PB + p0, POFF + p0,
-                           P - p0, tcoord, vol, param, S4, Gtab, k, blocks + p0 * 9);
+    for (long long p0 = 0; p0 < P; p0 += maxb) {
+        const long long cnt = std::min(maxb, P - p0);
+        hipLaunchKernelGGL(kern, dim3((unsigned)cnt), dim3(64), 0, s, PT + p0, PB + p0, POFF + p0, tcoord, vol, param,
+                           S4, Gtab, k, blocks + p0 * 9);
         HIP_CHECK(hipGetLastError());
     }
 }

@@ -23,9 +23,10 @@ void launch_projection(const double *tcoord, const double *vol, const int *tet_c
 void launch_green_grid(cd *A, const GridDesc &gd, int Lx, int Ly, int Lz, double k, hipStream_t s);
 void launch_fg_octant(const cd *F, cd *fg, int Lx, int Ly, int Lz, hipStream_t s);
 void launch_pg_table(cd *Gtab, const GridDesc &gd, double k, hipStream_t s);
+// reach: a bound on the distance between points of two tets of the near zone
 void launch_near_blocks(const int *PT, const int *PB, const uint8_t *POFF, long long P, const double *tcoord,
-                        const double *vol, const cd *param, const cd *S4, const cd *Gtab, double k, cf *blocks,
-                        hipStream_t s);
+                        const double *vol, const cd *param, const cd *S4, const cd *Gtab, double k, double reach,
+                        cf *blocks, hipStream_t s);
 void launch_vswf(const double *tcoord, const double *vol, int N, int Nmax, double k, cd *mat, int ncol,
                  hipStream_t s);
 

@@ -72,6 +72,22 @@ def test_near_blocks(ops):
     assert err.max() < 2 * 2.0 ** -23, err.max()
 
 
+@pytest.mark.parametrize('ka', [0.3, 0.9, 8.0])
+def test_near_blocks_series(ka):
+    """The three variants of the near-zone kernel: k times the near zone's reach
+    (2.6 a on this mesh) within 1.5, within 4, and beyond."""
+    from scadyn_amd import native
+    c, e, param, k = sphere_case(ka=ka)
+    say(f'near-zone blocks at ka {ka}')
+    g = native.Operator(c, e, param, k)
+    blk = g.export('blocks').astype(np.complex128)
+    g.close()
+    ref = oracle_operator(ka=ka).sp_mat.astype(np.complex128)
+    scale = np.abs(ref).reshape(len(ref), -1).max(axis=1)
+    err = np.abs(blk - ref).reshape(len(ref), -1).max(axis=1) / scale
+    assert err.max() < 2 * 2.0 ** -23, err.max()
+
+
 def test_matvec(ops):
     from oracle import pfft_ref
     g, o = ops
