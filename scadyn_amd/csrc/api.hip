@@ -176,7 +176,6 @@ struct scadyn_operator {
     scadyn_opts opts;
     double k = 0;
     HostGeometry g;
-    NearPairs np;
     GridDesc gd;
     int L[3] = {0, 0, 0}, Hh[3] = {0, 0, 0};
     DevMem mem;
@@ -184,7 +183,7 @@ struct scadyn_operator {
     cd *d_param = nullptr, *d_S4 = nullptr, *d_fg = nullptr, *d_tw = nullptr;
     cf *d_S4f = nullptr, *d_fgf = nullptr, *d_twf = nullptr;  // complex64 copies (mixed precision)
     int *d_tet_cube = nullptr, *d_cube_start = nullptr, *d_perm = nullptr;
-    int *d_ne_cubes = nullptr;  // non-empty cubes (only with np.cube_rows)
+    int *d_ne_cubes = nullptr;  // non-empty cubes
     int n_ne_cubes = 0;
     cf *d_blocks = nullptr;
     int64_t *d_row_start = nullptr;
@@ -332,6 +331,24 @@ static uint64_t morton3(int x, int y, int z) {
     return spread((uint64_t)x) | spread((uint64_t)y) << 1 | spread((uint64_t)z) << 2;
 }
 
+// the near-zone pair list of an operator in device memory of its own; rows:
+// also the operator's row entries
+struct PairList {
+    DevMem mem;
+    int *T = nullptr, *B = nullptr;
+    uint8_t *off = nullptr;
+};
+static void make_pairs(scadyn_operator *op, PairList &pl, bool rows) {
+    const size_t P = (size_t)op->nblocks;
+    pl.T = pl.mem.alloc<int>(P);
+    pl.B = pl.mem.alloc<int>(P);
+    pl.off = pl.mem.alloc<uint8_t>(P);
+    uint32_t *pos = pl.mem.alloc<uint32_t>((size_t)27 * op->g.N);
+    uint32_t *tot = pl.mem.alloc<uint32_t>((size_t)op->g.N_cubes);
+    launch_near_pairs(op->d_cube_start, op->d_perm, op->d_row_start, op->gd, pos, tot, pl.T, pl.B, pl.off,
+                      rows ? op->d_ent_col : nullptr, rows ? op->d_ent_blk : nullptr, op->s);
+}
+
 // Bound on the distance between points of two tets of the near zone: their
 // centroids lie in cubes at most one apart per axis, i.e. within two cube
 // edges per axis.
@@ -357,11 +374,12 @@ static void create_operator(scadyn_operator *op, const scadyn_mesh &mesh, const 
     // host-side validation and indexing first: mesh errors surface without a device
     HostGeometry &g = op->g;
     build_geometry(mesh, opts, g);
-    build_near_pairs(g, op->np);
+    NearRows rows;
+    build_near_rows(g, rows);
     HIP_CHECK(hipSetDevice(op->device));
     HIP_CHECK(hipStreamCreateWithFlags(&op->s, hipStreamNonBlocking));
     hipStream_t s = op->s;
-    op->nblocks = (long long)op->np.T.size();
+    op->nblocks = rows.P;
     GridDesc &gd = op->gd;
     for (int c = 0; c < 3; ++c) gd.min[c] = g.min_coord[c];
     gd.delta = g.delta;
@@ -385,7 +403,7 @@ static void create_operator(scadyn_operator *op, const scadyn_mesh &mesh, const 
     op->d_tet_cube = M.upload(g.tet_cube, s);
     op->d_cube_start = M.upload(g.cube_start, s);
     op->d_perm = M.upload(g.perm, s);
-    if (op->np.cube_rows) {
+    {
         // non-empty cubes in Morton (Z-curve) order of their coordinates: the
         // gather's waves in flight at once then cover a compact block of
         // cubes rather than a slab of whole x rows (measured 2-3% faster at
@@ -462,23 +480,17 @@ static void create_operator(scadyn_operator *op, const scadyn_mesh &mesh, const 
     {
         cd *d_G = M.alloc<cd>(27 * 125);
         launch_pg_table(d_G, gd, k, s);
-        int *d_PT = M.upload(op->np.T, s);
-        int *d_PB = M.upload(op->np.B, s);
-        uint8_t *d_PO = M.upload(op->np.off, s);
+        op->d_row_start = M.upload(rows.row_start, s);
+        const size_t E = (size_t)rows.row_start[N];
+        op->d_ent_col = M.alloc<int>(E);
+        op->d_ent_blk = M.alloc<uint32_t>(E);
         op->d_blocks = M.alloc<cf>((size_t)op->nblocks * 9);
-        launch_near_blocks(d_PT, d_PB, d_PO, op->nblocks, op->d_tcoord, op->d_vol, op->d_param, op->d_S4, d_G, k,
+        PairList pl;
+        make_pairs(op, pl, true);
+        launch_near_blocks(pl.T, pl.B, pl.off, op->nblocks, op->d_tcoord, op->d_vol, op->d_param, op->d_S4, d_G, k,
                            near_reach(g), op->d_blocks, s);
-        op->d_row_start = M.upload(op->np.row_start, s);
-        op->d_ent_col = M.upload(op->np.ent_col, s);
-        op->d_ent_blk = M.upload(op->np.ent_blk, s);
         HIP_CHECK(hipStreamSynchronize(s));
-        M.release(d_PT);
-        M.release(d_PB);
-        M.release(d_PO);
         M.release(d_G);
-        std::vector<int>().swap(op->np.ent_col);
-        std::vector<uint32_t>().swap(op->np.ent_blk);
-        std::vector<uint8_t>().swap(op->np.off);
     }
     // ---- FFT(G) (src/build_G.f90)
     {
@@ -1370,7 +1382,7 @@ static Footprint footprint_of(const HostGeometry &g, long long P, const scadyn_o
     f.op = N * (96 + 8 + 16 + 4 + 4) + 4 * (g.N_cubes + 1) + 1728 * N + 72 * (size_t)P + 8 * (N + 1) +
            8 * 2 * (size_t)P + cdb * H[0] * H[1] * H[2] + cdb * (L[0] + L[1] + L[2]);
     if (o.precision == SCADYN_PREC_MIXED) f.op += 864 * N + 8 * H[0] * H[1] * H[2];
-    f.setup = 2 * cdb * L[0] * L[1] * L[2] + 9 * (size_t)P + cdb * 27 * 27 * 27 + cdb * 98 * 27;
+    f.setup = 2 * cdb * L[0] * L[1] * L[2] + 9 * (size_t)P + 4 * (27 * N + g.N_cubes) + cdb * 27 * 125 + cdb * 98 * 27;
     // solve workspace (workspace(), restart_space()): per slot the Krylov
     // vectors (slot_vec_bytes: the basis storage of the solve) and two
     // complex128-sized grids; the reduction partials of up to 2048 row-sweep
@@ -1709,7 +1721,7 @@ int scadyn_op_info(const scadyn_operator *op, int64_t info[16], double dinfo[4])
         info[10] = op->ws ? op->ws->B : 0;
         info[11] = (int64_t)(op->mem.bytes + (op->ws ? op->ws->mem.bytes : 0));
         info[12] = op->last_outer_rounds;
-        info[13] = op->np.cube_rows ? 1 : 0;
+        info[13] = 1;
         if (op->ws)  // tile widths of the five line-FFT passes, 8 bits each (FP64, FP32)
             for (int q = 0; q < 5; ++q) {
                 info[14] |= (int64_t)(op->ws->mv.pass[0][q].ti & 0xff) << (8 * q);
@@ -1745,10 +1757,16 @@ int scadyn_op_export(const scadyn_operator *opc, int32_t what, void *host, int64
         HIP_CHECK(hipMemcpy(host, op->d_blocks, nbytes, hipMemcpyDeviceToHost));
     } else if (what == SCADYN_EXPORT_BLKIND) {
         if (nbytes != (int64_t)sizeof(int32_t) * 2 * op->nblocks) fail(SCADYN_ERR_ARG, "size mismatch");
+        PairList pl;
+        make_pairs(op, pl, false);
+        std::vector<int> T((size_t)op->nblocks), B((size_t)op->nblocks);
+        HIP_CHECK(hipMemcpyAsync(T.data(), pl.T, sizeof(int) * T.size(), hipMemcpyDeviceToHost, op->s));
+        HIP_CHECK(hipMemcpyAsync(B.data(), pl.B, sizeof(int) * B.size(), hipMemcpyDeviceToHost, op->s));
+        HIP_CHECK(hipStreamSynchronize(op->s));
         int32_t *o = (int32_t *)host;
         for (long long p = 0; p < op->nblocks; ++p) {
-            o[2 * p] = op->g.perm[op->np.T[p]] + 1;
-            o[2 * p + 1] = op->g.perm[op->np.B[p]] + 1;
+            o[2 * p] = op->g.perm[T[p]] + 1;
+            o[2 * p + 1] = op->g.perm[B[p]] + 1;
         }
     } else if (what == SCADYN_EXPORT_FG) {
         size_t n = (size_t)op->Hh[0] * op->Hh[1] * op->Hh[2];
@@ -2031,11 +2049,11 @@ int scadyn_footprint(const scadyn_mesh *mesh, const scadyn_opts *opts, int32_t n
     check_opts(o);
     HostGeometry g;
     build_geometry(*mesh, o, g);
-    NearPairs np;
-    build_near_pairs(g, np);
+    NearRows rows;
+    build_near_rows(g, rows);
     const int ncol = 2 * ((nmax + 1) * (nmax + 1) - 1);
     const int B = o.batch > 0 ? std::min(o.batch, ncol) : std::min(ncol, 64);
-    *bytes = (int64_t)footprint_of(g, (long long)np.T.size(), o, nmax, B).peak();
+    *bytes = (int64_t)footprint_of(g, rows.P, o, nmax, B).peak();
     ABI_CATCH
 }
 
@@ -2081,9 +2099,9 @@ int scadyn_server_submit(scadyn_server *sv, const scadyn_mesh *mesh, const scady
     check_opts(r->opts);
     HostGeometry g;
     build_geometry(*mesh, r->opts, g);
-    NearPairs np;
-    build_near_pairs(g, np);
-    r->fp = footprint_of(g, (long long)np.T.size(), r->opts, nmax, std::min(r->opts.batch, ncol)).peak();
+    NearRows rows;
+    build_near_rows(g, rows);
+    r->fp = footprint_of(g, rows.P, r->opts, nmax, std::min(r->opts.batch, ncol)).peak();
     if (r->fp > sv->budget)
         fail(SCADYN_ERR_MEMORY, "request needs " + std::to_string(r->fp) + " device bytes, budget is " +
                                     std::to_string(sv->budget));

@@ -1,4 +1,4 @@
-// Host-side setup: grid, cube boxes, tet -> cube map, near-zone pair lists,
+// Host-side setup: grid, cube boxes, tet -> cube map, near-zone row offsets,
 // the 98x27 pseudo-inverse, and FFT length planning.  Integer/indexing work
 // that the reference does serially on the host in src/geometry.f90,
 // src/sparse_mat.f90:13-60 and src/precorrection.f90:182-258.
@@ -131,103 +131,28 @@ void build_geometry(const scadyn_mesh &mesh, const scadyn_opts &opts, HostGeomet
     }
 }
 
-void build_near_pairs(const HostGeometry &g, NearPairs &np) {
-    // src/precorrection.f90:182-258: test cube, near cube (z,y,x order),
-    // test tet, basis tet, keep reference ids tet_B >= tet_T.
-    np.T.clear();
-    np.B.clear();
-    np.off.clear();
-    for (int tc = 0; tc < g.N_cubes; ++tc) {
-        int t0 = g.cube_start[tc], t1 = g.cube_start[tc + 1];
+void build_near_rows(const HostGeometry &g, NearRows &nr) {
+    nr.row_start.assign((size_t)g.N + 1, 0);
+    int64_t e = 0;
+    for (int c = 0; c < g.N_cubes; ++c) {
+        const int t0 = g.cube_start[c], t1 = g.cube_start[c + 1];
         if (t0 == t1) continue;
-        int cx = tc % g.ncx, cy = (tc / g.ncx) % g.ncy, cz = tc / (g.ncx * g.ncy);
-        for (int dz = -1; dz <= 1; ++dz) {
-            int zz = cz + dz;
-            if (zz < 0 || zz >= g.ncz) continue;
-            for (int dy = -1; dy <= 1; ++dy) {
-                int yy = cy + dy;
-                if (yy < 0 || yy >= g.ncy) continue;
-                for (int dx = -1; dx <= 1; ++dx) {
-                    int xx = cx + dx;
-                    if (xx < 0 || xx >= g.ncx) continue;
-                    int bc = xx + g.ncx * (yy + g.ncy * zz);
-                    uint8_t off = (uint8_t)((dx + 1) + 3 * (dy + 1) + 9 * (dz + 1));
-                    for (int T = t0; T < t1; ++T)
-                        for (int B = g.cube_start[bc]; B < g.cube_start[bc + 1]; ++B)
-                            if (g.perm[B] >= g.perm[T]) {
-                                np.T.push_back(T);
-                                np.B.push_back(B);
-                                np.off.push_back(off);
-                            }
-                }
+        const int cx = c % g.ncx, cy = (c / g.ncx) % g.ncy, cz = c / (g.ncx * g.ncy);
+        // the near cubes of one (z, y) line are consecutive
+        int64_t len = 0;
+        for (int zz = std::max(cz - 1, 0); zz <= std::min(cz + 1, g.ncz - 1); ++zz)
+            for (int yy = std::max(cy - 1, 0); yy <= std::min(cy + 1, g.ncy - 1); ++yy) {
+                const int line = g.ncx * (yy + g.ncy * zz);
+                len += g.cube_start[line + std::min(cx + 1, g.ncx - 1) + 1] - g.cube_start[line + std::max(cx - 1, 0)];
             }
+        for (int t = t0; t < t1; ++t) {
+            nr.row_start[t] = e;
+            e += len;
         }
     }
-    // row lists: row T gets (B, p), row B gets (T, p | transpose) when T != B
-    const size_t P = np.T.size();
-    if (P >= (size_t)BLK_TRANSPOSE) fail(SCADYN_ERR_UNSUPPORTED, "too many near-zone blocks");
-    np.row_start.assign(g.N + 1, 0);
-    for (size_t p = 0; p < P; ++p) {
-        np.row_start[np.T[p] + 1]++;
-        if (np.T[p] != np.B[p]) np.row_start[np.B[p] + 1]++;
-    }
-    for (int i = 0; i < g.N; ++i) np.row_start[i + 1] += np.row_start[i];
-    np.ent_col.resize(np.row_start[g.N]);
-    np.ent_blk.resize(np.row_start[g.N]);
-    std::vector<int64_t> fill(np.row_start.begin(), np.row_start.end() - 1);
-    for (size_t p = 0; p < P; ++p) {
-        int64_t e = fill[np.T[p]]++;
-        np.ent_col[e] = np.B[p];
-        np.ent_blk[e] = (uint32_t)p;
-        if (np.T[p] != np.B[p]) {
-            e = fill[np.B[p]]++;
-            np.ent_col[e] = np.T[p];
-            np.ent_blk[e] = (uint32_t)p | BLK_TRANSPOSE;
-        }
-    }
-    // order each row by (near-cube offset, column tet) and check that it holds
-    // every tet of the near cubes exactly once
-    np.cube_rows = true;
-    std::vector<int64_t> key;
-    for (int t = 0; t < g.N; ++t) {
-        const int64_t r0 = np.row_start[t], r1 = np.row_start[t + 1];
-        const int ct = g.tet_cube[t];
-        const int tx = ct % g.ncx, ty = (ct / g.ncx) % g.ncy, tz = ct / (g.ncx * g.ncy);
-        key.resize(r1 - r0);
-        for (int64_t e = r0; e < r1; ++e) {
-            const int cc = g.tet_cube[np.ent_col[e]];
-            const int dx = cc % g.ncx - tx, dy = (cc / g.ncx) % g.ncy - ty, dz = cc / (g.ncx * g.ncy) - tz;
-            key[e - r0] = (int64_t)((dx + 1) + 3 * (dy + 1) + 9 * (dz + 1)) * g.N + np.ent_col[e];
-        }
-        // insertion sort: rows are short and close to sorted
-        for (int64_t a = 1; a < r1 - r0; ++a) {
-            const int64_t k = key[a];
-            const int col = np.ent_col[r0 + a];
-            const uint32_t blk = np.ent_blk[r0 + a];
-            int64_t b = a - 1;
-            while (b >= 0 && key[b] > k) {
-                key[b + 1] = key[b];
-                np.ent_col[r0 + b + 1] = np.ent_col[r0 + b];
-                np.ent_blk[r0 + b + 1] = np.ent_blk[r0 + b];
-                --b;
-            }
-            key[b + 1] = k;
-            np.ent_col[r0 + b + 1] = col;
-            np.ent_blk[r0 + b + 1] = blk;
-        }
-        if (!np.cube_rows) continue;
-        int64_t e = r0;
-        for (int dz = -1; dz <= 1 && np.cube_rows; ++dz)
-            for (int dy = -1; dy <= 1 && np.cube_rows; ++dy)
-                for (int dx = -1; dx <= 1 && np.cube_rows; ++dx) {
-                    const int xx = tx + dx, yy = ty + dy, zz = tz + dz;
-                    if (xx < 0 || xx >= g.ncx || yy < 0 || yy >= g.ncy || zz < 0 || zz >= g.ncz) continue;
-                    const int bc = xx + g.ncx * (yy + g.ncy * zz);
-                    for (int c = g.cube_start[bc]; c < g.cube_start[bc + 1]; ++c)
-                        if (e >= r1 || np.ent_col[e++] != c) np.cube_rows = false;
-                }
-        if (e != r1) np.cube_rows = false;
-    }
+    nr.row_start[g.N] = e;
+    nr.P = (e + g.N) / 2;
+    if (nr.P >= (long long)BLK_TRANSPOSE) fail(SCADYN_ERR_UNSUPPORTED, "too many near-zone blocks");
 }
 
 // Hestenes one-sided Jacobi SVD of A (m x n, column-major), m >= n.

@@ -141,24 +141,18 @@ struct HostGeometry {
 // Builds the grid/cube structures; throws on orientation and grid errors.
 void build_geometry(const scadyn_mesh &mesh, const scadyn_opts &opts, HostGeometry &g);
 
-// Near-zone pair list in the reference's storage order: for block p,
-// (T[p], B[p]) are internal tet ids with reference ids perm[T] <= perm[B],
-// off[p] in [0,27) is the cube offset (dx+1) + 3(dy+1) + 9(dz+1) from T's cube
-// to B's cube.
-struct NearPairs {
-    std::vector<int> T, B;
-    std::vector<uint8_t> off;
-    // row lists over internal tets: entries (column tet, block id | TRANSPOSE)
-    std::vector<int64_t> row_start;
-    std::vector<int> ent_col;
-    std::vector<uint32_t> ent_blk;
-    // true when every row lists exactly the tets of its cube's near cubes, in
-    // near-cube order (dz, dy, dx ascending) and ascending tet id within a
-    // cube: then the entries of all tets of one cube line up by position
-    bool cube_rows = false;
+// Near-zone rows.  The near zone of a tet is every tet of the <= 27 cubes
+// around its own; the reference stores each unordered pair once (the 3 x 3 block
+// of a pair also serves the other row, transposed).  The entries of row t are in
+// near-cube order (dz, dy, dx ascending) and ascending tet id within a cube, so
+// those of all tets of one cube line up by position.  The pairs themselves and
+// each entry's block are made on the device (launch_near_pairs, setup.hpp).
+struct NearRows {
+    std::vector<int64_t> row_start;  // first entry of each row, N + 1
+    long long P = 0;                 // stored blocks: (entries + N) / 2
 };
 constexpr uint32_t BLK_TRANSPOSE = 0x80000000u;
-void build_near_pairs(const HostGeometry &g, NearPairs &np);
+void build_near_rows(const HostGeometry &g, NearRows &nr);
 
 // SVD pseudo-inverse (one-sided Jacobi), singular values <= thr dropped.
 // A is m x n column-major; returns n x m column-major.

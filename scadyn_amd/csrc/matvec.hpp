@@ -21,8 +21,7 @@ struct MatvecArgs {
     const int *ent_col = nullptr;
     const uint32_t *ent_blk = nullptr;
     const cf *blocks = nullptr;
-    // non-empty cubes; set only when the near-zone rows are in cube order
-    // (NearPairs::cube_rows), which the per-cube gather relies on
+    // non-empty cubes, in the order the per-cube gather takes them
     const int *ne_cubes = nullptr;
     int n_ne = 0;
     double k2 = 0;

@@ -398,6 +398,120 @@ __global__ void k_fg_octant(const cd *__restrict__ F, cd *__restrict__ fg, int L
     }
 }
 
+// ---- near-zone pairs ------------------------------------------------------------
+// One wave per cube in each kernel; the tets of a cube are sorted by reference
+// id, so the basis tets of a near cube that a test tet keeps (id >= its own) are
+// the tail of that cube from one position on.  A position s = 27 t0 + o n + (T -
+// t0) numbers the (near cube o, test tet T) of the cube t0 .. t0 + n - 1 in
+// storage order; pos[s] becomes the id of its first block.  Bound by the writes
+// of the pair and entry lists.  At 43,248 tets (6.4 M entries) an operator is
+// set up in 33 ms; with the pairs pushed, counted and sorted one by one on the
+// host, and the lists copied over, it took 110 ms, at 369,390 tets 222 ms.
+__device__ inline int near_cube(int c, int o, const GridDesc &g) {
+    const int x = c % g.ncx + o % 3 - 1, y = (c / g.ncx) % g.ncy + (o / 3) % 3 - 1, z = c / (g.ncx * g.ncy) + o / 9 - 1;
+    if (x < 0 || x >= g.ncx || y < 0 || y >= g.ncy || z < 0 || z >= g.ncz) return -1;
+    return x + g.ncx * (y + g.ncy * z);
+}
+// first tet of [b, e) whose reference id is >= id
+__device__ inline int first_from(const int *__restrict__ perm, int b, int e, int id) {
+    while (b < e) {
+        const int m = (b + e) >> 1;
+        if (perm[m] < id)
+            b = m + 1;
+        else
+            e = m;
+    }
+    return b;
+}
+__global__ __launch_bounds__(64) void k_pair_count(const int *__restrict__ cs, const int *__restrict__ perm, GridDesc g,
+                                                   uint32_t *__restrict__ tot) {
+    const int c = blockIdx.x, t0 = cs[c], n = cs[c + 1] - t0;
+    int sum = 0;
+    for (int s = threadIdx.x; s < 27 * n; s += 64) {
+        const int nc = near_cube(c, s / n, g);
+        if (nc >= 0) sum += cs[nc + 1] - first_from(perm, cs[nc], cs[nc + 1], perm[t0 + s % n]);
+    }
+    for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
+    if (threadIdx.x == 0) tot[c] = (uint32_t)sum;
+}
+// exclusive prefix sum of tot[0 .. n), in place, by one workgroup
+__global__ __launch_bounds__(1024) void k_scan(uint32_t *__restrict__ tot, int n) {
+    __shared__ uint32_t part[1024];
+    const int per = (n + 1023) / 1024, b = min((int)threadIdx.x * per, n), e = min(b + per, n);
+    uint32_t a = 0;
+    for (int i = b; i < e; ++i) a += tot[i];
+    part[threadIdx.x] = a;
+    __syncthreads();
+    for (int o = 1; o < 1024; o <<= 1) {
+        const uint32_t v = (int)threadIdx.x >= o ? part[threadIdx.x - o] : 0;
+        __syncthreads();
+        part[threadIdx.x] += v;
+        __syncthreads();
+    }
+    uint32_t run = part[threadIdx.x] - a;
+    for (int i = b; i < e; ++i) {
+        const uint32_t v = tot[i];
+        tot[i] = run;
+        run += v;
+    }
+}
+__global__ __launch_bounds__(64) void k_pair_fill(const int *__restrict__ cs, const int *__restrict__ perm, GridDesc g,
+                                                  const uint32_t *__restrict__ base, uint32_t *__restrict__ pos,
+                                                  int *__restrict__ PT, int *__restrict__ PB,
+                                                  uint8_t *__restrict__ PO) {
+    const int c = blockIdx.x, lane = threadIdx.x, t0 = cs[c], n = cs[c + 1] - t0;
+    uint32_t run = base[c];
+    for (int s0 = 0; s0 < 27 * n; s0 += 64) {
+        const int s = s0 + lane, o = s / max(n, 1), T = t0 + s % max(n, 1);
+        int b = 0, cnt = 0;
+        const int nc = s < 27 * n ? near_cube(c, o, g) : -1;
+        if (nc >= 0) {
+            b = first_from(perm, cs[nc], cs[nc + 1], perm[T]);
+            cnt = cs[nc + 1] - b;
+        }
+        int inc = cnt;
+        for (int d = 1; d < 64; d <<= 1) {
+            const int v = __shfl_up(inc, d, 64);
+            if (lane >= d) inc += v;
+        }
+        const uint32_t p = run + (uint32_t)(inc - cnt);
+        if (s < 27 * n) pos[(size_t)27 * t0 + s] = p;
+        for (int i = 0; i < cnt; ++i) {
+            PT[p + i] = T;
+            PB[p + i] = b + i;
+            PO[p + i] = (uint8_t)o;
+        }
+        run += (uint32_t)__shfl(inc, 63, 64);
+    }
+}
+__global__ __launch_bounds__(64) void k_row_fill(const int *__restrict__ cs, const int *__restrict__ perm, GridDesc g,
+                                                 const int64_t *__restrict__ row_start,
+                                                 const uint32_t *__restrict__ pos, int *__restrict__ ent_col,
+                                                 uint32_t *__restrict__ ent_blk) {
+    const int c = blockIdx.x, t0 = cs[c], t1 = cs[c + 1], n = t1 - t0;
+    if (n == 0) return;
+    int col = 0;  // entries of the near cubes before o
+    for (int o = 0; o < 27; ++o) {
+        const int nc = near_cube(c, o, g);
+        if (nc < 0) continue;
+        const int b0 = cs[nc], b1 = cs[nc + 1], m = b1 - b0;
+        for (int l = threadIdx.x; l < n * m; l += 64) {
+            const int T = t0 + l / m, B = b0 + l % m;
+            uint32_t blk;
+            if (perm[B] >= perm[T])
+                blk = pos[(size_t)27 * t0 + (size_t)o * n + (T - t0)] + (uint32_t)(B - first_from(perm, b0, b1, perm[T]));
+            else
+                blk = (pos[(size_t)27 * b0 + (size_t)(26 - o) * m + (B - b0)] +
+                       (uint32_t)(T - first_from(perm, t0, t1, perm[B]))) |
+                      BLK_TRANSPOSE;
+            const int64_t r = row_start[T] + col + l % m;
+            ent_col[r] = B;
+            ent_blk[r] = blk;
+        }
+        col += m;
+    }
+}
+
 // ---- near-zone G between box nodes for the 27 cube offsets ---------------------
 // Gtab[off][t] = G(node of the test box, node of the basis box) for the node
 // difference (tx, ty, tz) - 2, t = tx + 5 ty + 25 tz, plus the offset between
@@ -778,6 +892,18 @@ void launch_fg_octant(const cd *F, cd *fg, int Lx, int Ly, int Lz, hipStream_t s
 }
 void launch_pg_table(cd *Gtab, const GridDesc &gd, double k, hipStream_t s) {
     hipLaunchKernelGGL(k_pg_table, dim3((27 * 125 + 255) / 256), dim3(256), 0, s, Gtab, gd, k);
+    HIP_CHECK(hipGetLastError());
+}
+void launch_near_pairs(const int *cube_start, const int *perm, const int64_t *row_start, const GridDesc &gd,
+                       uint32_t *pos, uint32_t *tot, int *PT, int *PB, uint8_t *PO, int *ent_col, uint32_t *ent_blk,
+                       hipStream_t s) {
+    const int nc = gd.ncx * gd.ncy * gd.ncz;
+    hipLaunchKernelGGL(k_pair_count, dim3(nc), dim3(64), 0, s, cube_start, perm, gd, tot);
+    hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, s, tot, nc);
+    hipLaunchKernelGGL(k_pair_fill, dim3(nc), dim3(64), 0, s, cube_start, perm, gd, tot, pos, PT, PB, PO);
+    if (ent_blk)
+        hipLaunchKernelGGL(k_row_fill, dim3(nc), dim3(64), 0, s, cube_start, perm, gd, row_start, pos, ent_col,
+                           ent_blk);
     HIP_CHECK(hipGetLastError());
 }
 void launch_near_blocks(const int *PT, const int *PB, const uint8_t *POFF, long long P, const double *tcoord,

@@ -23,6 +23,14 @@ void launch_projection(const double *tcoord, const double *vol, const int *tet_c
 void launch_green_grid(cd *A, const GridDesc &gd, int Lx, int Ly, int Lz, double k, hipStream_t s);
 void launch_fg_octant(const cd *F, cd *fg, int Lx, int Ly, int Lz, hipStream_t s);
 void launch_pg_table(cd *Gtab, const GridDesc &gd, double k, hipStream_t s);
+// Near-zone pairs in the reference's storage order (src/precorrection.f90:182-258:
+// test cube, near cube, test tet, basis tet with reference id >= the test
+// tet's): internal ids PT[p], PB[p] and cube offset PO[p] = (dx+1) + 3(dy+1) +
+// 9(dz+1).  With ent_blk also the block id (| BLK_TRANSPOSE) and column tet of
+// every row entry.  pos (27 N) and tot (N_cubes + 1) are scratch.
+void launch_near_pairs(const int *cube_start, const int *perm, const int64_t *row_start, const GridDesc &gd,
+                       uint32_t *pos, uint32_t *tot, int *PT, int *PB, uint8_t *PO, int *ent_col, uint32_t *ent_blk,
+                       hipStream_t s);
 // reach: a bound on the distance between points of two tets of the near zone
 void launch_near_blocks(const int *PT, const int *PB, const uint8_t *POFF, long long P, const double *tcoord,
                         const double *vol, const cd *param, const cd *S4, const cd *Gtab, double k, double reach,

@@ -72,6 +72,29 @@ def test_near_blocks(ops):
     assert err.max() < 2 * 2.0 ** -23, err.max()
 
 
+@pytest.mark.parametrize('body', ['one cube', 'refined', 'ellipsoid'])
+def test_near_pairs(body):
+    """The device's pair list against the oracle's loops: one cube of 6 tets, cubes
+    of up to 17 tets (rows longer than a wave), a ragged grid with empty cubes."""
+    from oracle import pfft_ref
+    from scadyn_amd import meshgen, native
+    if body == 'one cube':
+        c, e = meshgen.sphere(1)
+    elif body == 'refined':
+        c, e, _, _ = refined_sphere_case()
+    else:
+        c, e = meshgen.gaussian_ellipsoid(n_cells=10)
+    say(f'near-zone pairs: {body}, {e.shape[0]} tets')
+    g = native.Operator(c, e, np.full(e.shape[0], 2.5 + 0.01j), 1.0 / np.abs(c).max())
+    ind = g.export('blkind')
+    assert g.info()['n_blocks'] == ind.shape[0]
+    x = np.random.default_rng(3).standard_normal((1, 3 * e.shape[0])) + 0j
+    assert np.isfinite(g.matvec(x)).all()
+    g.close()
+    pairs = np.array([(T, B) for T, B, _, _ in pfft_ref.near_pairs(pfft_ref.build_geometry(c, e))])
+    assert np.array_equal(ind - 1, pairs)
+
+
 @pytest.mark.parametrize('ka', [0.3, 0.9, 8.0])
 def test_near_blocks_series(ka):
     """The three variants of the near-zone kernel: k times the near zone's reach
