@@ -337,15 +337,17 @@ struct PairList {
     DevMem mem;
     int *T = nullptr, *B = nullptr;
     uint8_t *off = nullptr;
+    uint32_t *self = nullptr;
 };
 static void make_pairs(scadyn_operator *op, PairList &pl, bool rows) {
     const size_t P = (size_t)op->nblocks;
     pl.T = pl.mem.alloc<int>(P);
     pl.B = pl.mem.alloc<int>(P);
     pl.off = pl.mem.alloc<uint8_t>(P);
+    pl.self = pl.mem.alloc<uint32_t>((size_t)op->g.N);
     uint32_t *pos = pl.mem.alloc<uint32_t>((size_t)27 * op->g.N);
     uint32_t *tot = pl.mem.alloc<uint32_t>((size_t)op->g.N_cubes);
-    launch_near_pairs(op->d_cube_start, op->d_perm, op->d_row_start, op->gd, pos, tot, pl.T, pl.B, pl.off,
+    launch_near_pairs(op->d_cube_start, op->d_perm, op->d_row_start, op->gd, pos, tot, pl.T, pl.B, pl.off, pl.self,
                       rows ? op->d_ent_col : nullptr, rows ? op->d_ent_blk : nullptr, op->s);
 }
 
@@ -478,7 +480,7 @@ static void create_operator(scadyn_operator *op, const scadyn_mesh &mesh, const 
     }
     // ---- near zone
     {
-        cd *d_G = M.alloc<cd>(27 * 125);
+        cd *d_G = M.alloc<cd>(27 * 27 * 27);
         launch_pg_table(d_G, gd, k, s);
         op->d_row_start = M.upload(rows.row_start, s);
         const size_t E = (size_t)rows.row_start[N];
@@ -487,8 +489,8 @@ static void create_operator(scadyn_operator *op, const scadyn_mesh &mesh, const 
         op->d_blocks = M.alloc<cf>((size_t)op->nblocks * 9);
         PairList pl;
         make_pairs(op, pl, true);
-        launch_near_blocks(pl.T, pl.B, pl.off, op->nblocks, op->d_tcoord, op->d_vol, op->d_param, op->d_S4, d_G, k,
-                           near_reach(g), op->d_blocks, s);
+        launch_near_blocks(pl.T, pl.B, pl.off, pl.self, op->nblocks, N, op->d_tcoord, op->d_vol, op->d_param, op->d_S4,
+                           d_G, k, near_reach(g), op->d_blocks, s);
         HIP_CHECK(hipStreamSynchronize(s));
         M.release(d_G);
     }
@@ -1382,7 +1384,7 @@ static Footprint footprint_of(const HostGeometry &g, long long P, const scadyn_o
     f.op = N * (96 + 8 + 16 + 4 + 4) + 4 * (g.N_cubes + 1) + 1728 * N + 72 * (size_t)P + 8 * (N + 1) +
            8 * 2 * (size_t)P + cdb * H[0] * H[1] * H[2] + cdb * (L[0] + L[1] + L[2]);
     if (o.precision == SCADYN_PREC_MIXED) f.op += 864 * N + 8 * H[0] * H[1] * H[2];
-    f.setup = 2 * cdb * L[0] * L[1] * L[2] + 9 * (size_t)P + 4 * (27 * N + g.N_cubes) + cdb * 27 * 125 + cdb * 98 * 27;
+    f.setup = 2 * cdb * L[0] * L[1] * L[2] + 9 * (size_t)P + 4 * (28 * N + g.N_cubes) + cdb * 27 * 27 * 27 + cdb * 98 * 27;
     // solve workspace (workspace(), restart_space()): per slot the Krylov
     // vectors (slot_vec_bytes: the basis storage of the solve) and two
     // complex128-sized grids; the reduction partials of up to 2048 row-sweep

@@ -151,6 +151,86 @@ __device__ inline v3 tet_point(const double *tc, double x1, double x2, double x3
     return p;
 }
 
+// ---- analytical integrals of 1/R and R over a flat triangle -----------------
+// (src/singularity_subtraction.f90:15-108), returns K1 = int 1/R dS, K2 = int R dS
+__device__ void analytic_tri(v3 p0, v3 p1, v3 p2, v3 n, v3 r, double &K1, double &K2) {
+    v3 p[3] = {p0, p1, p2};
+    const double w0 = dot3(sub3(r, p0), n);
+    const double aw0 = fabs(w0);
+    double k1 = 0.0;
+    double tl[3], I1[3];
+    const int e1[3] = {1, 2, 0}, e2[3] = {2, 0, 1};
+#pragma unroll
+    for (int l = 0; l < 3; ++l) {
+        v3 pl1 = p[e1[l]], pl2 = p[e2[l]];
+        v3 slv = sub3(pl2, pl1);
+        double nsl = sqrt(dot3(slv, slv));
+        v3 sl = mk3(slv.x / nsl, slv.y / nsl, slv.z / nsl);
+        v3 ml = cross3(sl, n);
+        v3 pl1mr = sub3(pl1, r);
+        double tl0 = dot3(pl1mr, ml);
+        v3 pl2mpl1 = sub3(pl2, pl1);
+        double ll = sqrt(dot3(pl2mpl1, pl2mpl1));
+        double sml = dot3(pl1mr, sl);
+        double spl = sml + ll;
+        v3 rmplm1 = sub3(r, pl2);
+        double Rpl = sqrt(dot3(rmplm1, rmplm1));
+        double Rml = sqrt(dot3(pl1mr, pl1mr));
+        double R0l = sqrt(tl0 * tl0 + w0 * w0);
+        double Km3 = 0.0;
+        if (aw0 > 1.0e-10) {
+            double Bl = atan((tl0 * spl) / (R0l * R0l + aw0 * Rpl)) -
+                        atan((tl0 * sml) / (R0l * R0l + aw0 * Rml));
+            Km3 = 1.0 / aw0 * Bl;
+        }
+        double Il;
+        if ((Rml + sml) > (Rpl - spl))
+            Il = log(fabs((Rpl + spl) / (Rml + sml)));
+        else
+            Il = log(fabs((Rml - sml) / (Rpl - spl)));
+        k1 = k1 + 1.0 / (-1.0 + 2.0) * (-1.0 * w0 * w0 * Km3 + tl0 * Il);
+        tl[l] = tl0;
+        I1[l] = 1.0 / (1.0 + 1.0) * (spl * Rpl - sml * Rml + 1.0 * R0l * R0l * Il);
+    }
+    K1 = k1;
+    K2 = 1.0 / (1.0 + 2.0) * (1.0 * w0 * w0 * k1 + (tl[0] * I1[0] + tl[1] * I1[1] + tl[2] * I1[2]));
+}
+
+// G - (1/R - k^2 R / 2)/(4 pi), the smooth remainder (singularity_subtraction.f90:146-152)
+__device__ inline cd green_remainder(double R, double k) {
+    double f = 1.0 / (4 * PI_D) * 1.0 * 1.0 * (1.0 / R);
+    f = f + 1.0 / (4 * PI_D) * (k * k) * (-0.5) * R;
+    cd G0 = green(R, k);
+    return cmk(G0.x - f, G0.y);
+}
+
+// int_V G(rf, r') dV' over tet B (singularity_subtraction_int_V_G), 24-point rule
+__device__ cd int_V_G(v3 rf, double k, const double *tcB, double vB, double cut) {
+    cd intR = cmk(0, 0);
+    for (int i = 0; i < 24; ++i) {
+        v3 pb = tet_point(tcB, c_tet24_p[3 * i], c_tet24_p[3 * i + 1], c_tet24_p[3 * i + 2]);
+        double wb = c_tet24_w[i] * 6.0 * vB;
+        double RR = dist3(pb, rf);
+        cd II = (RR < cut) ? cmk(0.0, k / (4.0 * PI_D)) : green_remainder(RR, k);
+        intR = cadd(intR, cscale(II, wb));
+    }
+    double r4a = 0.0, r4b = 0.0;
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {
+        v3 p0, p1, p2;
+        tet_face(tcB, f, p0, p1, p2);
+        v3 n = tri_normal(p0, p1, p2);
+        double K1, K2;
+        analytic_tri(p0, p1, p2, n, rf, K1, K2);
+        double a1 = dot3(n, sub3(p0, rf));
+        r4a = r4a + a1 * K1 * 0.5;
+        r4b = r4b + a1 * K2 * 0.25;
+    }
+    double f2 = 1.0 / (4 * PI_D) * 1.0 * 1.0 * r4a;
+    f2 = f2 + 1.0 / (4 * PI_D) * (k * k) * (-0.5) * r4b;
+    return cmk(intR.x + f2, intR.y);
+}
+
 // ---- near-zone kernels -------------------------------------------------------
 // The elementary functions of these kernels, each within about an ulp: seeds
 // from the hardware reciprocals, refined; logarithm and arctangent as series in
@@ -458,7 +538,7 @@ __global__ __launch_bounds__(1024) void k_scan(uint32_t *__restrict__ tot, int n
 __global__ __launch_bounds__(64) void k_pair_fill(const int *__restrict__ cs, const int *__restrict__ perm, GridDesc g,
                                                   const uint32_t *__restrict__ base, uint32_t *__restrict__ pos,
                                                   int *__restrict__ PT, int *__restrict__ PB,
-                                                  uint8_t *__restrict__ PO) {
+                                                  uint8_t *__restrict__ PO, uint32_t *__restrict__ self) {
     const int c = blockIdx.x, lane = threadIdx.x, t0 = cs[c], n = cs[c + 1] - t0;
     uint32_t run = base[c];
     for (int s0 = 0; s0 < 27 * n; s0 += 64) {
@@ -476,6 +556,7 @@ __global__ __launch_bounds__(64) void k_pair_fill(const int *__restrict__ cs, co
         }
         const uint32_t p = run + (uint32_t)(inc - cnt);
         if (s < 27 * n) pos[(size_t)27 * t0 + s] = p;
+        if (s < 27 * n && o == 13) self[T] = p;  // in its own cube a tet's first basis tet is itself
         for (int i = 0; i < cnt; ++i) {
             PT[p + i] = T;
             PB[p + i] = b + i;
@@ -513,34 +594,161 @@ __global__ __launch_bounds__(64) void k_row_fill(const int *__restrict__ cs, con
 }
 
 // ---- near-zone G between box nodes for the 27 cube offsets ---------------------
-// Gtab[off][t] = G(node of the test box, node of the basis box) for the node
-// difference (tx, ty, tz) - 2, t = tx + 5 ty + 25 tz, plus the offset between
-// the boxes; 0 when the nodes coincide (compute_pG, src/precorrection.f90:21-46;
-// the 27 x 27 matrix of an offset has these 125 values)
+// Gtab[off][j][i] = G(node i of the test box, node j of the basis box), 0 when
+// the nodes coincide (compute_pG, src/precorrection.f90:21-46); i fastest, as the
+// lanes of k_near_blocks read it
 __global__ void k_pg_table(cd *__restrict__ Gtab, GridDesc gd, double k) {
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= 27 * 125) return;
-    const int t = e % 125, off = e / 125;
+    if (e >= 27 * 27 * 27) return;
+    const int i = e % 27, j = (e / 27) % 27, off = e / 729;
+    const int ox = off % 3 - 1, oy = (off / 3) % 3 - 1, oz = off / 9 - 1;
     // test box based at node (0,0,0) of a reference cube (2,2,2), basis box at
     // (2+2ox, 2+2oy, 2+2oz); coordinates as min + delta*index
-    const int dt[3] = {t % 5 - 2, (t / 5) % 5 - 2, t / 25 - 2};
-    const int o[3] = {off % 3 - 1, (off / 3) % 3 - 1, off / 9 - 1};
-    bool same = true;
-    double d2 = 0;
-    for (int c = 0; c < 3; ++c) {
-        // a pair of nodes with this difference: test node i, basis node i - dt
-        const int i = dt[c] > 0 ? dt[c] : 0, j = i - dt[c];
-        const int ti = 2 + i, bi = 2 + 2 * o[c] + j;
-        same = same && ti == bi;
-        const double a = (gd.min[c] + gd.delta * ti) - (gd.min[c] + gd.delta * bi);
-        d2 += a * a;
+    int ti[3] = {2 + i % 3, 2 + (i / 3) % 3, 2 + i / 9};
+    int bi[3] = {2 + 2 * ox + j % 3, 2 + 2 * oy + (j / 3) % 3, 2 + 2 * oz + j / 9};
+    cd v = cmk(0, 0);
+    if (!(ti[0] == bi[0] && ti[1] == bi[1] && ti[2] == bi[2])) {
+        double d2 = 0;
+        for (int c = 0; c < 3; ++c) {
+            double a = (gd.min[c] + gd.delta * ti[c]) - (gd.min[c] + gd.delta * bi[c]);
+            d2 += a * a;
+        }
+        v = green(sqrt(d2), k);
     }
-    Gtab[e] = same ? cmk(0, 0) : green(sqrt(d2), k);
+    Gtab[e] = v;
 }
 
 __device__ inline double wave_sum(double v) {
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
     return v;
+}
+
+// Self blocks (test tet = basis tet), one wave64 each, 4 per workgroup.  Their
+// entries are the largest of a row by one to two orders, so how they round to
+// complex64 decides the stored operator's error; they are evaluated operation
+// by operation as the reference does, closed-form remainders and arctangents
+// included, and stay apart from the reordered sums of k_near_blocks.  One block
+// of 77: 1.8 of 24 ms at 43,248 tets.
+__global__ __launch_bounds__(256) void k_self_blocks(
+    const uint32_t *__restrict__ self, const int *__restrict__ PT, const int *__restrict__ PB,
+    const uint8_t *__restrict__ POFF, int N, const double *__restrict__ tcoord, const double *__restrict__ vol,
+    const cd *__restrict__ param, const cd *__restrict__ S4, const cd *__restrict__ Gtab, double k,
+    cf *__restrict__ blocks) {
+    __shared__ cd u_s[4][4][27];  // per wave: G * S_B channels
+    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const long long t = (long long)blockIdx.x * 4 + wv;
+    const bool valid = t < N;
+    const size_t p = self[valid ? t : N - 1];  // idle waves recompute the last block, never store
+    const int T = PT[p], B = PB[p], off = POFF[p];
+    const double *tcT = tcoord + 12 * (size_t)T;
+    const double *tcB = tcoord + 12 * (size_t)B;
+    const double vT = vol[T], vB = vol[B];
+    const cd *ST = S4 + (size_t)T * 108, *SB = S4 + (size_t)B * 108;
+    const cd *G = Gtab + (size_t)off * 729;
+
+    // --- correction: u_c = G S_B[c]  (precorrect_const, src/precorrection.f90:50-82)
+    for (int e = lane; e < 108; e += 64) {
+        const int i = e % 27, ch = e / 27;
+        cd acc = cmk(0, 0);
+        for (int j = 0; j < 27; ++j) cfma(acc, G[27 * j + i], SB[j * 4 + ch]);
+        u_s[wv][ch][i] = acc;
+    }
+    __syncthreads();
+    // 10 bilinear forms: a = S_T . u_0 ; corr2(a,b) = D_a,T . u_{1+b}
+    cd cform = cmk(0, 0);
+    if (lane < 10) {
+        const int ca = lane == 0 ? 0 : 1 + (lane - 1) / 3;
+        const int cb = lane == 0 ? 0 : 1 + (lane - 1) % 3;
+        for (int i = 0; i < 27; ++i) cfma(cform, ST[i * 4 + ca], u_s[wv][cb][i]);
+    }
+
+    // --- V_V: 24-point rule on both tets (integrate_V_V_G, src/precorrection.f90:729-760)
+    cd vv = cmk(0, 0);
+    if (lane < 24) {
+        double wsum = 0.0;
+        for (int i = 0; i < 24; ++i) wsum += c_tet24_w[i] * 6.0 * vB;
+        const double cut = 1.0e-10 * pow(wsum, (double)(1.0f / 3.0f));
+        v3 rf = tet_point(tcT, c_tet24_p[3 * lane], c_tet24_p[3 * lane + 1], c_tet24_p[3 * lane + 2]);
+        double wt = c_tet24_w[lane] * 6.0 * vT;
+        vv = cscale(int_V_G(rf, k, tcB, vB, cut), wt);
+    }
+
+    // --- dV_dV: face pairs x 7-point rules (integrate_dV_dV_G, :764-806)
+    cd dd[9];
+#pragma unroll
+    for (int q = 0; q < 9; ++q) dd[q] = cmk(0, 0);
+    for (int item = lane; item < 112; item += 64) {
+        const int ft = item / 28, fb = (item / 7) % 4, i = item % 7;
+        v3 t0, t1, t2, b0, b1, b2;
+        tet_face(tcT, ft, t0, t1, t2);
+        tet_face(tcB, fb, b0, b1, b2);
+        v3 Tn = tri_normal(t0, t1, t2);
+        v3 Bn = tri_normal(b0, b1, b2);
+        double tww = tri_ww1(t0, t1, t2);
+        double bww = tri_ww1(b0, b1, b2);
+        v3 rf = tri_point(t0, t1, t2, c_tri7_p[2 * i], c_tri7_p[2 * i + 1]);
+        double wt = c_tri7_w[i] * tww;
+        double wsum = 0.0;
+        for (int j = 0; j < 7; ++j) wsum += c_tri7_w[j] * bww;
+        const double cut = 1.0e-10 * sqrt(wsum);
+        cd intR = cmk(0, 0);
+        for (int j = 0; j < 7; ++j) {
+            v3 pb = tri_point(b0, b1, b2, c_tri7_p[2 * j], c_tri7_p[2 * j + 1]);
+            double R = dist3(pb, rf);
+            cd II = (R < cut) ? cmk(0.0, k / (4.0 * PI_D)) : green_remainder(R, k);
+            intR = cadd(intR, cscale(II, c_tri7_w[j] * bww));
+        }
+        double K1, K2;
+        analytic_tri(b0, b1, b2, Bn, rf, K1, K2);
+        double f2 = 1.0 / (4 * PI_D) * 1.0 * 1.0 * K1;
+        f2 = f2 + 1.0 / (4 * PI_D) * (k * k) * (-0.5) * K2;
+        cd s = cscale(cmk(intR.x + f2, intR.y), wt);
+        const double tn[3] = {Tn.x, Tn.y, Tn.z}, bn[3] = {Bn.x, Bn.y, Bn.z};
+#pragma unroll
+        for (int a = 0; a < 3; ++a)
+#pragma unroll
+            for (int b = 0; b < 3; ++b) dd[a + 3 * b] = cadd(dd[a + 3 * b], cscale(s, tn[a] * bn[b]));
+    }
+
+    // --- reductions over the wave
+    double vvr = wave_sum(vv.x), vvi = wave_sum(vv.y);
+    double ddr[9], ddi[9];
+#pragma unroll
+    for (int q = 0; q < 9; ++q) {
+        ddr[q] = wave_sum(dd[q].x);
+        ddi[q] = wave_sum(dd[q].y);
+    }
+    double cfr[10], cfi[10];
+#pragma unroll
+    for (int q = 0; q < 10; ++q) {
+        cfr[q] = __shfl(cform.x, q, 64);
+        cfi[q] = __shfl(cform.y, q, 64);
+    }
+    if (lane == 0 && valid) {
+        const double sc = sqrt(vT * vB);
+        const double inv = 1.0 / sqrt(vB * vT);
+        const double k2 = k * k;
+        cd epsm1 = cmk(0, 0);
+        const bool self = (T == B);
+        if (self) {
+            cd e = param[T];
+            epsm1 = cdiv(cmk(1.0, 0.0), cmk(e.x - 1.0, e.y));
+        }
+#pragma unroll
+        for (int a = 0; a < 3; ++a)
+#pragma unroll
+            for (int b = 0; b < 3; ++b) {
+                cd corr = (a == b) ? cmk(cfr[0] * sc, cfi[0] * sc) : cmk(0, 0);
+                cd corr2 = cmk(cfr[1 + 3 * a + b] * sc, cfi[1 + 3 * a + b] * sc);
+                cd alok1 = (a == b) ? cmk(vvr, vvi) : cmk(0, 0);
+                cd t1 = csub(alok1, corr);
+                cd t2 = csub(cmk(ddr[a + 3 * b], ddi[a + 3 * b]), corr2);
+                cd inner = cadd(cmk(-k2 * t1.x, -k2 * t1.y), t2);
+                cd alok = (self && a == b) ? epsm1 : cmk(0, 0);
+                cd val = cadd(alok, cmk(inv * inner.x, inv * inner.y));
+                blocks[p * 9 + a + 3 * b] = make_float2((float)val.x, (float)val.y);
+            }
+    }
 }
 
 // quadrature point and rule weight
@@ -566,7 +774,7 @@ struct NearLds {
 // flat over the lanes: 24 x 24 volume pairs in 9 rounds, the 16 face pairs of
 // 7 x 7 points on 4 lanes each, and all 208 triangle integrals together in 4
 // rounds; points, normals and edges are computed once per block into LDS.
-// Measured at 43,248 tets (3.22 M blocks, ka 2): 23.2 ms, 3,350 vector
+// Measured at 43,248 tets (3.22 M blocks, ka 2): 23.5 ms, 3,350 vector
 // instructions per block at 83% of the issue rate.  With one quadrature point or
 // face pair per lane (24 and 112 of 64 and 128 lanes busy), closed-form
 // remainders and six atan per triangle it took 136.2 ms, with the flat layout and
@@ -574,18 +782,18 @@ struct NearLds {
 template <int SER, bool GENERAL>
 __global__ __launch_bounds__(64, 4) void k_near_blocks(
     const int *__restrict__ PT, const int *__restrict__ PB, const uint8_t *__restrict__ POFF,
-    const double *__restrict__ tcoord, const double *__restrict__ vol,
-    const cd *__restrict__ param, const cd *__restrict__ S4, const cd *__restrict__ Gtab, double k,
-    cf *__restrict__ blocks) {
+    const double *__restrict__ tcoord, const double *__restrict__ vol, const cd *__restrict__ S4,
+    const cd *__restrict__ Gtab, double k, cf *__restrict__ blocks) {
     __shared__ NearLds L;
     const int lane = threadIdx.x;
     const size_t p = blockIdx.x;
     const int T = PT[p], B = PB[p], off = POFF[p];
+    if (T == B) return;  // k_self_blocks
     const double *tcT = tcoord + 12 * (size_t)T;
     const double *tcB = tcoord + 12 * (size_t)B;
     const double vT = vol[T], vB = vol[B];
     const cd *ST = S4 + (size_t)T * 108;
-    const cd *G = Gtab + off * 125;
+    const cd *G = Gtab + off * 729;
     const double k4pi = k / (4.0 * PI_D), i4pi = 1.0 / (4.0 * PI_D), k2 = k * k;
 
     // --- points, normals, edges, S_B
@@ -633,14 +841,15 @@ __global__ __launch_bounds__(64, 4) void k_near_blocks(
     __syncthreads();
 
     // --- correction: u_c = G S_B[c]  (precorrect_const, src/precorrection.f90:50-82);
-    // lane (i, half): box node i, channels 2 half and 2 half + 1
+    // lane (i, half): box node i, channels 2 half and 2 half + 1.  The projections'
+    // weights alternate in sign and cancel by several digits, so these sums run in
+    // one fixed order, node by node
     if (lane < 54) {
         const int i = lane % 27, c = 2 * (lane / 27);
-        const int bi = i % 3 + 5 * ((i / 3) % 3) + 25 * (i / 9);
         cd a0 = cmk(0, 0), a1 = a0;
-#pragma unroll 3
+#pragma unroll 9
         for (int j = 0; j < 27; ++j) {
-            const cd g = G[62 + bi - (j % 3 + 5 * ((j / 3) % 3) + 25 * (j / 9))];
+            const cd g = G[27 * j + i];
             cfma(a0, g, L.SB[4 * j + c]);
             cfma(a1, g, L.SB[4 * j + c + 1]);
         }
@@ -648,20 +857,14 @@ __global__ __launch_bounds__(64, 4) void k_near_blocks(
         L.u[(c + 1) * 27 + i] = a1;
     }
     __syncthreads();
-    // 10 bilinear forms on 4 lanes each: S_T . u_0 ; corr2(a,b) = D_a,T . u_{1+b}
-    {
+    // 10 bilinear forms: S_T . u_0 ; corr2(a,b) = D_a,T . u_{1+b}
+    if (lane < 10) {
+        const int ca = lane == 0 ? 0 : 1 + (lane - 1) / 3;
+        const int cb = lane == 0 ? 0 : 1 + (lane - 1) % 3;
         cd c = cmk(0, 0);
-        const int q = lane >> 2;
-        if (q < 10) {
-            const int ca = q == 0 ? 0 : 1 + (q - 1) / 3;
-            const int cb = q == 0 ? 0 : 1 + (q - 1) % 3;
-            for (int i = lane & 3; i < 27; i += 4) cfma(c, ST[i * 4 + ca], L.u[cb * 27 + i]);
-        }
-        for (int o = 1; o < 4; o <<= 1) {
-            c.x += __shfl_xor(c.x, o, 64);
-            c.y += __shfl_xor(c.y, o, 64);
-        }
-        if (q < 10 && (lane & 3) == 0) L.form[q] = c;
+#pragma unroll 9
+        for (int i = 0; i < 27; ++i) cfma(c, ST[i * 4 + ca], L.u[cb * 27 + i]);
+        L.form[lane] = c;
     }
 
     // --- V_V: 24-point rule on both tets (integrate_V_V_G, src/precorrection.f90:729-760)
@@ -752,15 +955,8 @@ __global__ __launch_bounds__(64, 4) void k_near_blocks(
         const double inv = 1.0 / sqrt(vB * vT);
         const cd c1 = cscale(L.form[0], sc), c2 = cscale(L.form[1 + 3 * a + b], sc);
         cd inner = csub(dd, c2);
-        cd val = cmk(0, 0);
-        if (a == b) {
-            inner = cadd(inner, cmk(-k2 * (vvr - c1.x), -k2 * (vvi - c1.y)));
-            if (T == B) {
-                const cd e = param[T];
-                val = cdiv(cmk(1.0, 0.0), cmk(e.x - 1.0, e.y));
-            }
-        }
-        val = cadd(val, cscale(inner, inv));
+        if (a == b) inner = cadd(inner, cmk(-k2 * (vvr - c1.x), -k2 * (vvi - c1.y)));
+        const cd val = cscale(inner, inv);
         blocks[p * 9 + lane] = make_float2((float)val.x, (float)val.y);
     }
 }
@@ -891,27 +1087,27 @@ void launch_fg_octant(const cd *F, cd *fg, int Lx, int Ly, int Lz, hipStream_t s
     HIP_CHECK(hipGetLastError());
 }
 void launch_pg_table(cd *Gtab, const GridDesc &gd, double k, hipStream_t s) {
-    hipLaunchKernelGGL(k_pg_table, dim3((27 * 125 + 255) / 256), dim3(256), 0, s, Gtab, gd, k);
+    hipLaunchKernelGGL(k_pg_table, dim3((27 * 27 * 27 + 255) / 256), dim3(256), 0, s, Gtab, gd, k);
     HIP_CHECK(hipGetLastError());
 }
 void launch_near_pairs(const int *cube_start, const int *perm, const int64_t *row_start, const GridDesc &gd,
-                       uint32_t *pos, uint32_t *tot, int *PT, int *PB, uint8_t *PO, int *ent_col, uint32_t *ent_blk,
-                       hipStream_t s) {
+                       uint32_t *pos, uint32_t *tot, int *PT, int *PB, uint8_t *PO, uint32_t *self,
+                       int *ent_col, uint32_t *ent_blk, hipStream_t s) {
     const int nc = gd.ncx * gd.ncy * gd.ncz;
     hipLaunchKernelGGL(k_pair_count, dim3(nc), dim3(64), 0, s, cube_start, perm, gd, tot);
     hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, s, tot, nc);
-    hipLaunchKernelGGL(k_pair_fill, dim3(nc), dim3(64), 0, s, cube_start, perm, gd, tot, pos, PT, PB, PO);
+    hipLaunchKernelGGL(k_pair_fill, dim3(nc), dim3(64), 0, s, cube_start, perm, gd, tot, pos, PT, PB, PO, self);
     if (ent_blk)
         hipLaunchKernelGGL(k_row_fill, dim3(nc), dim3(64), 0, s, cube_start, perm, gd, row_start, pos, ent_col,
                            ent_blk);
     HIP_CHECK(hipGetLastError());
 }
-void launch_near_blocks(const int *PT, const int *PB, const uint8_t *POFF, long long P, const double *tcoord,
-                        const double *vol, const cd *param, const cd *S4, const cd *Gtab, double k, double reach,
-                        cf *blocks, hipStream_t s) {
+void launch_near_blocks(const int *PT, const int *PB, const uint8_t *POFF, const uint32_t *self, long long P, int N,
+                        const double *tcoord, const double *vol, const cd *param, const cd *S4, const cd *Gtab,
+                        double k, double reach, cf *blocks, hipStream_t s) {
     // the shortest series that covers every pair of points of the near zone
-    // (k reach bounds kR): at 43,248 tets 11 terms take 23.2 ms, 17 terms 24.9 ms
-    // and the general variant 31.8 ms (at ka 25, where part of the pairs take
+    // (k reach bounds kR): at 43,248 tets 11 terms take 23.5 ms, 17 terms 25.3 ms
+    // and the general variant 31.6 ms (at ka 25, where part of the pairs take
     // sincos)
     const double x = k * reach;
     auto kern = x <= SERIES_X_SHORT ? &k_near_blocks<SERIES_SHORT, false>
@@ -920,10 +1116,13 @@ void launch_near_blocks(const int *PT, const int *PB, const uint8_t *POFF, long 
     const long long maxb = 1LL << 30;
     for (long long p0 = 0; p0 < P; p0 += maxb) {
         const long long cnt = std::min(maxb, P - p0);
-        hipLaunchKernelGGL(kern, dim3((unsigned)cnt), dim3(64), 0, s, PT + p0, PB + p0, POFF + p0, tcoord, vol, param,
-                           S4, Gtab, k, blocks + p0 * 9);
+        hipLaunchKernelGGL(kern, dim3((unsigned)cnt), dim3(64), 0, s, PT + p0, PB + p0, POFF + p0, tcoord, vol, S4, Gtab,
+                           k, blocks + p0 * 9);
         HIP_CHECK(hipGetLastError());
     }
+    hipLaunchKernelGGL(k_self_blocks, dim3((N + 3) / 4), dim3(256), 0, s, self, PT, PB, POFF, N, tcoord, vol, param, S4,
+                       Gtab, k, blocks);
+    HIP_CHECK(hipGetLastError());
 }
 void launch_vswf(const double *tcoord, const double *vol, int N, int Nmax, double k, cd *mat, int ncol,
                  hipStream_t s) {

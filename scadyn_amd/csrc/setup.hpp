@@ -26,15 +26,15 @@ void launch_pg_table(cd *Gtab, const GridDesc &gd, double k, hipStream_t s);
 // Near-zone pairs in the reference's storage order (src/precorrection.f90:182-258:
 // test cube, near cube, test tet, basis tet with reference id >= the test
 // tet's): internal ids PT[p], PB[p] and cube offset PO[p] = (dx+1) + 3(dy+1) +
-// 9(dz+1).  With ent_blk also the block id (| BLK_TRANSPOSE) and column tet of
+// 9(dz+1).  self[t]: the block of tet t with itself.  With ent_blk also the block id (| BLK_TRANSPOSE) and column tet of
 // every row entry.  pos (27 N) and tot (N_cubes + 1) are scratch.
 void launch_near_pairs(const int *cube_start, const int *perm, const int64_t *row_start, const GridDesc &gd,
-                       uint32_t *pos, uint32_t *tot, int *PT, int *PB, uint8_t *PO, int *ent_col, uint32_t *ent_blk,
-                       hipStream_t s);
+                       uint32_t *pos, uint32_t *tot, int *PT, int *PB, uint8_t *PO, uint32_t *self,
+                       int *ent_col, uint32_t *ent_blk, hipStream_t s);
 // reach: a bound on the distance between points of two tets of the near zone
-void launch_near_blocks(const int *PT, const int *PB, const uint8_t *POFF, long long P, const double *tcoord,
-                        const double *vol, const cd *param, const cd *S4, const cd *Gtab, double k, double reach,
-                        cf *blocks, hipStream_t s);
+void launch_near_blocks(const int *PT, const int *PB, const uint8_t *POFF, const uint32_t *self, long long P, int N,
+                        const double *tcoord, const double *vol, const cd *param, const cd *S4, const cd *Gtab,
+                        double k, double reach, cf *blocks, hipStream_t s);
 void launch_vswf(const double *tcoord, const double *vol, int N, int Nmax, double k, cd *mat, int ncol,
                  hipStream_t s);
 
