@@ -526,19 +526,27 @@ static void make_matvec_space(scadyn_operator *op, int B, MatvecSpace &ms) {
     ms.grid1 = ms.mem.alloc<cd>(gsz);
     ms.in_off = ms.mem.alloc<long long>(B);
     ms.active = ms.mem.alloc<int>(B);
-    const size_t budget = 64 * 1024;
+    // Tile widths of the register kernel.  Transforms: 256 bytes of columns (16
+    // complex128, 32 complex64), half where that takes more than 64 KiB of LDS.
+    // Convolutions: 16 columns, 8 beyond 48 KiB; they are bound by instructions
+    // and latency, not by the width of their accesses, and more workgroups fit.
+    // Measured over lengths 24 to 270 and batches 3 to 64, widths 4 to 32: the rule
+    // is within 3% of the fastest width (convolution of 210 points, 64 slots,
+    // complex128: 8 columns 10.9 ms, 16 11.8; of 160 points 8 5.2, 16 4.6;
+    // complex64, 160 points: 16 2.7, 32 2.6; 105 points: 16 0.78, 32 0.85).
+    // Timing every width on the batch's own grids, as was done before, cost 45 ms of
+    // a 225 ms bar (43,248 tets, FP64).
+    const size_t budget = 64 * 1024, conv_budget = 48 * 1024;
     const bool reg = op->opts.fft_kernel == 0;
     for (int pr = 0; pr < 2; ++pr) {
         const size_t el = pr == 0 ? sizeof(cd) : sizeof(cf);
         make_line_pass(ms.pass[pr][0], Lx, Nx, Lx, nb, (long long)Ny * Nz, budget, el, reg);
         make_line_pass(ms.pass[pr][1], Ly, Ny, Ly, (long long)Lx * nb, Nz, budget, el, reg);
-        make_line_pass(ms.pass[pr][2], Lz, Nz, Nz, (long long)Ly * Lx * nb, 1, budget, el, reg);
+        make_line_pass(ms.pass[pr][2], Lz, Nz, Nz, (long long)Ly * Lx * nb, 1, conv_budget, el, reg, 16);
         make_line_pass(ms.pass[pr][3], Ly, Ly, Ny, (long long)Lx * nb, Nz, budget, el, reg);
         make_line_pass(ms.pass[pr][4], Lx, Lx, Nx, nb, (long long)Ny * Nz, budget, el, reg);
     }
 }
-
-static void tune_fft_tiles(scadyn_operator *op, MatvecSpace &ms);
 
 static Workspace &workspace(scadyn_operator *op, int B) {
     const int m = op->opts.maxit;
@@ -550,7 +558,6 @@ static Workspace &workspace(scadyn_operator *op, int B) {
     w.n = 3LL * op->g.N;
     const size_t nB = (size_t)w.n * B;
     make_matvec_space(op, B, w.mv);
-    tune_fft_tiles(op, w.mv);
     if (f16_basis(op)) {
         w.Vh = w.mem.alloc<ch>((size_t)(m + 1) * nB);
         w.Wf = w.mem.alloc<cf>(nB);
@@ -720,80 +727,6 @@ static void run_matvec(scadyn_operator *op, MatvecSpace &w, const C *xin, const 
                      c * (Nx * Ny * Nz * nB + 27.0 * 4 * g.N) + (c + 16.0) * 3 * g.N * w.B + 80.0 * op->nblocks);
         launch_gather_near<C>(a, op->s);
     }
-}
-
-// Autotuner of the line-FFT tiles.  For every register pass of a large batch
-// (and both precisions when the operator is mixed), each candidate tile width
-// (4 to 32 inner columns per workgroup) is timed on the batch's own grids and
-// the fastest kept; the planner's default wins ties within 3%.  Small grids
-// keep the default (tuning would cost more than it saves).
-template <typename C>
-static void run_pass(scadyn_operator *op, MatvecSpace &ms, int q, const LinePass &p) {
-    C *g0 = (C *)ms.grid0, *g1 = (C *)ms.grid1;
-    const C *tw = OpData<C>::tw(op);
-    const C *twq = q == 0 || q == 4 ? tw : (q == 1 || q == 3 ? tw + op->L[0] : tw + op->L[0] + op->L[1]);
-    if (q == 2) {
-        ConvInfo ci;
-        ci.Lx = op->L[0];
-        ci.Ly = op->L[1];
-        ci.Lz = op->L[2];
-        ci.Hx = op->Hh[0];
-        ci.Hy = op->Hh[1];
-        ci.nb = 4LL * ms.B;
-        launch_line_conv<C>(p, g0, g0, twq, OpData<C>::fg(op), ci, op->s);  // in place, as in run_matvec
-    } else {
-        launch_line_fft<C>(p, g0, g1, twq, q < 2 ? -1 : +1, op->s);
-    }
-}
-
-static void tune_fft_tiles(scadyn_operator *op, MatvecSpace &ms) {
-    const size_t gsz = (size_t)op->L[0] * op->L[1] * op->g.Nz * 4 * ms.B;
-    if (op->opts.fft_kernel != 0 || gsz < ((size_t)1 << 24)) return;
-    hipStream_t s = op->s;
-    HIP_CHECK(hipMemsetAsync(ms.grid0, 0, sizeof(cd) * gsz, s));
-    HIP_CHECK(hipMemsetAsync(ms.grid1, 0, sizeof(cd) * gsz, s));
-    hipEvent_t e0, e1;
-    HIP_CHECK(hipEventCreate(&e0));
-    HIP_CHECK(hipEventCreate(&e1));
-    // candidates may use the device's whole LDS per workgroup (160 KiB on MI355X;
-    // the planner's defaults stay within 64 KiB)
-    int lds_dev = 0;
-    HIP_CHECK(hipDeviceGetAttribute(&lds_dev, hipDeviceAttributeMaxSharedMemoryPerBlock, op->device));
-    const size_t budget = std::max<size_t>(64 * 1024, (size_t)lds_dev);
-    const int nprec = op->opts.precision == SCADYN_PREC_MIXED ? 2 : 1;
-    for (int pr = 0; pr < nprec; ++pr) {
-        if (pr == 1 && !op->d_fgf) break;  // no complex64 operator data yet
-        const size_t el = pr == 0 ? sizeof(cd) : sizeof(cf);
-        for (int q = 0; q < 5; ++q) {
-            LinePass &p = ms.pass[pr][q];
-            if (!p.reg) continue;
-            LinePass keep = p;
-            float best = 0.0f;
-            const int cand[] = {p.ti, 4, 8, 16, 32};
-            for (int ci = 0; ci < 5; ++ci) {
-                LinePass c = p;
-                if (ci > 0 && (cand[ci] == p.ti || !set_line_tile(c, cand[ci], budget, el))) continue;
-                for (int rep = 0; rep < 3; ++rep) {  // first run warms up
-                    if (rep == 1) HIP_CHECK(hipEventRecord(e0, s));
-                    if (pr == 0)
-                        run_pass<cd>(op, ms, q, c);
-                    else
-                        run_pass<cf>(op, ms, q, c);
-                }
-                HIP_CHECK(hipEventRecord(e1, s));
-                HIP_CHECK(hipEventSynchronize(e1));
-                float t = 0.0f;
-                HIP_CHECK(hipEventElapsedTime(&t, e0, e1));
-                if (ci == 0 || t < 0.97f * best) {
-                    best = t;
-                    keep = c;
-                }
-            }
-            p = keep;
-        }
-    }
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
 }
 
 // pack/unpack between host order [b][3N] (reference tets) and [row][B] (internal)

@@ -268,25 +268,15 @@ size_t line_pass_lds(const LinePass &p, size_t elem) {
 
 // Register-kernel tile width ti: the largest power of two <= want that fits the
 // inner extent, the LDS budget and the kernel's thread bound.
-static int reg_tile(int L, int rmax, long long inner, size_t lds_budget, size_t elem, int want) {
+static int reg_tile(int L, int rows, long long inner, size_t lds_budget, size_t elem, int want) {
     const int tmax = reg_max_threads(elem);
     int ti = want;
-    while (ti > 1 && (ti > inner || elem * ((size_t)L + (size_t)L * ti) > lds_budget || ti * rmax > tmax)) ti /= 2;
+    while (ti > 1 && (ti > inner || elem * ((size_t)L + (size_t)L * ti) > lds_budget || ti * rows > tmax)) ti /= 2;
     return ti;
 }
 
-bool set_line_tile(LinePass &p, int ti, size_t lds_budget, size_t elem) {
-    if (!p.reg) return false;
-    const int rmax = std::max(p.rad[0], p.rad[1]);
-    const int t = reg_tile(p.L, rmax, p.inner, lds_budget, elem, ti);
-    if (t != ti) return false;
-    p.ti = ti;
-    p.threads = ((ti * rmax + 63) / 64) * 64;
-    return true;
-}
-
 void make_line_pass(LinePass &p, int L, int n_in, int n_out, long long inner, long long outer, size_t lds_budget,
-                    size_t elem, bool allow_reg) {
+                    size_t elem, bool allow_reg, int want) {
     p.L = L;
     p.n_in = n_in;
     p.n_out = n_out;
@@ -301,15 +291,25 @@ void make_line_pass(LinePass &p, int L, int n_in, int n_out, long long inner, lo
         for (int r1 = 20; r1 >= 2; --r1)
             if (L % r1 == 0 && reg_radix_ok(r1) && reg_radix_ok(L / r1) && r1 >= L / r1) best = r1;
         if (best) {
-            const int r1 = best, r2 = L / best, rmax = std::max(r1, r2);
+            const int r1 = best, r2 = L / best;
+            // A thread holds R1 points in the radix-R1 stages, so in the others it
+            // takes as many items of R2 points as fit the same registers.  With
+            // R1 >= 2 R2 (105 = 15 x 7) that halves the threads of a tile, all of
+            // them busy in every stage, and twice the tiles are in flight
+            const int items = std::min(r1 / r2, 3), rows = (r1 + items - 1) / items;
             // tile: 16 columns of 16-byte or 32 of 8-byte elements (256 contiguous bytes per row)
-            const int ti = reg_tile(L, rmax, inner, lds_budget, elem, elem >= 16 ? 16 : 32);
+            const int ti = reg_tile(L, rows, inner, lds_budget, elem, want ? want : (elem >= 16 ? 16 : 32));
             p.reg = 1;
             p.nrad = 2;
             p.rad[0] = r1;
             p.rad[1] = r2;
             p.ti = ti;
-            p.threads = ((ti * rmax + 63) / 64) * 64;
+            p.rows = rows;
+            p.items = items;
+            p.threads = ((ti * rows + 63) / 64) * 64;
+            p.in_full = n_in / r2, p.in_rem = n_in % r2;
+            p.out_full = n_out / r1, p.out_rem = n_out % r1;
+            p.conv_full = n_out / r2, p.conv_rem = n_out % r2;
             return;
         }
     }

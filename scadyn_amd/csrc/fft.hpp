@@ -22,6 +22,13 @@ struct LinePass {
     int ti = 0;           // tile width (inner columns per workgroup)
     int reg = 0;          // 1: two-stage register kernel, rad = {R1, R2}
     int threads = 256;    // workgroup size
+    // register kernel: thread rows of a tile, and items of the radix-R2 stages per
+    // thread (R1 >= R2: those stages have R1 items, the radix-R1 stages R2)
+    int rows = 0, items = 1;
+    // register kernel: point j + r LR of an item exists for every item j < LR when
+    // r < full, and for j < rem when r == full; LR = R2 for the inputs, R1 for the
+    // outputs of a transform, R2 for those of a convolution
+    int in_full = 0, in_rem = 0, out_full = 0, out_rem = 0, conv_full = 0, conv_rem = 0;
 };
 
 // Thread bound of the register line-FFT kernel: complex64 instances take at
@@ -37,13 +44,10 @@ struct ConvInfo {
 };
 
 // allow_reg: use the two-stage register kernel when L = R1 R2 with both
-// radices in the register set
+// radices in the register set; want: its tile width (0: 256 bytes of columns)
 void make_line_pass(LinePass &p, int L, int n_in, int n_out, long long inner, long long outer, size_t lds_budget,
-                    size_t elem, bool allow_reg = true);
+                    size_t elem, bool allow_reg = true, int want = 0);
 bool reg_radix_ok(int r);
-// register kernel: switch the tile width to ti (a power of two); false when ti
-// does not fit the pass (then p is unchanged)
-bool set_line_tile(LinePass &p, int ti, size_t lds_budget, size_t elem);
 template <typename C>
 void launch_line_reg(const LinePass &p, const C *in, C *out, const C *tw, int sign, const C *fg, const ConvInfo &ci,
                      int mode, hipStream_t s);

@@ -244,42 +244,59 @@ struct Ctx {
     int c;         // column within the tile
     int j;         // item index within the stage
     int sh;        // log2 of the tile width
-    size_t in0;    // element (o, line point 0, i) of the input
-    size_t out0;   // element (o, line point 0, i) of the output
+    // element (o, line point j, i) of the input and output, i kept inside the
+    // slab: in0/out0 elements plus in_lane/out_lane bytes.  The kernel makes the
+    // first parts uniform over a wave (wave_base), so that an access is one
+    // scalar base and one 32-bit lane offset for all its points.
+    size_t in0, out0;
+    unsigned in_lane = 0, out_lane = 0;
 };
 
-// Addressing is incremental: every stage walks its R elements with a running
-// pointer or index (one add each) instead of a product per element.
+// Addressing costs no vector instruction per element where it can be avoided:
+// the points of an item lie a uniform step apart (scalar adds), the tile width
+// 2^SH is a compile-time constant (LDS offsets become immediates; SH < 0 takes it
+// from x.sh), and which points r of an item exist is uniform but for one r: r <
+// full for every item, r == full for items below rem, none beyond.  Address
+// arithmetic, compares and selects were 36% of the convolution's vector
+// instructions before.  With threads that hold R1 points in every stage
+// (LinePass::items) the z convolution of a 43,248-tet sphere (105^2 lines of 105 =
+// 15 x 7 points, 256 columns) went from 1,790 to 1,489 us in complex128 (latency:
+// 3 waves per SIMD) and from 878 to 724 us in complex64 (vector issue); 160 = 16 x
+// 10 points (76 planes of 160^2, 256 columns) from 5,787 to 5,591 us and from
+// 3,448 to 3,105 us.
 
 // stage 1: radix R, x[j + r (L/R)] from HBM (zero beyond n_in), DFT, LDS
-template <int R, int SIGN, typename C>
+template <int R, int SIGN, int SH, typename C>
 HD void stage_first(const C *__restrict__ in, C *lds, const LinePass &p, const Ctx &x) {
     const int LR = p.L / R;
     if (x.j >= LR) return;
+    const int sh = SH >= 0 ? SH : x.sh;
     C v[R];
     const size_t step = (size_t)LR * p.inner;
-    const C *src = in + x.in0 + (size_t)x.j * p.inner;
-    int n = x.j;
+    const C *src = in + x.in0;
     sfor<0, R>([&](auto rr) {
         constexpr int r = CV(rr);
-        v[r] = (x.col_ok && n < p.n_in) ? *src : czero<C>();
+        // items below lim have this point: a uniform bound, so one compare
+        const int lim = r < p.in_full ? LR : (r == p.in_full ? p.in_rem : 0);
+        v[r] = czero<C>();
+        if (x.j < lim) v[r] = *reinterpret_cast<const C *>(reinterpret_cast<const char *>(src) + x.in_lane);
         src += step;
-        n += LR;
     });
     RDFT<R, SIGN, C>::run(v);
-    const int lb = ((x.j * R) << x.sh) + x.c;
+    const int lb = ((x.j * R) << sh) + x.c;
     sfor<0, R>([&](auto rr) {
         constexpr int r = CV(rr);
-        lds[lb + (r << x.sh)] = v[r];
+        lds[lb + (r << sh)] = v[r];
     });
 }
 
 // stage 2 operand load: LDS[j + r (L/R)] * W_L^(SIGN j r), then DFT
-template <int R, int SIGN, typename C>
-HD void stage_second(C *v, const C *lds, const C *tw, const LinePass &p, const Ctx &x) {
+template <int R, int SIGN, int SH, typename C>
+HD void stage_second(C *v, const C *lds, const C *tw, const LinePass &p, const Ctx &x, int j) {
     const int LR = p.L / R;
-    const int ls = LR << x.sh;
-    int li = (x.j << x.sh) + x.c;
+    const int sh = SH >= 0 ? SH : x.sh;
+    const int ls = LR << sh;
+    int li = (j << sh) + x.c;
     sfor<0, R>([&](auto rr) {
         constexpr int r = CV(rr);
         v[r] = lds[li];
@@ -288,7 +305,7 @@ HD void stage_second(C *v, const C *lds, const C *tw, const LinePass &p, const C
     int ti = 0;  // j r
     sfor<1, R>([&](auto rr) {
         constexpr int r = CV(rr);
-        ti += x.j;
+        ti += j;
         C w = tw[ti];
         if constexpr (SIGN > 0) w.y = -w.y;
         v[r] = cmul(v[r], w);
@@ -296,23 +313,23 @@ HD void stage_second(C *v, const C *lds, const C *tw, const LinePass &p, const C
     RDFT<R, SIGN, C>::run(v);
 }
 
-// stage 2 to HBM: outputs k = j + r (L/R), cropped to n_out
-template <int R, int SIGN, typename C>
-HD void stage_last(C *__restrict__ out, const C *lds, const C *tw, const LinePass &p,
-                                           const Ctx &x) {
-    const int LR = p.L / R;
-    if (x.j >= LR) return;
+// stage 2 to HBM: outputs k = j + r (L/R), cropped to n_out (full, rem: as
+// p.in_full and p.in_rem for the outputs of this stage)
+template <int R, int SIGN, int SH, typename C>
+HD void stage_last(C *__restrict__ out, const C *lds, const C *tw, const LinePass &p, const Ctx &x, int full,
+                   int rem, int m = 0) {
+    const int LR = p.L / R, j = x.j + m * p.rows;
+    if (j >= LR) return;
     C v[R];
-    stage_second<R, SIGN, C>(v, lds, tw, p, x);
+    stage_second<R, SIGN, SH, C>(v, lds, tw, p, x, j);
     if (!x.col_ok) return;
     const size_t step = (size_t)LR * p.inner;
-    C *dst = out + x.out0 + (size_t)x.j * p.inner;
-    int k = x.j;
+    C *dst = out + x.out0 + (size_t)(m * p.rows) * p.inner;
     sfor<0, R>([&](auto rr) {
         constexpr int r = CV(rr);
-        if (k < p.n_out) *dst = v[r];
+        const int lim = r < full ? LR : (r == full ? rem : 0);
+        if (j < lim) *reinterpret_cast<C *>(reinterpret_cast<char *>(dst) + x.out_lane) = v[r];
         dst += step;
-        k += LR;
     });
 }
 
@@ -320,37 +337,43 @@ HD void stage_last(C *__restrict__ out, const C *lds, const C *tw, const LinePas
 // stage 1 (radix R) on the same registers.  The inner index is below 2^31
 // (make_line_pass keeps larger passes off the register kernel), so the grid
 // point is found with 32-bit divisions.
-template <int R, typename C>
+template <int R, int SH, typename C>
 HD void conv_compute(C *v, const C *lds, const C *tw, const C *__restrict__ fg, const ConvInfo &ci, const LinePass &p,
-                     const Ctx &x) {
-    const int LR = p.L / R;
-    if (x.j >= LR) return;
-    stage_second<R, -1, C>(v, lds, tw, p, x);
-    if (x.col_ok) {
-        const unsigned xy = (unsigned)x.i / (unsigned)ci.nb;
+                     const Ctx &x, int m) {
+    const int LR = p.L / R, j = x.j + m * p.rows;
+    if (j >= LR) return;
+    stage_second<R, -1, SH, C>(v, lds, tw, p, x, j);
+    {
+        // a column beyond the slab takes column 0's factors (its outputs are not stored)
+        const unsigned xy = (x.col_ok ? (unsigned)x.i : 0u) / (unsigned)ci.nb;
         const int gy = (int)(xy / (unsigned)ci.Lx), gx = (int)(xy - (unsigned)gy * (unsigned)ci.Lx);
         const int kx = imin(gx, ci.Lx - gx), ky = imin(gy, ci.Ly - gy);
-        const C *f = fg + (size_t)ky * ci.Hx + kx;
-        const int zs = ci.Hy * ci.Hx;
-        int k = x.j;
+        // row min(k, Lz - k) of the octant as the smaller of two running byte
+        // offsets, in 32 bits (the octant is checked to stay below 2^32 bytes)
+        const unsigned zs = (unsigned)(ci.Hy * ci.Hx) * (unsigned)sizeof(C);
+        const unsigned f0 = (unsigned)(ky * ci.Hx + kx) * (unsigned)sizeof(C), step = (unsigned)LR * zs;
+        unsigned up = f0 + (unsigned)j * zs, down = f0 + (unsigned)(ci.Lz - j) * zs;
         sfor<0, R>([&](auto rr) {
             constexpr int r = CV(rr);
-            const int kz = imin(k, ci.Lz - k);
-            v[r] = cmul(v[r], f[(size_t)kz * zs]);
-            k += LR;
+            const unsigned f = up < down ? up : down;
+            v[r] = cmul(v[r], *reinterpret_cast<const C *>(reinterpret_cast<const char *>(fg) + f));
+            up += step;
+            down -= step;
         });
     }
     RDFT<R, +1, C>::run(v);
 }
 
 // second half, after a barrier: the inverse stage-1 outputs to LDS
-template <int R, typename C>
-HD void conv_store(const C *v, C *lds, const LinePass &p, const Ctx &x) {
-    if (x.j >= p.L / R) return;
-    const int lb = ((x.j * R) << x.sh) + x.c;
+template <int R, int SH, typename C>
+HD void conv_store(const C *v, C *lds, const LinePass &p, const Ctx &x, int m) {
+    const int j = x.j + m * p.rows;
+    if (j >= p.L / R) return;
+    const int sh = SH >= 0 ? SH : x.sh;
+    const int lb = ((j * R) << sh) + x.c;
     sfor<0, R>([&](auto rr) {
         constexpr int r = CV(rr);
-        lds[lb + (r << x.sh)] = v[r];
+        lds[lb + (r << sh)] = v[r];
     });
 }
 
@@ -370,8 +393,9 @@ HD Ctx make_ctx(const LinePass &p, long long block, int thread) {
     x.j = thread >> x.sh;
     x.i = i0 + x.c;
     x.col_ok = x.i < p.inner;
-    x.in0 = (size_t)x.o * p.n_in * (size_t)p.inner + (size_t)x.i;
-    x.out0 = (size_t)x.o * p.n_out * (size_t)p.inner + (size_t)x.i;
+    const size_t il = (size_t)(x.col_ok ? x.i : p.inner - 1);
+    x.in0 = ((size_t)x.o * p.n_in + x.j) * (size_t)p.inner + il;
+    x.out0 = ((size_t)x.o * p.n_out + x.j) * (size_t)p.inner + il;
     return x;
 }
 
@@ -379,21 +403,27 @@ HD Ctx make_ctx(const LinePass &p, long long block, int thread) {
 // of sign s): phase 0 = stage 1, phase 1 = stage 2.  MODE 1 (forward, x Fg,
 // inverse): phase 0 = forward stage 1, phase 1 = conv_compute (registers v),
 // phase 2 = conv_store, phase 3 = inverse stage 2.
-template <int MODE, typename C, int RMAX = 20>
+template <int MODE, typename C, int RMAX = 20, int SH = -1>
 HD void line_reg_phase(int phase, const C *__restrict__ in, C *__restrict__ out, C *lds, const C *tw,
                        const C *__restrict__ fg, const ConvInfo &ci, const LinePass &p, const Ctx &x, int sign,
                        C *v) {
     // RMAX: largest radix compiled into this instance (fewer VGPRs for small radices)
     const int R1 = p.rad[0], R2 = p.rad[1];
     const int s1 = (MODE == 0) ? sign : -1;
+    // the radix-R2 stages' items of a thread: x.j + m p.rows, m < p.items
+    auto second = [&](auto &&f) {
+        f(std::integral_constant<int, 0>{});
+        if (p.items > 1) f(std::integral_constant<int, 1>{});
+        if (p.items > 2) f(std::integral_constant<int, 2>{});
+    };
     if (phase == 0) {
 #define FIRST(R)                                          \
     case R:                                               \
         if constexpr (R <= RMAX) {                        \
             if (s1 < 0)                                   \
-                stage_first<R, -1, C>(in, lds, p, x);     \
+                stage_first<R, -1, SH, C>(in, lds, p, x);     \
             else                                          \
-                stage_first<R, +1, C>(in, lds, p, x);     \
+                stage_first<R, +1, SH, C>(in, lds, p, x);     \
         }                                                 \
         break;
         switch (R1) { REG_RADICES(FIRST) }
@@ -403,9 +433,13 @@ HD void line_reg_phase(int phase, const C *__restrict__ in, C *__restrict__ out,
     case R:                                                     \
         if constexpr (R <= RMAX) {                              \
             if (s1 < 0)                                         \
-                stage_last<R, -1, C>(out, lds, tw, p, x);       \
+                second([&](auto m) {                                    \
+                    stage_last<R, -1, SH, C>(out, lds, tw, p, x, p.out_full, p.out_rem, CV(m)); \
+                });                                                     \
             else                                                \
-                stage_last<R, +1, C>(out, lds, tw, p, x);       \
+                second([&](auto m) {                                    \
+                    stage_last<R, +1, SH, C>(out, lds, tw, p, x, p.out_full, p.out_rem, CV(m)); \
+                });                                                     \
         }                                                       \
         break;
         switch (R2) { REG_RADICES(LAST) }
@@ -413,21 +447,28 @@ HD void line_reg_phase(int phase, const C *__restrict__ in, C *__restrict__ out,
     } else if (phase == 1) {
 #define MID(R)                                                                     \
     case R:                                                                        \
-        if constexpr (R <= RMAX) conv_compute<R, C>(v, lds, tw, fg, ci, p, x);     \
+        if constexpr (R <= RMAX)                                                   \
+            second([&](auto m) {                                                   \
+                if constexpr ((CV(m) + 1) * R <= RMAX)                             \
+                    conv_compute<R, SH, C>(v + CV(m) * R, lds, tw, fg, ci, p, x, CV(m)); \
+            });                                                                    \
         break;
         switch (R2) { REG_RADICES(MID) }
 #undef MID
     } else if (phase == 2) {
 #define STO(R)                                                   \
     case R:                                                      \
-        if constexpr (R <= RMAX) conv_store<R, C>(v, lds, p, x); \
+        if constexpr (R <= RMAX)                                 \
+            second([&](auto m) {                                 \
+                if constexpr ((CV(m) + 1) * R <= RMAX) conv_store<R, SH, C>(v + CV(m) * R, lds, p, x, CV(m)); \
+            });                                                  \
         break;
         switch (R2) { REG_RADICES(STO) }
 #undef STO
     } else {
 #define ILAST(R)                                                            \
     case R:                                                                 \
-        if constexpr (R <= RMAX) stage_last<R, +1, C>(out, lds, tw, p, x);  \
+        if constexpr (R <= RMAX) stage_last<R, +1, SH, C>(out, lds, tw, p, x, p.conv_full, p.conv_rem);  \
         break;
         switch (R1) { REG_RADICES(ILAST) }
 #undef ILAST

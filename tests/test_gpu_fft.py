@@ -40,6 +40,30 @@ def test_register_vs_stockham(n_cells, fft_pad):
     b.close()
 
 
+@pytest.mark.parametrize('body,nrhs', [('ellipsoid', 1), ('ellipsoid', 3), ('ellipsoid', 33), ('sphere', 2),
+                                       ('sphere', 17)])
+def test_register_widths(body, nrhs):
+    """Tile widths and items per thread: axes of 112, 90 and 75 points (75 = 15 x 5:
+    three items a thread) and of 105 (15 x 7: two), with 4 to 132 columns a grid
+    point: narrower than every compiled width, partial last tiles, full ones."""
+    from scadyn_amd import meshgen, native
+    c, e = meshgen.gaussian_ellipsoid(n_cells=28) if body == 'ellipsoid' else meshgen.sphere(24)
+    c = meshgen.rescale_to_radius(c, e, 1e-7)
+    param = np.full(e.shape[0], 2.5 + 0.01j)
+    a = native.Operator(c, e, param, 2e7, precision=native.PREC_MIXED)
+    b = native.Operator(c, e, param, 2e7, precision=native.PREC_MIXED, fft_kernel=1)
+    inf = a.info()
+    say(f"{e.shape[0]} tets, {nrhs} vectors, fft {inf['Lx']}x{inf['Ly']}x{inf['Lz']}")
+    x = np.random.default_rng(9).standard_normal((2, nrhs, 3 * e.shape[0]))
+    x = x[0] + 1j * x[1]
+    for prec, tol in ((native.PREC_FP64, 1e-13), (native.PREC_MIXED, 2e-6)):
+        ya, yb = a.matvec(x, precision=prec), b.matvec(x, precision=prec)
+        for r in range(nrhs):
+            assert rel(ya[r], yb[r]) < tol
+    a.close()
+    b.close()
+
+
 def test_tuned_tiles():
     """A batch whose grids are large enough to be tuned (64 columns): the tile
     widths chosen are powers of two the kernels support, and the tuned matvec
