@@ -14,6 +14,7 @@
 #include <thread>
 
 #include "fft.hpp"
+#include "gather_core.hpp"
 #include "internal.hpp"
 #include "krylov.hpp"
 #include "matvec.hpp"
@@ -185,6 +186,8 @@ struct scadyn_operator {
     int *d_tet_cube = nullptr, *d_cube_start = nullptr, *d_perm = nullptr;
     int *d_ne_cubes = nullptr;  // non-empty cubes
     int n_ne_cubes = 0;
+    int2 *d_groups = nullptr;  // row groups of the gather
+    int n_groups = 0;
     cf *d_blocks = nullptr;
     int64_t *d_row_start = nullptr;
     int *d_ent_col = nullptr;
@@ -420,6 +423,16 @@ static void create_operator(scadyn_operator *op, const scadyn_mesh &mesh, const 
         std::vector<int> ne;
         for (const auto &kc : key) ne.push_back(kc.second);
         op->n_ne_cubes = (int)ne.size();
+        std::vector<int2> groups;
+        for (int c : ne) {
+            const int t0 = g.cube_start[c], n = g.cube_start[c + 1] - t0, k = (n + gcore::ROW_GT - 1) / gcore::ROW_GT;
+            for (int q = 0; q < k; ++q) {  // equal parts
+                const int a = t0 + (int)((long long)n * q / k), b = t0 + (int)((long long)n * (q + 1) / k);
+                groups.push_back(make_int2(c, 8 * a + (b - a)));
+            }
+        }
+        op->n_groups = (int)groups.size();
+        op->d_groups = M.upload(groups, s);
         if (!ne.empty()) op->d_ne_cubes = M.upload(ne, s);
     }
     {
@@ -680,6 +693,8 @@ static void run_matvec(scadyn_operator *op, MatvecSpace &w, const C *xin, const 
     a.blocks = op->d_blocks;
     a.ne_cubes = op->d_ne_cubes;
     a.n_ne = op->n_ne_cubes;
+    a.groups = op->d_groups;
+    a.n_groups = op->n_groups;
     a.k2 = op->k * op->k;
     a.slot_active = active;
     a.gather_kernel = op->opts.gather_kernel;
@@ -1314,7 +1329,7 @@ static Footprint footprint_of(const HostGeometry &g, long long P, const scadyn_o
         H[c] = L[c] / 2 + 1;
     }
     const size_t cdb = sizeof(cd);
-    f.op = N * (96 + 8 + 16 + 4 + 4) + 4 * (g.N_cubes + 1) + 1728 * N + 72 * (size_t)P + 8 * (N + 1) +
+    f.op = N * (96 + 8 + 16 + 4 + 4 + 8) + 4 * (g.N_cubes + 1) + 1728 * N + 72 * (size_t)P + 8 * (N + 1) +
            8 * 2 * (size_t)P + cdb * H[0] * H[1] * H[2] + cdb * (L[0] + L[1] + L[2]);
     if (o.precision == SCADYN_PREC_MIXED) f.op += 864 * N + 8 * H[0] * H[1] * H[2];
     f.setup = 2 * cdb * L[0] * L[1] * L[2] + 9 * (size_t)P + 4 * (28 * N + g.N_cubes) + cdb * 27 * 27 * 27 + cdb * 98 * 27;

@@ -7,8 +7,8 @@
 //    read as wave-uniform broadcasts while each lane streams its slot's 27 box
 //    nodes (gather, src/sparse.f90:47-77, and Y2 - k^2 Y,
 //    src/gmres_module.f90:148-153);
-//  * near part (matmul_Acorr_const, src/sparse_mat.f90:96-123): for each near
-//    cube, in chunks of VC column tets, lane (u, v) = (lane / VC, lane % VC)
+//  * near part (matmul_Acorr_const, src/sparse_mat.f90:96-123): for each x line of
+//    near cubes, in chunks of VC column tets, lane (u, v) = (lane / VC, lane % VC)
 //    fetches the block of row tet u and column tet v and stores it (complex64,
 //    as stored) as a dense 3x3, transposed when the pair is stored as (v, u);
 //    every lane then widens the chunk's blocks to the matvec precision and
@@ -16,7 +16,7 @@
 // The rows of a cube's tets list the near tets in the same order (near cube
 // offset, then tet id), so entry q of every row of the cube is column q.
 //
-// Work order.  Item w is (slot chunk w / n_ne, cube ne_cubes[w % n_ne]): one
+// Work order.  Item w is (slot chunk w / n, cube or row group w % n): one
 // chunk sweeps all cubes before the next, and the workgroups are renumbered so
 // that each XCD runs one contiguous range of items (xcd_remap).  Neighbouring
 // cubes then run at the same time on the same XCD, and the x of a near tet that
@@ -52,9 +52,27 @@ struct GatherArgs {
     double k2;
     const int *slot_active;
     cd *y;
+    // row groups of the vector kernel: cube, 8 x first row tet + rows (at most ROW_GT)
+    const int2 *groups = nullptr;
+    int n_groups = 0;
 };
 
-// row tets per pass (8 covers all tets of nearly every cube of a cube-split
+// Row tets and near columns per pass of the vector kernel: a wave takes a group
+// of up to ROW_GT tets of a cube (a cube of 6 is two waves), and one staged chunk
+// covers the columns of an x line of three near cubes (about 18; ROW_GT x ROW_VC <=
+// 64: one block per lane).
+//  * With all tets of a cube in one wave, 43,248 tets had 7,213 waves for the 1,024
+//    SIMDs (7.04 each, the last ones alone), three to a SIMD: vector issue
+//    43% busy.
+//  * A chunk is a chain of two dependent loads (entry, block) before its first use;
+//    27 chunks of one near cube each waited for it 27 times a pass.
+// Measured per launch, 64 slots, complex128 / complex64: 43,248 tets 1,632 / 768 us
+// before, 1,424 / 699 with these groups and one slot a lane, 1,275 / 613 with the
+// wave layout below; 146,784 tets 4,224 / 2,436 before, 3,415 / 2,023 now; 32 slots
+// of 369,390 tets 9,539 / 5,118 before, 4,732 / 2,972 now.  Groups of 2, 4 and 6 rows
+// (32, 16 and 10 columns) ran at 1,333 / 700, 1,411 / 706 and 1,410 / 649 us.
+constexpr int ROW_GT = 3, ROW_VC = 21;
+// of the matrix-core kernel (8 covers all tets of nearly every cube of a cube-split
 // mesh, so the near-zone x of a cube is fetched once) and column tets per
 // staged near chunk (GT x VC = 64: one block per lane)
 constexpr int GATHER_GT = 8, GATHER_VC = 8;
@@ -78,13 +96,11 @@ struct Item {
 };
 
 template <typename C>
-GC_HD Item make_item(const GatherArgs<C> &g, long long w, int lane) {
-    const int ci = (int)(w % g.n_ne);
-    const int braw = (int)(w / g.n_ne) * 64 + lane;
+GC_HD Item cube_item(const GatherArgs<C> &g, int c, int braw) {
     Item it;
     it.valid = braw < g.B;
     it.b = it.valid ? braw : g.B - 1;
-    it.c = g.ne_cubes[ci];
+    it.c = c;
     it.cx = it.c % g.ncx;
     it.cy = (it.c / g.ncx) % g.ncy;
     it.cz = it.c / (g.ncx * g.ncy);
@@ -92,6 +108,19 @@ GC_HD Item make_item(const GatherArgs<C> &g, long long w, int lane) {
     it.t1 = g.cube_start[it.c + 1];
     it.act = g.slot_active ? g.slot_active[it.b] != 0 : true;
     it.base = (size_t)(2 * it.cx) + (size_t)g.Nx * ((size_t)(2 * it.cy) + (size_t)g.Ny * (2 * it.cz));
+    return it;
+}
+template <typename C>
+GC_HD Item make_item(const GatherArgs<C> &g, long long w, int lane) {
+    return cube_item(g, g.ne_cubes[w % g.n_ne], (int)(w / g.n_ne) * 64 + lane);
+}
+// row group i of the list: t0 .. t1 - 1 are the group's rows
+template <typename C>
+GC_HD Item group_item(const GatherArgs<C> &g, int i) {
+    const int2 q = g.groups[i];
+    Item it = cube_item(g, q.x, 0);
+    it.t0 = q.y >> 3;
+    it.t1 = it.t0 + (q.y & 7);
     return it;
 }
 
@@ -224,21 +253,118 @@ GC_HD void write_out(const GatherArgs<C> &g, const Item &it, int tp, C (*acc)[3]
     }
 }
 
-// the near cubes of (cx, cy, cz) in row order; calls f(first tet, end tet)
+// ---- wave layout of the vector kernel ------------------------------------------
+// SB lanes hold NS slots each (slot, slot + SB), and the 64 / SB lane groups share
+// the columns of a chunk and the nodes of the box; the groups' sums are combined at
+// the end.  Every operand read from LDS then serves NS slots and 64 / SB columns.
+// A wave-wide LDS read returns its 64 copies at 128 bytes a cycle, also when all
+// lanes read one address: with one slot per lane and one column at a time the
+// block reads alone took the CU's LDS as long as the FMAs took its four SIMDs, and
+// every block was widened to complex128 once per wave and slot chunk.
+template <int SB, int NS>
+struct Slots {
+    int s[NS];      // slot used for loads
+    bool ok[NS];    // lane holds a real slot
+    int grp;        // lane group
+};
+template <int SB, int NS, typename C>
+GC_HD Slots<SB, NS> lane_slots(const GatherArgs<C> &g, int chunk, int lane) {
+    Slots<SB, NS> r;
+    r.grp = lane / SB;
+#pragma unroll
+    for (int i = 0; i < NS; ++i) {
+        const int b = chunk * (SB * NS) + i * SB + lane % SB;
+        r.ok[i] = b < g.B;
+        r.s[i] = r.ok[i] ? b : g.B - 1;
+    }
+    return r;
+}
+
+// the lane group's share of y_c += S_{c+1}^T g3 - k^2 S^T g_c over the 27 box nodes
+template <typename C, int NT, int SB, int NS>
+GC_HD void grid_share(const GatherArgs<C> &g, const Item &it, const Slots<SB, NS> &sl, const C *sm,
+                      C (*acc)[3][NS]) {
+    constexpr int G = 64 / SB;
+    typedef typename Prec<C>::real R;
+    const R kk = (R)g.k2;
+    const size_t B = (size_t)g.B;
+#pragma unroll 1
+    for (int j = sl.grp; j < 27; j += G) {
+        const C *gp = g.grid + (it.base + j % 3 + (size_t)g.Nx * ((j / 3) % 3 + (size_t)g.Ny * (j / 9))) * 4 * B;
+        C v[4][NS];
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+            for (int i = 0; i < NS; ++i) v[c][i] = gp[c * B + sl.s[i]];
+#pragma unroll
+        for (int u = 0; u < NT; ++u) {
+            const C *s = sm + u * 108 + j * 4;
+            const C s0 = cscale(s[0], -kk), s1 = s[1], s2 = s[2], s3 = s[3];
+#pragma unroll
+            for (int i = 0; i < NS; ++i) {
+                cfma(acc[u][0][i], s0, v[0][i]);
+                cfma(acc[u][1][i], s0, v[1][i]);
+                cfma(acc[u][2][i], s0, v[2][i]);
+                cfma(acc[u][0][i], s1, v[3][i]);
+                cfma(acc[u][1][i], s2, v[3][i]);
+                cfma(acc[u][2][i], s3, v[3][i]);
+            }
+        }
+    }
+}
+
+// the lane group's columns (grp, grp + 64 / SB, ...) of the staged blocks of column
+// tets v0 .. v0+nv-1; x of the next column is fetched while one is applied
+template <typename C, int NT, int VC, int SB, int NS>
+GC_HD void chunk_share(const GatherArgs<C> &g, const Slots<SB, NS> &sl, const long long *off, int v0, int nv,
+                       const cf *sm, C (*acc)[3][NS]) {
+    constexpr int G = 64 / SB;
+    const size_t B = (size_t)g.B;
+    C n[3][NS];
+    auto fetch = [&](int v) {
+        const C *xb = g.xin + (size_t)(3 * (v0 + v)) * B;
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+            for (int i = 0; i < NS; ++i) n[c][i] = xb[c * B + off[i]];
+    };
+    if (sl.grp < nv) fetch(sl.grp);
+#pragma unroll 1
+    for (int v = sl.grp; v < nv; v += G) {
+        C x[3][NS];
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+            for (int i = 0; i < NS; ++i) x[c][i] = n[c][i];
+        if (v + G < nv) fetch(v + G);
+#pragma unroll
+        for (int u = 0; u < NT; ++u) {
+            const cf *m = sm + (u * VC + v) * 9;  // column-major 3x3
+#pragma unroll
+            for (int r = 0; r < 3; ++r)
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                    const C a = Prec<C>::from(m[r + 3 * c]);
+#pragma unroll
+                    for (int i = 0; i < NS; ++i) cfma(acc[u][r][i], a, x[c][i]);
+                }
+        }
+    }
+}
+
+// the near cubes of (cx, cy, cz) in row order, those of one x line together
+// (their tets are consecutive); calls f(first tet, end tet)
 template <typename C, typename F>
 GC_HD void for_near_cubes(const GatherArgs<C> &g, const Item &it, F &&f) {
+    const int x0 = it.cx > 0 ? it.cx - 1 : 0, x1 = it.cx + 1 < g.ncx ? it.cx + 1 : it.cx;
     for (int dz = -1; dz <= 1; ++dz) {
         const int zz = it.cz + dz;
         if (zz < 0 || zz >= g.ncz) continue;
         for (int dy = -1; dy <= 1; ++dy) {
             const int yy = it.cy + dy;
             if (yy < 0 || yy >= g.ncy) continue;
-            for (int dx = -1; dx <= 1; ++dx) {
-                const int xx = it.cx + dx;
-                if (xx < 0 || xx >= g.ncx) continue;
-                const int nc = xx + g.ncx * (yy + g.ncy * zz);
-                f(g.cube_start[nc], g.cube_start[nc + 1]);
-            }
+            const int line = g.ncx * (yy + g.ncy * zz);
+            f(g.cube_start[line + x0], g.cube_start[line + x1 + 1]);
         }
     }
 }

@@ -24,6 +24,7 @@ void build_geometry(const scadyn_mesh &mesh, const scadyn_opts &opts, HostGeomet
     if (opts.near_zone != 1) fail(SCADYN_ERR_UNSUPPORTED, "only near_zone = 1 is implemented");
     if (opts.order != 0) fail(SCADYN_ERR_UNSUPPORTED, "only basis order 0 is implemented");
     const int N = mesh.n_tet, Nn = mesh.n_node;
+    if (N >= 1 << 28) fail(SCADYN_ERR_UNSUPPORTED, "more than 2^28 tets");
     g.N = N;
     g.Nnode = Nn;
     const double *X = mesh.coord;

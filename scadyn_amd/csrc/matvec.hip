@@ -13,45 +13,71 @@
 
 namespace scadyn {
 
-// scatter (sparse_T_matmul, src/sparse.f90:13-43, + vec2arr2), node-centric:
-// node p sums the stencil weights of the tets of the <= 8 cubes whose box holds p.
-template <typename C>
-__global__ __launch_bounds__(256) void k_scatter(const C *__restrict__ xin,
-                                                 const long long *__restrict__ in_off, int B,
-                                                 const int *__restrict__ cube_start,
-                                                 const C *__restrict__ S4, int Nx, int Ny, int Nz,
-                                                 int ncx, int ncy, int ncz, C *__restrict__ grid) {
-    const long long tot = (long long)Nx * Ny * Nz * B;
-    for (long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x; e < tot;
-         e += (long long)gridDim.x * blockDim.x) {
-        const int b = (int)(e % B);
-        const long long p = e / B;
-        const int px = (int)(p % Nx), py = (int)((p / Nx) % Ny), pz = (int)(p / ((long long)Nx * Ny));
-        const C *xb = xin + in_off[b] + b;
-        C a0 = Prec<C>::zero(), a1 = a0, a2 = a0, a3 = a0;
-        // cubes c with 2c <= p <= 2c+2 per axis
-        const int cx0 = max(0, (px - 1) / 2), cx1 = min(ncx - 1, px / 2);
-        const int cy0 = max(0, (py - 1) / 2), cy1 = min(ncy - 1, py / 2);
-        const int cz0 = max(0, (pz - 1) / 2), cz1 = min(ncz - 1, pz / 2);
-        for (int cz = cz0; cz <= cz1; ++cz)
-            for (int cy = cy0; cy <= cy1; ++cy)
-                for (int cx = cx0; cx <= cx1; ++cx) {
-                    const int c = cx + ncx * (cy + ncy * cz);
-                    const int j = (px - 2 * cx) + 3 * (py - 2 * cy) + 9 * (pz - 2 * cz);
-                    for (int t = cube_start[c]; t < cube_start[c + 1]; ++t) {
-                        const C *s = S4 + ((size_t)t * 27 + j) * 4;
-                        const C x0 = Prec<C>::from(xb[(size_t)(3 * t) * B]),
-                                x1 = Prec<C>::from(xb[(size_t)(3 * t + 1) * B]),
-                                x2 = Prec<C>::from(xb[(size_t)(3 * t + 2) * B]);
-                        const C s0 = s[0];
-                        cfma(a0, s0, x0);
-                        cfma(a1, s0, x1);
-                        cfma(a2, s0, x2);
-                        cfma(a3, s[1], x0);
-                        cfma(a3, s[2], x1);
-                        cfma(a3, s[3], x2);
-                    }
-                }
+// ---- narrow batches (fewer than 32 slots) --------------------------------------
+// One wave per grid node (or several, scatter) or tet (gather): the lanes are SB
+// slots (a power of two >= B) x 64 / SB groups that share the sum's terms, combined at the
+// end by a fixed exchange over the groups.  A few slots leave nothing to hide a
+// serial chain of loads behind, so what bounds these kernels is the number of
+// dependent rounds: 160 near tets and 27 nodes per row, about 20 tets per node,
+// divided by the groups.  With one thread per (row, slot), which walked them all,
+// 1,680 tets x 1 vector took 164 us (gather) and 29 us (scatter), now 13 and 11;
+// 24,708 tets x 1 206 and 37, now 95 and 26.
+template <typename C, int SB, int END = 64>
+__device__ inline C group_sum(C v) {
+#pragma unroll
+    for (int o = SB; o < END; o <<= 1) {
+        v.x += __shfl_xor(v.x, o, 64);
+        v.y += __shfl_xor(v.y, o, 64);
+    }
+    return v;
+}
+
+// scatter (sparse_T_matmul, src/sparse.f90:13-43, + vec2arr2): node p sums the
+// stencil weights of the tets of the <= 8 cubes whose box holds p
+template <typename C, int SB>
+__global__ __launch_bounds__(256) void k_scatter_narrow(const C *__restrict__ xin,
+                                                        const long long *__restrict__ in_off, int B,
+                                                        const int *__restrict__ cube_start,
+                                                        const C *__restrict__ S4, int Nx, int Ny, int Nz, int ncx,
+                                                        int ncy, int ncz, C *__restrict__ grid) {
+    // at most 16 groups: a node has about 20 tets, and with few slots a wave then
+    // takes several nodes
+    constexpr int G = 64 / SB < 16 ? 64 / SB : 16, NODES = 64 / (SB * G);
+    const int lane = threadIdx.x & 63, b = lane & (SB - 1), g = (lane / SB) % G;
+    const long long p = ((long long)blockIdx.x * 4 + (threadIdx.x >> 6)) * NODES + lane / (SB * G);
+    if (p >= (long long)Nx * Ny * Nz) return;  // a node's lanes leave together
+    const int px = (int)(p % Nx), py = (int)((p / Nx) % Ny), pz = (int)(p / ((long long)Nx * Ny));
+    const int bl = b < B ? b : B - 1;  // idle lanes load the last slot and store nothing
+    const C *xb = xin + in_off[bl] + bl;
+    C a0 = Prec<C>::zero(), a1 = a0, a2 = a0, a3 = a0;
+    // cubes c with 2c <= p <= 2c+2 per axis; those of one x line hold consecutive tets
+    const int cx0 = max(0, (px - 1) / 2), cx1 = min(ncx - 1, px / 2);
+    const int cy0 = max(0, (py - 1) / 2), cy1 = min(ncy - 1, py / 2);
+    const int cz0 = max(0, (pz - 1) / 2), cz1 = min(ncz - 1, pz / 2);
+    for (int cz = cz0; cz <= cz1; ++cz)
+        for (int cy = cy0; cy <= cy1; ++cy) {
+            const int line = ncx * (cy + ncy * cz);
+            const int t1 = cx1 >= cx0 ? cube_start[line + cx1 + 1] : 0, ts = cx1 >= cx0 ? cube_start[line + cx1] : 0;
+            const int j = 3 * (py - 2 * cy) + 9 * (pz - 2 * cz);
+            for (int t = (cx1 >= cx0 ? cube_start[line + cx0] : 0) + g; t < t1; t += G) {
+                const int jt = j + px - 2 * (t < ts ? cx0 : cx1);
+                const C *s = S4 + ((size_t)t * 27 + jt) * 4;
+                const C x0 = xb[(size_t)(3 * t) * B], x1 = xb[(size_t)(3 * t + 1) * B],
+                        x2 = xb[(size_t)(3 * t + 2) * B];
+                const C s0 = s[0];
+                cfma(a0, s0, x0);
+                cfma(a1, s0, x1);
+                cfma(a2, s0, x2);
+                cfma(a3, s[1], x0);
+                cfma(a3, s[2], x1);
+                cfma(a3, s[3], x2);
+            }
+        }
+    a0 = group_sum<C, SB, SB * G>(a0);
+    a1 = group_sum<C, SB, SB * G>(a1);
+    a2 = group_sum<C, SB, SB * G>(a2);
+    a3 = group_sum<C, SB, SB * G>(a3);
+    if (g == 0 && b < B) {
         C *gp = grid + (size_t)p * 4 * B + b;
         gp[0] = a0;
         gp[(size_t)B] = a1;
@@ -61,198 +87,69 @@ __global__ __launch_bounds__(256) void k_scatter(const C *__restrict__ xin,
 }
 
 // gather (sparse_eps_matmul, src/sparse.f90:47-77) + Y_aim = Y2 - k^2 Y (:148-153)
-// + symmetric near-zone blocks (matmul_Acorr_const, src/sparse_mat.f90:96-123).
-template <typename C>
-__global__ __launch_bounds__(256) void k_gather_near(
+// + symmetric near-zone blocks (matmul_Acorr_const, src/sparse_mat.f90:96-123)
+template <typename C, int SB>
+__global__ __launch_bounds__(256) void k_gather_narrow(
     const C *__restrict__ grid, const C *__restrict__ xin, const long long *__restrict__ in_off, int B,
     int N, const int *__restrict__ tet_cube, const C *__restrict__ S4, int Nx, int Ny, int ncx, int ncy,
     const int64_t *__restrict__ row_start, const int *__restrict__ ent_col,
     const uint32_t *__restrict__ ent_blk, const cf *__restrict__ blocks, double k2,
     const int *__restrict__ slot_active, cd *__restrict__ y) {
-    const long long tot = (long long)N * B;
-    for (long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x; e < tot;
-         e += (long long)gridDim.x * blockDim.x) {
-        const int b = (int)(e % B);
-        const int t = (int)(e / B);
-        cd *yo = y + (size_t)(3 * t) * B + b;
-        if (slot_active && !slot_active[b]) continue;  // inactive slots are not written
+    constexpr int G = 64 / SB;
+    typedef typename Prec<C>::real R;
+    const int lane = threadIdx.x & 63, b = lane & (SB - 1), g = lane / SB;
+    const int wib = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int t = blockIdx.x * 4 + wib;
+    if (t >= N) return;
+    const int bl = b < B ? b : B - 1;
+    C a0 = Prec<C>::zero(), a1 = a0, a2 = a0;
+    {
         const int c = tet_cube[t];
         const int cx = c % ncx, cy = (c / ncx) % ncy, cz = c / (ncx * ncy);
         const size_t base = (size_t)(2 * cx) + (size_t)Nx * ((size_t)(2 * cy) + (size_t)Ny * (2 * cz));
         const C *s = S4 + (size_t)t * 108;
-        C Y0 = Prec<C>::zero(), Y1 = Y0, Y2 = Y0, Z0 = Y0, Z1 = Y0, Z2 = Y0;
-        for (int jz = 0; jz < 3; ++jz)
-            for (int jy = 0; jy < 3; ++jy)
-                for (int jx = 0; jx < 3; ++jx) {
-                    const int j = jx + 3 * jy + 9 * jz;
-                    const size_t node = base + jx + (size_t)Nx * (jy + (size_t)Ny * jz);
-                    const C *g = grid + node * 4 * B + b;
-                    const C g0 = g[0], g1 = g[(size_t)B], g2 = g[(size_t)2 * B], g3 = g[(size_t)3 * B];
-                    const C *sj = s + j * 4;
-                    cfma(Y0, sj[0], g0);
-                    cfma(Y1, sj[0], g1);
-                    cfma(Y2, sj[0], g2);
-                    cfma(Z0, sj[1], g3);
-                    cfma(Z1, sj[2], g3);
-                    cfma(Z2, sj[3], g3);
-                }
-        // near zone
-        const C *xb = xin + in_off[b] + b;
-        C n0 = Prec<C>::zero(), n1 = n0, n2 = n0;
-        for (int64_t q = row_start[t]; q < row_start[t + 1]; ++q) {
-            const int col = ent_col[q];
-            const uint32_t eb = ent_blk[q];
-            const cf *a = blocks + (size_t)(eb & 0x7fffffffu) * 9;
-            const C x0 = Prec<C>::from(xb[(size_t)(3 * col) * B]),
-                    x1 = Prec<C>::from(xb[(size_t)(3 * col + 1) * B]),
-                    x2 = Prec<C>::from(xb[(size_t)(3 * col + 2) * B]);
-            C m[9];
-#pragma unroll
-            for (int i = 0; i < 9; ++i) m[i] = Prec<C>::from(a[i]);
-            if (eb & 0x80000000u) {
-                // transpose: y_i += sum_j A(j,i) x_j ; A(i,j) at i + 3j
-                cfma(n0, m[0], x0); cfma(n0, m[1], x1); cfma(n0, m[2], x2);
-                cfma(n1, m[3], x0); cfma(n1, m[4], x1); cfma(n1, m[5], x2);
-                cfma(n2, m[6], x0); cfma(n2, m[7], x1); cfma(n2, m[8], x2);
-            } else {
-                cfma(n0, m[0], x0); cfma(n0, m[3], x1); cfma(n0, m[6], x2);
-                cfma(n1, m[1], x0); cfma(n1, m[4], x1); cfma(n1, m[7], x2);
-                cfma(n2, m[2], x0); cfma(n2, m[5], x1); cfma(n2, m[8], x2);
-            }
-        }
-        typedef typename Prec<C>::real R;
         const R kk = (R)k2;
-        yo[0] = Prec<cd>::from(cadd(n0, csub(Z0, cscale(Y0, kk))));
-        yo[(size_t)B] = Prec<cd>::from(cadd(n1, csub(Z1, cscale(Y1, kk))));
-        yo[(size_t)2 * B] = Prec<cd>::from(cadd(n2, csub(Z2, cscale(Y2, kk))));
-    }
-}
-
-// ---- wave-uniform variants (slots in chunks of 64) ---------------------------
-// One wave64 owns one grid node (scatter) or one tet (gather) for 64 slots:
-// the node/tet index is wave-uniform (readfirstlane), so every per-node or
-// per-tet operand (cube ranges, S*, near-zone entries and blocks) is a scalar
-// load and only the slot-indexed x, grid and y accesses are vector loads,
-// each 64 consecutive complex numbers.
-template <typename C>
-__global__ __launch_bounds__(256) void k_scatter_w64(const C *__restrict__ xin,
-                                                     const long long *__restrict__ in_off, int B,
-                                                     const int *__restrict__ cube_start,
-                                                     const C *__restrict__ S4, int Nx, int Ny, int Nz,
-                                                     int ncx, int ncy, int ncz, C *__restrict__ grid) {
-    const int lane = threadIdx.x & 63;
-    const int nch = (B + 63) >> 6;  // last chunk may be partial: lanes >= B load slot B-1, store nothing
-    const long long nw = (long long)Nx * Ny * Nz * nch;
-    const int wib = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    for (long long w = (long long)blockIdx.x * 4 + wib; w < nw; w += (long long)gridDim.x * 4) {
-        const long long p = w / nch;
-        const int braw = (int)(w - p * nch) * 64 + lane;
-        const bool valid = braw < B;
-        const int b = valid ? braw : B - 1;
-        const int px = (int)(p % Nx), py = (int)((p / Nx) % Ny), pz = (int)(p / ((long long)Nx * Ny));
-        const C *xb = xin + in_off[b] + b;
-        C a0 = Prec<C>::zero(), a1 = a0, a2 = a0, a3 = a0;
-        const int cx0 = max(0, (px - 1) / 2), cx1 = min(ncx - 1, px / 2);
-        const int cy0 = max(0, (py - 1) / 2), cy1 = min(ncy - 1, py / 2);
-        const int cz0 = max(0, (pz - 1) / 2), cz1 = min(ncz - 1, pz / 2);
-        for (int cz = cz0; cz <= cz1; ++cz)
-            for (int cy = cy0; cy <= cy1; ++cy)
-                for (int cx = cx0; cx <= cx1; ++cx) {
-                    const int c = cx + ncx * (cy + ncy * cz);
-                    const int j = (px - 2 * cx) + 3 * (py - 2 * cy) + 9 * (pz - 2 * cz);
-                    const int t1 = cube_start[c + 1];
-                    for (int t = cube_start[c]; t < t1; ++t) {
-                        const C *s = S4 + ((size_t)t * 27 + j) * 4;
-                        const C x0 = Prec<C>::from(xb[(size_t)(3 * t) * B]),
-                                x1 = Prec<C>::from(xb[(size_t)(3 * t + 1) * B]),
-                                x2 = Prec<C>::from(xb[(size_t)(3 * t + 2) * B]);
-                        const C s0 = s[0];
-                        cfma(a0, s0, x0);
-                        cfma(a1, s0, x1);
-                        cfma(a2, s0, x2);
-                        cfma(a3, s[1], x0);
-                        cfma(a3, s[2], x1);
-                        cfma(a3, s[3], x2);
-                    }
-                }
-        if (valid) {
-            C *gp = grid + (size_t)p * 4 * B + b;
-            gp[0] = a0;
-            gp[(size_t)B] = a1;
-            gp[(size_t)2 * B] = a2;
-            gp[(size_t)3 * B] = a3;
+        for (int j = g; j < 27; j += G) {
+            const C *gp = grid + (base + j % 3 + (size_t)Nx * ((j / 3) % 3 + (size_t)Ny * (j / 9))) * 4 * B + bl;
+            const C g3 = gp[(size_t)3 * B];
+            const C *sj = s + j * 4;
+            const C s0 = cscale(sj[0], -kk);
+            cfma(a0, s0, gp[0]);
+            cfma(a1, s0, gp[(size_t)B]);
+            cfma(a2, s0, gp[(size_t)2 * B]);
+            cfma(a0, sj[1], g3);
+            cfma(a1, sj[2], g3);
+            cfma(a2, sj[3], g3);
         }
     }
-}
-
-template <typename C>
-__global__ __launch_bounds__(256) void k_gather_near_w64(
-    const C *__restrict__ grid, const C *__restrict__ xin, const long long *__restrict__ in_off, int B,
-    int N, const int *__restrict__ tet_cube, const C *__restrict__ S4, int Nx, int Ny, int ncx, int ncy,
-    const int64_t *__restrict__ row_start, const int *__restrict__ ent_col,
-    const uint32_t *__restrict__ ent_blk, const cf *__restrict__ blocks, double k2,
-    const int *__restrict__ slot_active, cd *__restrict__ y) {
-    const int lane = threadIdx.x & 63;
-    const int nch = (B + 63) >> 6;  // last chunk may be partial: lanes >= B load slot B-1, store nothing
-    const long long nw = (long long)N * nch;
-    const int wib = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    for (long long w = (long long)blockIdx.x * 4 + wib; w < nw; w += (long long)gridDim.x * 4) {
-        const int t = (int)(w / nch);
-        const int braw = (int)(w - (long long)t * nch) * 64 + lane;
-        const bool valid = braw < B;
-        const int b = valid ? braw : B - 1;
-        if (!valid) continue;
+    const C *xb = xin + in_off[bl] + bl;
+    const int64_t q1 = row_start[t + 1];
+#pragma unroll 2
+    for (int64_t q = row_start[t] + g; q < q1; q += G) {
+        const int col = ent_col[q];
+        const uint32_t eb = ent_blk[q];
+        const cf *a = blocks + (size_t)(eb & 0x7fffffffu) * 9;
+        const C x0 = xb[(size_t)(3 * col) * B], x1 = xb[(size_t)(3 * col + 1) * B], x2 = xb[(size_t)(3 * col + 2) * B];
+        // A(i, j) at i + 3 j, or of the transposed block at j + 3 i
+        const int si = eb & 0x80000000u ? 3 : 1, sj = 4 - si;
+        cfma(a0, Prec<C>::from(a[0]), x0);
+        cfma(a0, Prec<C>::from(a[sj]), x1);
+        cfma(a0, Prec<C>::from(a[2 * sj]), x2);
+        cfma(a1, Prec<C>::from(a[si]), x0);
+        cfma(a1, Prec<C>::from(a[4]), x1);
+        cfma(a1, Prec<C>::from(a[si + 2 * sj]), x2);
+        cfma(a2, Prec<C>::from(a[2 * si]), x0);
+        cfma(a2, Prec<C>::from(a[2 * si + sj]), x1);
+        cfma(a2, Prec<C>::from(a[8]), x2);
+    }
+    a0 = group_sum<C, SB>(a0);
+    a1 = group_sum<C, SB>(a1);
+    a2 = group_sum<C, SB>(a2);
+    if (g == 0 && b < B && (!slot_active || slot_active[b])) {  // inactive slots are not written
         cd *yo = y + (size_t)(3 * t) * B + b;
-        if (slot_active && !slot_active[b]) continue;  // inactive slots are not written
-        const int c = tet_cube[t];
-        const int cx = c % ncx, cy = (c / ncx) % ncy, cz = c / (ncx * ncy);
-        const size_t base = (size_t)(2 * cx) + (size_t)Nx * ((size_t)(2 * cy) + (size_t)Ny * (2 * cz));
-        const C *s = S4 + (size_t)t * 108;
-        C Y0 = Prec<C>::zero(), Y1 = Y0, Y2 = Y0, Z0 = Y0, Z1 = Y0, Z2 = Y0;
-        for (int jz = 0; jz < 3; ++jz)
-            for (int jy = 0; jy < 3; ++jy)
-#pragma unroll
-                for (int jx = 0; jx < 3; ++jx) {
-                    const int j = jx + 3 * jy + 9 * jz;
-                    const size_t node = base + jx + (size_t)Nx * (jy + (size_t)Ny * jz);
-                    const C *g = grid + node * 4 * B + b;
-                    const C g0 = g[0], g1 = g[(size_t)B], g2 = g[(size_t)2 * B], g3 = g[(size_t)3 * B];
-                    const C *sj = s + j * 4;
-                    cfma(Y0, sj[0], g0);
-                    cfma(Y1, sj[0], g1);
-                    cfma(Y2, sj[0], g2);
-                    cfma(Z0, sj[1], g3);
-                    cfma(Z1, sj[2], g3);
-                    cfma(Z2, sj[3], g3);
-                }
-        const C *xb = xin + in_off[b] + b;
-        C n0 = Prec<C>::zero(), n1 = n0, n2 = n0;
-        const int64_t q1 = row_start[t + 1];
-        for (int64_t q = row_start[t]; q < q1; ++q) {
-            const int col = ent_col[q];
-            const uint32_t eb = ent_blk[q];
-            const cf *a = blocks + (size_t)(eb & 0x7fffffffu) * 9;
-            const C x0 = Prec<C>::from(xb[(size_t)(3 * col) * B]),
-                    x1 = Prec<C>::from(xb[(size_t)(3 * col + 1) * B]),
-                    x2 = Prec<C>::from(xb[(size_t)(3 * col + 2) * B]);
-            C m[9];
-#pragma unroll
-            for (int i = 0; i < 9; ++i) m[i] = Prec<C>::from(a[i]);
-            if (eb & 0x80000000u) {
-                cfma(n0, m[0], x0); cfma(n0, m[1], x1); cfma(n0, m[2], x2);
-                cfma(n1, m[3], x0); cfma(n1, m[4], x1); cfma(n1, m[5], x2);
-                cfma(n2, m[6], x0); cfma(n2, m[7], x1); cfma(n2, m[8], x2);
-            } else {
-                cfma(n0, m[0], x0); cfma(n0, m[3], x1); cfma(n0, m[6], x2);
-                cfma(n1, m[1], x0); cfma(n1, m[4], x1); cfma(n1, m[7], x2);
-                cfma(n2, m[2], x0); cfma(n2, m[5], x1); cfma(n2, m[8], x2);
-            }
-        }
-        typedef typename Prec<C>::real R;
-        const R kk = (R)k2;
-        yo[0] = Prec<cd>::from(cadd(n0, csub(Z0, cscale(Y0, kk))));
-        yo[(size_t)B] = Prec<cd>::from(cadd(n1, csub(Z1, cscale(Y1, kk))));
-        yo[(size_t)2 * B] = Prec<cd>::from(cadd(n2, csub(Z2, cscale(Y2, kk))));
+        yo[0] = Prec<cd>::from(a0);
+        yo[(size_t)B] = Prec<cd>::from(a1);
+        yo[(size_t)2 * B] = Prec<cd>::from(a2);
     }
 }
 
@@ -262,7 +159,7 @@ __global__ __launch_bounds__(256) void k_gather_near_w64(
 // every node of the block lies in the boxes of the same <= 8 cubes (a-1..a per
 // axis), so the wave loads each of their tets' x once for all 8 nodes, instead
 // of once per node.  Per node the sum runs over cubes and tets in the same
-// order as k_scatter.
+// order: z, y, x.
 template <typename C>
 __global__ __launch_bounds__(256) void k_scatter_blk_w64(const C *__restrict__ xin,
                                                          const long long *__restrict__ in_off, int B,
@@ -358,23 +255,32 @@ __global__ __launch_bounds__(256) void k_scatter_blk_w64(const C *__restrict__ x
 }
 
 // Gather + near zone with the per-tet operands staged in LDS, one 64-thread
-// workgroup per (non-empty cube, 64-slot chunk); the steps are in
+// workgroup per (row group of a cube, 64-slot chunk); the steps are in
 // gather_core.hpp (shared with the host self-test).  Staging keeps many
 // operand fetches in flight (wave-uniform operands read through scalar loads
 // would wait on each other).
-template <typename C, int NT, int GT, int VC>
-__device__ __forceinline__ void gather_pass(const gcore::GatherArgs<C> &g, const gcore::Item &it, int tp, int lane,
+template <typename C, int NT, int GT, int VC, int SB, int NS>
+__device__ __forceinline__ void gather_pass(const gcore::GatherArgs<C> &g, const gcore::Item &it, int chunk, int lane,
                                             unsigned char *smraw) {
     C *sm = (C *)smraw;         // S* records of the pass's tets
     cf *smb = (cf *)smraw;      // then the near-zone blocks of each chunk
     using namespace gcore;
-    C acc[NT][3];
-    zero_acc<C, NT>(acc);
-    __syncthreads();  // the previous pass's reads of sm are done
-    stage_s4(g, tp, NT, lane, sm);
+    const Slots<SB, NS> sl = lane_slots<SB, NS>(g, chunk, lane);
+    C acc[NT][3][NS];
+#pragma unroll
+    for (int u = 0; u < NT; ++u)
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+            for (int i = 0; i < NS; ++i) acc[u][c][i] = Prec<C>::zero();
+    long long off[NS];
+#pragma unroll
+    for (int i = 0; i < NS; ++i) off[i] = g.in_off[sl.s[i]] + sl.s[i];
+    __syncthreads();  // the previous item's reads of sm are done
+    stage_s4(g, it.t0, NT, lane, sm);
     __syncthreads();
-    grid_part<C, NT>(g, it, sm, acc);
-    const int64_t rsu = lane_row_start<C, GT, VC>(g, tp, NT, lane);
+    grid_share<C, NT, SB, NS>(g, it, sl, sm, acc);
+    const int64_t rsu = lane_row_start<C, GT, VC>(g, it.t0, NT, lane);
     int q = 0;
     for_near_cubes(g, it, [&](int c0, int c1) {
         for (int v0 = c0; v0 < c1; v0 += VC) {
@@ -382,37 +288,57 @@ __device__ __forceinline__ void gather_pass(const gcore::GatherArgs<C> &g, const
             __syncthreads();
             stage_blocks<C, GT, VC>(g, NT, nv, q, lane, rsu, smb);
             __syncthreads();
-            chunk_part<C, NT, VC>(g, it, v0, nv, smb, acc);
+            chunk_share<C, NT, VC, SB, NS>(g, sl, off, v0, nv, smb, acc);
             q += nv;
         }
     });
-    write_out<C, NT>(g, it, tp, acc);
+    // the groups' sums, by a fixed exchange; group i (two groups: slot i of a lane)
+    // or group 0 writes
+    bool act[NS];
+#pragma unroll
+    for (int i = 0; i < NS; ++i) act[i] = sl.ok[i] && (!g.slot_active || g.slot_active[sl.s[i]]);
+#pragma unroll
+    for (int u = 0; u < NT; ++u) {
+        cd *yo = g.y + (size_t)(3 * (it.t0 + u)) * g.B;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            if constexpr (SB == 32 && NS == 2) {
+                const bool hi = sl.grp != 0;
+                C mine = hi ? acc[u][c][1] : acc[u][c][0], give = hi ? acc[u][c][0] : acc[u][c][1];
+                give.x = __shfl_xor(give.x, 32, 64);
+                give.y = __shfl_xor(give.y, 32, 64);
+                if (hi ? act[1] : act[0])  // inactive slots are not written
+                    yo[(size_t)c * g.B + (hi ? sl.s[1] : sl.s[0])] = Prec<cd>::from(cadd(mine, give));
+            } else {
+#pragma unroll
+                for (int i = 0; i < NS; ++i) {
+                    const C v = group_sum<C, SB>(acc[u][c][i]);
+                    if (sl.grp == 0 && act[i]) yo[(size_t)c * g.B + sl.s[i]] = Prec<cd>::from(v);
+                }
+            }
+        }
+    }
 }
 
-template <typename C, int GT, int VC>
+template <typename C, int GT, int VC, int SB, int NS>
 __global__ __launch_bounds__(64, 3) void k_gather_lds(gcore::GatherArgs<C> g) {
     using namespace gcore;
-    static_assert(GT == 8, "the pass switch below covers 1..8 row tets");
+    static_assert(GT <= 3, "the passes below cover 1..3 row tets");
     __shared__ __align__(16) unsigned char sm[Shape<C, GT, VC>::BYTES];
     const int lane = threadIdx.x;
-    const long long nw = (long long)g.n_ne * ((g.B + 63) >> 6);
+    const long long nw = (long long)g.n_groups * ((g.B + SB * NS - 1) / (SB * NS));
     for (long long b = blockIdx.x; b < nw; b += gridDim.x) {
         // one item per workgroup when the grid covers all items (the launch
         // below); a grid-stride remainder keeps plain order
         const long long w = nw == gridDim.x ? xcd_remap(b, nw) : b;
-        const Item it = make_item(g, w, lane);
-        for (int tp = it.t0; tp < it.t1; tp += GT) {
-            switch (min(GT, it.t1 - tp)) {  // wave-uniform
-                case 1: gather_pass<C, 1, GT, VC>(g, it, tp, lane, sm); break;
-                case 2: gather_pass<C, 2, GT, VC>(g, it, tp, lane, sm); break;
-                case 3: gather_pass<C, 3, GT, VC>(g, it, tp, lane, sm); break;
-                case 4: gather_pass<C, 4, GT, VC>(g, it, tp, lane, sm); break;
-                case 5: gather_pass<C, 5, GT, VC>(g, it, tp, lane, sm); break;
-                case 6: gather_pass<C, 6, GT, VC>(g, it, tp, lane, sm); break;
-                case 7: gather_pass<C, 7, GT, VC>(g, it, tp, lane, sm); break;
-                default: gather_pass<C, 8, GT, VC>(g, it, tp, lane, sm); break;
-            }
-        }
+        const int chunk = (int)(w / g.n_groups);
+        const Item it = group_item(g, (int)(w - (long long)chunk * g.n_groups));
+        const int nt = it.t1 - it.t0;  // wave-uniform
+#define PASS(N)                                                                          \
+    if constexpr (GT >= N)                                                               \
+        if (nt == N) gather_pass<C, N, GT, VC, SB, NS>(g, it, chunk, lane, sm);
+        PASS(1) PASS(2) PASS(3)
+#undef PASS
     }
 }
 
@@ -532,64 +458,97 @@ __global__ __launch_bounds__(64, 3) void k_gather_mf(gcore::GatherArgs<cf> g) {
     }
 }
 
-// slot-chunk (wave64-per-item) kernels when the last 64-slot chunk is at least
-// half full: even then they beat the slot-per-lane kernels, which share no
-// operand loads between the tets of a cube or the nodes of a block
-static bool wave_slots(int B) { return B % 64 == 0 || B % 64 >= 32; }
+// Widths, us per launch in complex128 (complex64 orders them alike).  Scatter: the
+// narrow kernel to 24 slots (24,708 tets: 16 slots 85 against 115 in a 64-slot
+// chunk, 24 slots 126 and 128; 43,248 tets, 24 slots 206 and 198).  Gather: one tet a
+// wave to 4 slots (1,680 tets x 3: 18; it reads every block by single lanes, which
+// costs more than it saves from 8: 24,708 tets 259 against 142), then row groups
+// with the lanes' slots fitted to the batch (24,708 tets: 16 slots 213, 24 slots
+// 348, with one thread per row and slot 462 and 637).
+constexpr int SCATTER_NARROW = 24, GATHER_NARROW = 4;
 
 static unsigned grid_for(long long tot, int bs) {
     long long g = (tot + bs - 1) / bs;
     return (unsigned)std::min<long long>(std::max<long long>(g, 1), 1LL << 20);
 }
 
+// f(integral constant SB): the lanes' slots of a narrow batch of B
+template <typename F>
+static void narrow_slots(int B, F &&f) {
+    if (B <= 1)
+        f(std::integral_constant<int, 1>{});
+    else if (B <= 2)
+        f(std::integral_constant<int, 2>{});
+    else if (B <= 4)
+        f(std::integral_constant<int, 4>{});
+    else if (B <= 8)
+        f(std::integral_constant<int, 8>{});
+    else if (B <= 16)
+        f(std::integral_constant<int, 16>{});
+    else
+        f(std::integral_constant<int, 32>{});
+}
+
 template <typename C>
 void launch_scatter(const MatvecArgs<C> &a, hipStream_t s) {
-    if (wave_slots(a.B)) {
+    if (a.B > SCATTER_NARROW) {
         const long long nw = (long long)((a.Nx + 1) / 2) * ((a.Ny + 1) / 2) * ((a.Nz + 1) / 2) * ((a.B + 63) / 64);
         hipLaunchKernelGGL((k_scatter_blk_w64<C>), dim3(grid_for(nw, 4)), dim3(256), 0, s, a.xin, a.in_off, a.B,
                            a.cube_start, a.S4, a.Nx, a.Ny, a.Nz, a.ncx, a.ncy, a.ncz, a.grid_in);
-        HIP_CHECK(hipGetLastError());
-        return;
+    } else {
+        const long long nodes = (long long)a.Nx * a.Ny * a.Nz;
+        narrow_slots(a.B, [&](auto sb) {
+            constexpr int SB = decltype(sb)::value, per = SB < 4 ? 16 / SB : 4;  // nodes per workgroup
+            hipLaunchKernelGGL((k_scatter_narrow<C, SB>), dim3((unsigned)((nodes + per - 1) / per)), dim3(256), 0, s,
+                               a.xin, a.in_off, a.B, a.cube_start, a.S4, a.Nx, a.Ny, a.Nz, a.ncx, a.ncy, a.ncz,
+                               a.grid_in);
+        });
     }
-    long long tot = (long long)a.Nx * a.Ny * a.Nz * a.B;
-    hipLaunchKernelGGL((k_scatter<C>), dim3(grid_for(tot, 256)), dim3(256), 0, s, a.xin, a.in_off, a.B,
-                       a.cube_start, a.S4, a.Nx, a.Ny, a.Nz, a.ncx, a.ncy, a.ncz, a.grid_in);
     HIP_CHECK(hipGetLastError());
 }
 
 template <typename C>
 void launch_gather_near(const MatvecArgs<C> &a, hipStream_t s) {
-    if (wave_slots(a.B) && a.ne_cubes) {
-        const long long nw = (long long)a.n_ne * ((a.B + 63) / 64);
-        const gcore::GatherArgs<C> g = {a.grid_out, a.xin,     a.in_off,    a.B,      a.ne_cubes,
-                                        a.n_ne,     a.cube_start, a.S4,      a.Nx,     a.Ny,
-                                        a.ncx,      a.ncy,       a.ncz,       a.row_start, a.ent_blk,
-                                        a.blocks,   a.k2,        a.slot_active, a.y};
-        if constexpr (std::is_same<C, cf>::value) {
-            if (a.gather_kernel == 1) {
-                hipLaunchKernelGGL((k_gather_mf<gcore::GATHER_GT, gcore::GATHER_VC>), dim3(grid_for(nw, 1)), dim3(64),
-                                   0, s, g);
-                HIP_CHECK(hipGetLastError());
-                return;
-            }
+    if (a.B <= GATHER_NARROW) {
+        narrow_slots(a.B, [&](auto sb) {
+            constexpr int SB = decltype(sb)::value;
+            if constexpr (SB <= GATHER_NARROW)
+                hipLaunchKernelGGL((k_gather_narrow<C, SB>), dim3((unsigned)((a.N + 3) / 4)), dim3(256), 0, s,
+                                   a.grid_out, a.xin, a.in_off, a.B, a.N, a.tet_cube, a.S4, a.Nx, a.Ny, a.ncx, a.ncy,
+                                   a.row_start, a.ent_col, a.ent_blk, a.blocks, a.k2, a.slot_active, a.y);
+        });
+        HIP_CHECK(hipGetLastError());
+        return;
+    }
+    gcore::GatherArgs<C> g = {a.grid_out, a.xin,     a.in_off,    a.B,      a.ne_cubes,
+                                    a.n_ne,     a.cube_start, a.S4,      a.Nx,     a.Ny,
+                                    a.ncx,      a.ncy,       a.ncz,       a.row_start, a.ent_blk,
+                                    a.blocks,   a.k2,        a.slot_active, a.y};
+    g.groups = a.groups;
+    g.n_groups = a.n_groups;
+    if constexpr (std::is_same<C, cf>::value) {
+        if (a.gather_kernel == 1) {
+            hipLaunchKernelGGL((k_gather_mf<gcore::GATHER_GT, gcore::GATHER_VC>), dim3(grid_for((long long)a.n_ne * ((a.B + 63) / 64), 1)),
+                               dim3(64), 0, s, g);
+            HIP_CHECK(hipGetLastError());
+            return;
         }
-        hipLaunchKernelGGL((k_gather_lds<C, gcore::GATHER_GT, gcore::GATHER_VC>), dim3(grid_for(nw, 1)), dim3(64), 0, s,
-                           g);
-        HIP_CHECK(hipGetLastError());
-        return;
     }
-    if (wave_slots(a.B)) {
-        const long long nw = (long long)a.N * ((a.B + 63) / 64);
-        hipLaunchKernelGGL((k_gather_near_w64<C>), dim3(grid_for(nw, 4)), dim3(256), 0, s, a.grid_out, a.xin,
-                           a.in_off, a.B, a.N, a.tet_cube, a.S4, a.Nx, a.Ny, a.ncx, a.ncy, a.row_start, a.ent_col,
-                           a.ent_blk, a.blocks, a.k2, a.slot_active, a.y);
-        HIP_CHECK(hipGetLastError());
-        return;
-    }
-    long long tot = (long long)a.N * a.B;
-    hipLaunchKernelGGL((k_gather_near<C>), dim3(grid_for(tot, 256)), dim3(256), 0, s, a.grid_out, a.xin,
-                       a.in_off, a.B, a.N, a.tet_cube, a.S4, a.Nx, a.Ny, a.ncx, a.ncy, a.row_start, a.ent_col,
-                       a.ent_blk, a.blocks, a.k2, a.slot_active, a.y);
+    auto go = [&](auto sb, auto ns) {
+        constexpr int SB = decltype(sb)::value, NS = decltype(ns)::value;
+        const long long nw = (long long)a.n_groups * ((a.B + SB * NS - 1) / (SB * NS));
+        hipLaunchKernelGGL((k_gather_lds<C, gcore::ROW_GT, gcore::ROW_VC, SB, NS>), dim3(grid_for(nw, 1)), dim3(64), 0,
+                           s, g);
+    };
+    typedef std::integral_constant<int, 1> one;
+    if (a.B > 32)
+        go(std::integral_constant<int, 32>{}, std::integral_constant<int, 2>{});
+    else if (a.B > 16)
+        go(std::integral_constant<int, 32>{}, one{});
+    else if (a.B > 8)
+        go(std::integral_constant<int, 16>{}, one{});
+    else
+        go(std::integral_constant<int, 8>{}, one{});
     HIP_CHECK(hipGetLastError());
 }
 

@@ -24,6 +24,8 @@ struct MatvecArgs {
     // non-empty cubes, in the order the per-cube gather takes them
     const int *ne_cubes = nullptr;
     int n_ne = 0;
+    const int2 *groups = nullptr;  // row groups of those cubes (gather_core.hpp)
+    int n_groups = 0;
     double k2 = 0;
     const int *slot_active = nullptr;  // optional per-slot mask
     int gather_kernel = 0;             // complex64: 1 = near zone on the matrix cores
