@@ -785,25 +785,32 @@ static int auto_batch(scadyn_operator *op, int ncols) {
     size_t per = slot_bytes(op, op->opts.maxit);
     size_t cap = (size_t)(0.75 * (double)free_b) / std::max<size_t>(per, 1);
     if (cap == 0) fail(SCADYN_ERR_MEMORY, "not enough device memory for one RHS slot");
-    // Up to 64 slots; above 64 columns, split them into the fewest equal
-    // generations of at most 128 slots that fill their last 64-slot chunk to at
-    // least 48 (the slot-chunk kernels then idle at most a quarter of a chunk)
-    // and fit in memory: no nearly empty final generation of refills.
+    // Above 64 columns, equal generations of at most 128 slots.  A step costs about
+    // one part per slot (transforms, Krylov sweeps; idle slots too) and half a part
+    // per lane of the 64-slot chunks that the scatter and gather run, so take the
+    // split with the least of that over all generations, the fewest where two are
+    // equal: 70 columns run as one batch of 70 rather than as 64 and 6 (the
+    // 43,248-tet FP64 bar: 126 ms instead of 163; the 24,708-tet mixed bar 167 instead of
+    // 237).
     int B = std::min(64, ncols);
-    if (ncols > 64)
-        for (int gen = (ncols + 127) / 128; gen <= ncols / 48; ++gen) {
+    if (ncols > 64) {
+        long long best = -1;
+        for (int gen = (ncols + 127) / 128; gen <= (ncols + 31) / 32; ++gen) {
             const int Bg = (ncols + gen - 1) / gen;
-            if ((Bg % 64 == 0 || Bg % 64 >= 48) && (size_t)Bg <= cap) {
+            if ((size_t)Bg > cap) continue;
+            const long long cost = (long long)gen * (Bg + 32 * ((Bg + 63) / 64));
+            if (best < 0 || cost < best) {
+                best = cost;
                 B = Bg;
-                break;
             }
         }
+    }
     // memory, not the column count, limits the batch
     const bool capped = cap < (size_t)std::min(ncols, 128);
     B = (int)std::min<size_t>((size_t)B, cap);
-    // a memory-capped batch keeps the slot-chunk kernels: round down to a width
-    // whose last 64-slot chunk holds at least 48 slots
-    if (B > 64 && B % 64 != 0 && B % 64 < 48) B -= B % 64;
+    // a memory-capped batch: round down to a width whose last 64-slot chunk holds
+    // at least 48 slots
+    if (capped && B > 64 && B % 64 != 0 && B % 64 < 48) B -= B % 64;
     // a capped batch whose last chunk is nearly full is completed to 64 slots
     // when that still fits within 0.85 of the free memory: a full chunk runs
     // each slot faster (824k-tet sphere, mixed: 64 slots 1.18 columns/s, 59
