@@ -57,21 +57,16 @@ struct GatherArgs {
     int n_groups = 0;
 };
 
-// Row tets and near columns per pass of the vector kernel: a wave takes a group
-// of up to ROW_GT tets of a cube (a cube of 6 is two waves), and one staged chunk
-// covers the columns of an x line of three near cubes (about 18; ROW_GT x ROW_VC <=
-// 64: one block per lane).
-//  * With all tets of a cube in one wave, 43,248 tets had 7,213 waves for the 1,024
-//    SIMDs (7.04 each, the last ones alone), three to a SIMD: vector issue
-//    43% busy.
-//  * A chunk is a chain of two dependent loads (entry, block) before its first use;
-//    27 chunks of one near cube each waited for it 27 times a pass.
+// Row tets of a wave and near columns per staged chunk of the vector kernel: a row
+// group is up to ROW_GT tets of a cube, and a chunk covers the columns of an x line of
+// three near cubes (about 18; half the rows x ROW_VC <= 64: a block of either half per
+// lane).  A chunk is a chain of two dependent loads (entry, block) before its first
+// use; chunks of one near cube waited for it 27 times a pass, these 9 times.
 // Measured per launch, 64 slots, complex128 / complex64: 43,248 tets 1,632 / 768 us
-// before, 1,424 / 699 with these groups and one slot a lane, 1,275 / 613 with the
-// wave layout below; 146,784 tets 4,224 / 2,436 before, 3,415 / 2,023 now; 32 slots
-// of 369,390 tets 9,539 / 5,118 before, 4,732 / 2,972 now.  Groups of 2, 4 and 6 rows
-// (32, 16 and 10 columns) ran at 1,333 / 700, 1,411 / 706 and 1,410 / 649 us.
-constexpr int ROW_GT = 3, ROW_VC = 21;
+// with one slot a lane, all tets of a cube in a wave and one near cube a chunk, 1,306 /
+// 626 now; 146,784 tets 4,224 / 2,436 before, 3,488 / 2,054 now; 32 slots of 369,390
+// tets 9,539 / 5,118 before, 4,829 / 3,170 now.
+constexpr int ROW_GT = 6, ROW_VC = 21;
 // of the matrix-core kernel (8 covers all tets of nearly every cube of a cube-split
 // mesh, so the near-zone x of a cube is fetched once) and column tets per
 // staged near chunk (GT x VC = 64: one block per lane)
@@ -254,18 +249,21 @@ GC_HD void write_out(const GatherArgs<C> &g, const Item &it, int tp, C (*acc)[3]
 }
 
 // ---- wave layout of the vector kernel ------------------------------------------
-// SB lanes hold NS slots each (slot, slot + SB), and the 64 / SB lane groups share
-// the columns of a chunk and the nodes of the box; the groups' sums are combined at
-// the end.  Every operand read from LDS then serves NS slots and 64 / SB columns.
-// A wave-wide LDS read returns its 64 copies at 128 bytes a cycle, also when all
-// lanes read one address: with one slot per lane and one column at a time the
+// SB lanes hold NS slots each (slot, slot + SB), and the 64 / SB lane groups take NT
+// rows each: group g the rows g NT .. g NT + NT - 1 of the wave's row group (rows
+// past its end compute on stale LDS and are not written).  Every operand read from
+// LDS then serves NS slots and 64 / SB rows, and a column's x is loaded once for
+// all rows.  A wave-wide LDS read returns its 64 copies at 128 bytes a cycle, also
+// when all lanes read one address: with one slot per lane and one row at a time the
 // block reads alone took the CU's LDS as long as the FMAs took its four SIMDs, and
-// every block was widened to complex128 once per wave and slot chunk.
+// every block was widened to complex128 once per wave and slot chunk.  A row's sum
+// still runs node by node and column by column, as the reference's loops do: the
+// complex64 product keeps its rounding, whatever the batch width.
 template <int SB, int NS>
 struct Slots {
-    int s[NS];      // slot used for loads
-    bool ok[NS];    // lane holds a real slot
-    int grp;        // lane group
+    int s[NS];    // slot used for loads
+    bool ok[NS];  // lane holds a real slot
+    int grp;      // lane group
 };
 template <int SB, int NS, typename C>
 GC_HD Slots<SB, NS> lane_slots(const GatherArgs<C> &g, int chunk, int lane) {
@@ -280,22 +278,35 @@ GC_HD Slots<SB, NS> lane_slots(const GatherArgs<C> &g, int chunk, int lane) {
     return r;
 }
 
-// the lane group's share of y_c += S_{c+1}^T g3 - k^2 S^T g_c over the 27 box nodes
-template <typename C, int NT, int SB, int NS>
-GC_HD void grid_share(const GatherArgs<C> &g, const Item &it, const Slots<SB, NS> &sl, const C *sm,
-                      C (*acc)[3][NS]) {
-    constexpr int G = 64 / SB;
+// the lane's rows of y_c += S_{c+1}^T g3 - k^2 S^T g_c over the 27 box nodes; sm: the
+// S* records of the lane group's rows.  In complex64 the next node is fetched
+// while one is applied (complex128 has no registers to spare for it).
+template <typename C, int NT, int NS>
+GC_HD void grid_rows(const GatherArgs<C> &g, const Item &it, const int *slot, const C *sm, C (*acc)[3][NS]) {
     typedef typename Prec<C>::real R;
     const R kk = (R)g.k2;
     const size_t B = (size_t)g.B;
-#pragma unroll 1
-    for (int j = sl.grp; j < 27; j += G) {
+    constexpr bool PREFETCH = sizeof(C) == 8;
+    C v[4][NS], n[4][NS];
+    auto fetch = [&](int j, C(*d)[NS]) {
         const C *gp = g.grid + (it.base + j % 3 + (size_t)g.Nx * ((j / 3) % 3 + (size_t)g.Ny * (j / 9))) * 4 * B;
-        C v[4][NS];
 #pragma unroll
         for (int c = 0; c < 4; ++c)
 #pragma unroll
-            for (int i = 0; i < NS; ++i) v[c][i] = gp[c * B + sl.s[i]];
+            for (int i = 0; i < NS; ++i) d[c][i] = gp[c * B + slot[i]];
+    };
+    if (PREFETCH) fetch(0, n);
+#pragma unroll 1
+    for (int j = 0; j < 27; ++j) {
+        if (PREFETCH) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+#pragma unroll
+                for (int i = 0; i < NS; ++i) v[c][i] = n[c][i];
+            if (j + 1 < 27) fetch(j + 1, n);
+        } else {
+            fetch(j, v);
+        }
 #pragma unroll
         for (int u = 0; u < NT; ++u) {
             const C *s = sm + u * 108 + j * 4;
@@ -313,12 +324,11 @@ GC_HD void grid_share(const GatherArgs<C> &g, const Item &it, const Slots<SB, NS
     }
 }
 
-// the lane group's columns (grp, grp + 64 / SB, ...) of the staged blocks of column
-// tets v0 .. v0+nv-1; x of the next column is fetched while one is applied
-template <typename C, int NT, int VC, int SB, int NS>
-GC_HD void chunk_share(const GatherArgs<C> &g, const Slots<SB, NS> &sl, const long long *off, int v0, int nv,
-                       const cf *sm, C (*acc)[3][NS]) {
-    constexpr int G = 64 / SB;
+// the staged blocks of column tets v0 .. v0+nv-1 applied to the lane's rows (sm: the
+// first block of its group's rows); x of the next column is fetched while one is
+// applied
+template <typename C, int NT, int VC, int NS>
+GC_HD void chunk_rows(const GatherArgs<C> &g, const long long *off, int v0, int nv, const cf *sm, C (*acc)[3][NS]) {
     const size_t B = (size_t)g.B;
     C n[3][NS];
     auto fetch = [&](int v) {
@@ -328,15 +338,15 @@ GC_HD void chunk_share(const GatherArgs<C> &g, const Slots<SB, NS> &sl, const lo
 #pragma unroll
             for (int i = 0; i < NS; ++i) n[c][i] = xb[c * B + off[i]];
     };
-    if (sl.grp < nv) fetch(sl.grp);
+    fetch(0);
 #pragma unroll 1
-    for (int v = sl.grp; v < nv; v += G) {
+    for (int v = 0; v < nv; ++v) {
         C x[3][NS];
 #pragma unroll
         for (int c = 0; c < 3; ++c)
 #pragma unroll
             for (int i = 0; i < NS; ++i) x[c][i] = n[c][i];
-        if (v + G < nv) fetch(v + G);
+        if (v + 1 < nv) fetch(v + 1);
 #pragma unroll
         for (int u = 0; u < NT; ++u) {
             const cf *m = sm + (u * VC + v) * 9;  // column-major 3x3
@@ -348,6 +358,51 @@ GC_HD void chunk_share(const GatherArgs<C> &g, const Slots<SB, NS> &sl, const lo
 #pragma unroll
                     for (int i = 0; i < NS; ++i) cfma(acc[u][r][i], a, x[c][i]);
                 }
+        }
+    }
+}
+
+// Narrow complex128 batches: the lane groups share the columns and nodes of the same
+// rows instead (group g the columns g, g + G, ..., G = 64 / SB); their sums are
+// combined at the end
+template <typename C, int NT, int SB>
+GC_HD void grid_share(const GatherArgs<C> &g, const Item &it, const Slots<SB, 1> &sl, const C *sm, C (*acc)[3]) {
+    typedef typename Prec<C>::real R;
+    const R kk = (R)g.k2;
+    const size_t B = (size_t)g.B;
+#pragma unroll 1
+    for (int j = sl.grp; j < 27; j += 64 / SB) {
+        const C *gp =
+            g.grid + (it.base + j % 3 + (size_t)g.Nx * ((j / 3) % 3 + (size_t)g.Ny * (j / 9))) * 4 * B + sl.s[0];
+        const C v0 = gp[0], v1 = gp[B], v2 = gp[2 * B], v3 = gp[3 * B];
+#pragma unroll
+        for (int u = 0; u < NT; ++u) {
+            const C *s = sm + u * 108 + j * 4;
+            const C s0 = cscale(s[0], -kk);
+            cfma(acc[u][0], s0, v0);
+            cfma(acc[u][1], s0, v1);
+            cfma(acc[u][2], s0, v2);
+            cfma(acc[u][0], s[1], v3);
+            cfma(acc[u][1], s[2], v3);
+            cfma(acc[u][2], s[3], v3);
+        }
+    }
+}
+template <typename C, int NT, int VC, int SB>
+GC_HD void chunk_share(const GatherArgs<C> &g, const Slots<SB, 1> &sl, long long off, int v0, int nv, const cf *sm,
+                       C (*acc)[3]) {
+    const size_t B = (size_t)g.B;
+#pragma unroll 1
+    for (int v = sl.grp; v < nv; v += 64 / SB) {
+        const C *xb = g.xin + (size_t)(3 * (v0 + v)) * B + off;
+        const C x[3] = {xb[0], xb[B], xb[2 * B]};
+#pragma unroll
+        for (int u = 0; u < NT; ++u) {
+            const cf *m = sm + (u * VC + v) * 9;  // column-major 3x3
+#pragma unroll
+            for (int r = 0; r < 3; ++r)
+#pragma unroll
+                for (int c = 0; c < 3; ++c) cfma(acc[u][r], Prec<C>::from(m[r + 3 * c]), x[c]);
         }
     }
 }

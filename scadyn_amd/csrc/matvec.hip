@@ -259,12 +259,13 @@ __global__ __launch_bounds__(256) void k_scatter_blk_w64(const C *__restrict__ x
 // gather_core.hpp (shared with the host self-test).  Staging keeps many
 // operand fetches in flight (wave-uniform operands read through scalar loads
 // would wait on each other).
-template <typename C, int NT, int GT, int VC, int SB, int NS>
+template <typename C, int NT, int VC, int SB, int NS>
 __device__ __forceinline__ void gather_pass(const gcore::GatherArgs<C> &g, const gcore::Item &it, int chunk, int lane,
                                             unsigned char *smraw) {
-    C *sm = (C *)smraw;         // S* records of the pass's tets
+    C *sm = (C *)smraw;         // S* records of the group's tets
     cf *smb = (cf *)smraw;      // then the near-zone blocks of each chunk
     using namespace gcore;
+    const int rows = it.t1 - it.t0;
     const Slots<SB, NS> sl = lane_slots<SB, NS>(g, chunk, lane);
     C acc[NT][3][NS];
 #pragma unroll
@@ -277,54 +278,45 @@ __device__ __forceinline__ void gather_pass(const gcore::GatherArgs<C> &g, const
 #pragma unroll
     for (int i = 0; i < NS; ++i) off[i] = g.in_off[sl.s[i]] + sl.s[i];
     __syncthreads();  // the previous item's reads of sm are done
-    stage_s4(g, it.t0, NT, lane, sm);
+    stage_s4(g, it.t0, rows, lane, sm);
     __syncthreads();
-    grid_share<C, NT, SB, NS>(g, it, sl, sm, acc);
-    const int64_t rsu = lane_row_start<C, GT, VC>(g, it.t0, NT, lane);
+    grid_rows<C, NT, NS>(g, it, sl.s, sm + sl.grp * NT * 108, acc);
+    // a lane stages one block of the first and one of the last ROW_GT / 2 rows
+    constexpr int HT = ROW_GT / 2;
+    const int64_t rs0 = lane_row_start<C, HT, VC>(g, it.t0, min(rows, HT), lane),
+                  rs1 = lane_row_start<C, HT, VC>(g, it.t0 + HT, rows - HT, lane);
     int q = 0;
     for_near_cubes(g, it, [&](int c0, int c1) {
         for (int v0 = c0; v0 < c1; v0 += VC) {
             const int nv = min(VC, c1 - v0);
             __syncthreads();
-            stage_blocks<C, GT, VC>(g, NT, nv, q, lane, rsu, smb);
+            stage_blocks<C, HT, VC>(g, min(rows, HT), nv, q, lane, rs0, smb);
+            if (rows > HT) stage_blocks<C, HT, VC>(g, rows - HT, nv, q, lane, rs1, smb + HT * VC * 9);
             __syncthreads();
-            chunk_share<C, NT, VC, SB, NS>(g, sl, off, v0, nv, smb, acc);
+            chunk_rows<C, NT, VC, NS>(g, off, v0, nv, smb + sl.grp * NT * VC * 9, acc);
             q += nv;
         }
     });
-    // the groups' sums, by a fixed exchange; group i (two groups: slot i of a lane)
-    // or group 0 writes
-    bool act[NS];
 #pragma unroll
-    for (int i = 0; i < NS; ++i) act[i] = sl.ok[i] && (!g.slot_active || g.slot_active[sl.s[i]]);
+    for (int i = 0; i < NS; ++i) {
+        if (!sl.ok[i] || (g.slot_active && !g.slot_active[sl.s[i]])) continue;  // inactive slots are not written
 #pragma unroll
-    for (int u = 0; u < NT; ++u) {
-        cd *yo = g.y + (size_t)(3 * (it.t0 + u)) * g.B;
+        for (int u = 0; u < NT; ++u) {
+            const int row = sl.grp * NT + u;
+            if (row >= rows) continue;
+            cd *yo = g.y + (size_t)(3 * (it.t0 + row)) * g.B + sl.s[i];
 #pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            if constexpr (SB == 32 && NS == 2) {
-                const bool hi = sl.grp != 0;
-                C mine = hi ? acc[u][c][1] : acc[u][c][0], give = hi ? acc[u][c][0] : acc[u][c][1];
-                give.x = __shfl_xor(give.x, 32, 64);
-                give.y = __shfl_xor(give.y, 32, 64);
-                if (hi ? act[1] : act[0])  // inactive slots are not written
-                    yo[(size_t)c * g.B + (hi ? sl.s[1] : sl.s[0])] = Prec<cd>::from(cadd(mine, give));
-            } else {
-#pragma unroll
-                for (int i = 0; i < NS; ++i) {
-                    const C v = group_sum<C, SB>(acc[u][c][i]);
-                    if (sl.grp == 0 && act[i]) yo[(size_t)c * g.B + sl.s[i]] = Prec<cd>::from(v);
-                }
-            }
+            for (int c = 0; c < 3; ++c) yo[(size_t)c * g.B] = Prec<cd>::from(acc[u][c][i]);
         }
     }
 }
 
-template <typename C, int GT, int VC, int SB, int NS>
+template <typename C, int VC, int SB, int NS>
 __global__ __launch_bounds__(64, 3) void k_gather_lds(gcore::GatherArgs<C> g) {
     using namespace gcore;
-    static_assert(GT <= 3, "the passes below cover 1..3 row tets");
-    __shared__ __align__(16) unsigned char sm[Shape<C, GT, VC>::BYTES];
+    constexpr int G = 64 / SB, NTMAX = (ROW_GT + G - 1) / G;  // lane groups, rows of each
+    static_assert(NTMAX <= 3 && ROW_GT / 2 * VC <= 64, "passes below; one block of each half per lane");
+    __shared__ __align__(16) unsigned char sm[Shape<C, G * NTMAX, VC>::BYTES];
     const int lane = threadIdx.x;
     const long long nw = (long long)g.n_groups * ((g.B + SB * NS - 1) / (SB * NS));
     for (long long b = blockIdx.x; b < nw; b += gridDim.x) {
@@ -333,12 +325,71 @@ __global__ __launch_bounds__(64, 3) void k_gather_lds(gcore::GatherArgs<C> g) {
         const long long w = nw == gridDim.x ? xcd_remap(b, nw) : b;
         const int chunk = (int)(w / g.n_groups);
         const Item it = group_item(g, (int)(w - (long long)chunk * g.n_groups));
-        const int nt = it.t1 - it.t0;  // wave-uniform
+        const int nt = (it.t1 - it.t0 + G - 1) / G;  // wave-uniform
 #define PASS(N)                                                                          \
-    if constexpr (GT >= N)                                                               \
-        if (nt == N) gather_pass<C, N, GT, VC, SB, NS>(g, it, chunk, lane, sm);
+    if constexpr (NTMAX >= N)                                                            \
+        if (nt == N) gather_pass<C, N, VC, SB, NS>(g, it, chunk, lane, sm);
         PASS(1) PASS(2) PASS(3)
 #undef PASS
+    }
+}
+
+// complex128, 5 to 32 slots: three rows at a time, the columns shared by the lane
+// groups (24,708 tets x 7: 153 us against 231 with the rows shared; complex64 keeps
+// the order of its sums)
+template <typename C, int NT, int VC, int SB>
+__device__ __forceinline__ void gather_cols(const gcore::GatherArgs<C> &g, const gcore::Item &it, int tp, int chunk,
+                                            int lane, unsigned char *smraw) {
+    C *sm = (C *)smraw;
+    cf *smb = (cf *)smraw;
+    using namespace gcore;
+    const Slots<SB, 1> sl = lane_slots<SB, 1>(g, chunk, lane);
+    C acc[NT][3];
+    zero_acc<C, NT>(acc);
+    const long long off = g.in_off[sl.s[0]] + sl.s[0];
+    __syncthreads();  // the previous rows' reads of sm are done
+    stage_s4(g, tp, NT, lane, sm);
+    __syncthreads();
+    grid_share<C, NT, SB>(g, it, sl, sm, acc);
+    const int64_t rs = lane_row_start<C, ROW_GT / 2, VC>(g, tp, NT, lane);
+    int q = 0;
+    for_near_cubes(g, it, [&](int c0, int c1) {
+        for (int v0 = c0; v0 < c1; v0 += VC) {
+            const int nv = min(VC, c1 - v0);
+            __syncthreads();
+            stage_blocks<C, ROW_GT / 2, VC>(g, NT, nv, q, lane, rs, smb);
+            __syncthreads();
+            chunk_share<C, NT, VC, SB>(g, sl, off, v0, nv, smb, acc);
+            q += nv;
+        }
+    });
+    const bool write = sl.grp == 0 && sl.ok[0] && (!g.slot_active || g.slot_active[sl.s[0]]);
+#pragma unroll
+    for (int u = 0; u < NT; ++u)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const C v = group_sum<C, SB>(acc[u][c]);
+            if (write) g.y[(size_t)(3 * (tp + u) + c) * g.B + sl.s[0]] = Prec<cd>::from(v);
+        }
+}
+
+template <typename C, int VC, int SB>
+__global__ __launch_bounds__(64, 3) void k_gather_cols(gcore::GatherArgs<C> g) {
+    using namespace gcore;
+    constexpr int HT = ROW_GT / 2;
+    static_assert(HT == 3 && HT * VC <= 64, "passes below; one block per lane");
+    __shared__ __align__(16) unsigned char sm[Shape<C, HT, VC>::BYTES];
+    const int lane = threadIdx.x;
+    const long long nw = (long long)g.n_groups * 2 * ((g.B + SB - 1) / SB);
+    for (long long b = blockIdx.x; b < nw; b += gridDim.x) {
+        const long long w = nw == gridDim.x ? xcd_remap(b, nw) : b;
+        const int chunk = (int)(w / (2 * g.n_groups));
+        const int i = (int)(w - (long long)chunk * 2 * g.n_groups);
+        const Item it = group_item(g, i >> 1);
+        const int tp = it.t0 + (i & 1 ? HT : 0), nt = min(HT, it.t1 - tp);  // wave-uniform
+        if (nt == 1) gather_cols<C, 1, VC, SB>(g, it, tp, chunk, lane, sm);
+        if (nt == 2) gather_cols<C, 2, VC, SB>(g, it, tp, chunk, lane, sm);
+        if (nt == 3) gather_cols<C, 3, VC, SB>(g, it, tp, chunk, lane, sm);
     }
 }
 
@@ -462,9 +513,7 @@ __global__ __launch_bounds__(64, 3) void k_gather_mf(gcore::GatherArgs<cf> g) {
 // narrow kernel to 24 slots (24,708 tets: 16 slots 85 against 115 in a 64-slot
 // chunk, 24 slots 126 and 128; 43,248 tets, 24 slots 206 and 198).  Gather: one tet a
 // wave to 4 slots (1,680 tets x 3: 18; it reads every block by single lanes, which
-// costs more than it saves from 8: 24,708 tets 259 against 142), then row groups
-// with the lanes' slots fitted to the batch (24,708 tets: 16 slots 213, 24 slots
-// 348, with one thread per row and slot 462 and 637).
+// costs more than it saves from 8: 24,708 tets 259 against 142), then row groups.
 constexpr int SCATTER_NARROW = 24, GATHER_NARROW = 4;
 
 static unsigned grid_for(long long tot, int bs) {
@@ -534,21 +583,42 @@ void launch_gather_near(const MatvecArgs<C> &a, hipStream_t s) {
             return;
         }
     }
-    auto go = [&](auto sb, auto ns) {
+    using gcore::ROW_VC;
+    if constexpr (std::is_same<C, cd>::value)
+        if (a.B <= 32) {
+            auto cols = [&](auto sb) {
+                constexpr int SB = decltype(sb)::value;
+                hipLaunchKernelGGL((k_gather_cols<C, ROW_VC, SB>), dim3(grid_for(2LL * a.n_groups, 1)), dim3(64), 0, s, g);
+            };
+            if (a.B > 16)
+                cols(std::integral_constant<int, 32>{});
+            else if (a.B > 8)
+                cols(std::integral_constant<int, 16>{});
+            else
+                cols(std::integral_constant<int, 8>{});
+            HIP_CHECK(hipGetLastError());
+            return;
+        }
+    auto rows = [&](auto sb, auto ns) {
         constexpr int SB = decltype(sb)::value, NS = decltype(ns)::value;
         const long long nw = (long long)a.n_groups * ((a.B + SB * NS - 1) / (SB * NS));
-        hipLaunchKernelGGL((k_gather_lds<C, gcore::ROW_GT, gcore::ROW_VC, SB, NS>), dim3(grid_for(nw, 1)), dim3(64), 0,
-                           s, g);
+        hipLaunchKernelGGL((k_gather_lds<C, ROW_VC, SB, NS>), dim3(grid_for(nw, 1)), dim3(64), 0, s, g);
     };
     typedef std::integral_constant<int, 1> one;
-    if (a.B > 32)
-        go(std::integral_constant<int, 32>{}, std::integral_constant<int, 2>{});
-    else if (a.B > 16)
-        go(std::integral_constant<int, 32>{}, one{});
-    else if (a.B > 8)
-        go(std::integral_constant<int, 16>{}, one{});
-    else
-        go(std::integral_constant<int, 8>{}, one{});
+    typedef std::integral_constant<int, 32> half;
+    // two slots a lane where that still leaves two waves for each of the 1024 SIMDs
+    // (24,708 tets, 64 slots: 789 us against 847 with one; 4,686 tets, 48 slots 275
+    // against 233)
+    if (a.B > 32 && (long long)a.n_groups * ((a.B + 63) / 64) >= 2048)
+        rows(half{}, std::integral_constant<int, 2>{});
+    else if (sizeof(C) == 16 || a.B > 16)
+        rows(half{}, one{});
+    else if constexpr (sizeof(C) == 8) {
+        if (a.B > 8)
+            rows(std::integral_constant<int, 16>{}, one{});
+        else
+            rows(std::integral_constant<int, 8>{}, one{});
+    }
     HIP_CHECK(hipGetLastError());
 }
 
