@@ -44,10 +44,11 @@ void launch_mgs_reduce(const KrylovDims &d, int k, const SlotState *st, cd *H, c
 // verify = 1: restart residuals are true FP64 residuals and decide convergence
 // against tol_true (mixed precision); an Arnoldi estimate below tol times the
 // cycle's starting residual ends a cycle
+// host, host_err: the new states and *err also go to page-locked host memory
 // park = 1: a slot whose cycle ends goes to PH_PARK instead of PH_RESTART
 void launch_slot_update(const KrylovDims &d, SlotState *st, cd *H, cd *cs, cd *sn, cd *g, cd *y,
                         const double *nrm2, const double *nav2, double tol, int restart, int verify, double tol_true,
-                        int park, hipStream_t s);
+                        int park, SlotState *host, const int *err, int *host_err, hipStream_t s);
 // PH_PARK -> PH_RESTART for every slot (a cycle boundary of the batch)
 void launch_unpark(const KrylovDims &d, SlotState *st, hipStream_t s);
 // basis V stored as complex128 or (mixed precision) complex64; x in X (n x B)
