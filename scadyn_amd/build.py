@@ -6,7 +6,7 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, 'csrc')
 LIB = os.path.join(HERE, 'libscadyn_amd.so')
-SOURCES = ['api.hip', 'geom.hip', 'setup.hip', 'fft.hip', 'fft_reg.hip', 'fft_reg_c64.hip', 'matvec.hip', 'krylov.hip', 'consumer.hip']
+SOURCES = ['api.hip', 'geom.hip', 'pinv.hip', 'setup.hip', 'fft.hip', 'fft_reg.hip', 'fft_reg_c64.hip', 'matvec.hip', 'krylov.hip', 'consumer.hip']
 OBJDIR = os.path.join(HERE, '_build')
 
 HIPCC_FLAGS = [
@@ -103,14 +103,15 @@ def build(verbose=False):
 SELFTEST = os.path.join(OBJDIR, 'fft_selftest')
 SELFTESTS = {'fft': ('fft_selftest.hip', SELFTEST), 'bmgs': ('bmgs_selftest.hip', os.path.join(OBJDIR, 'bmgs_selftest')),
              'gather': ('gather_selftest.hip', os.path.join(OBJDIR, 'gather_selftest')),
-             'mgsb': ('mgsb_selftest.hip', os.path.join(OBJDIR, 'mgsb_selftest'))}
+             'mgsb': ('mgsb_selftest.hip', os.path.join(OBJDIR, 'mgsb_selftest')),
+             'pinv': ('pinv_selftest.hip', os.path.join(OBJDIR, 'pinv_selftest'))}
 
 
 def build_selftest(verbose=False, which='fft'):
     """Host self-tests of kernel code (CPU only, AddressSanitizer on the host
     code): 'fft' the register FFT stages (links the library for the pass
     planner), 'bmgs' the block Gram-Schmidt bodies, 'gather' the LDS-staged
-    per-cube gather."""
+    per-cube gather, 'pinv' the pseudo-inverse (from the library)."""
     hipcc = os.environ.get('HIPCC', '/opt/rocm/bin/hipcc')
     os.makedirs(OBJDIR, exist_ok=True)
     src, exe = SELFTESTS[which]

@@ -156,65 +156,6 @@ void build_near_rows(const HostGeometry &g, NearRows &nr) {
     if (nr.P >= (long long)BLK_TRANSPOSE) fail(SCADYN_ERR_UNSUPPORTED, "too many near-zone blocks");
 }
 
-// Hestenes one-sided Jacobi SVD of A (m x n, column-major), m >= n.
-// Replaces ZGESVD in pinv (src/possu.f90:369-422): pinv = V diag(1/s) U^H.
-std::vector<cd> pinv_jacobi(const std::vector<cd> &A0, int m, int n, double thr) {
-    std::vector<cd> A = A0, V((size_t)n * n, cmk(0, 0));
-    for (int i = 0; i < n; ++i) V[(size_t)i * n + i] = cmk(1, 0);
-    auto col = [&](std::vector<cd> &M, int rows, int j) { return &M[(size_t)j * rows]; };
-    for (int sweep = 0; sweep < 60; ++sweep) {
-        double off = 0.0;
-        for (int p = 0; p < n - 1; ++p)
-            for (int q = p + 1; q < n; ++q) {
-                cd *ap = col(A, m, p), *aq = col(A, m, q);
-                double alpha = 0, beta = 0;
-                cd gam = cmk(0, 0);
-                for (int i = 0; i < m; ++i) {
-                    alpha += cabs2(ap[i]);
-                    beta += cabs2(aq[i]);
-                    gam = cadd(gam, cmulc(ap[i], aq[i]));
-                }
-                double ag = std::sqrt(cabs2(gam));
-                if (ag == 0.0) continue;
-                double rel = ag / std::sqrt(alpha * beta);
-                off = std::max(off, rel);
-                if (rel < 1e-17) continue;
-                // phase so that ap^H (aq e^{-i phi}) is real positive
-                cd ph = cmk(gam.x / ag, -gam.y / ag);
-                double zeta = (beta - alpha) / (2.0 * ag);
-                double t = (zeta >= 0 ? 1.0 : -1.0) / (std::fabs(zeta) + std::sqrt(1.0 + zeta * zeta));
-                double c = 1.0 / std::sqrt(1.0 + t * t), s = c * t;
-                for (int i = 0; i < m; ++i) {
-                    cd x = ap[i], y = cmul(aq[i], ph);
-                    ap[i] = csub(cscale(x, c), cscale(y, s));
-                    aq[i] = cadd(cscale(x, s), cscale(y, c));
-                }
-                cd *vp = col(V, n, p), *vq = col(V, n, q);
-                for (int i = 0; i < n; ++i) {
-                    cd x = vp[i], y = cmul(vq[i], ph);
-                    vp[i] = csub(cscale(x, c), cscale(y, s));
-                    vq[i] = cadd(cscale(x, s), cscale(y, c));
-                }
-            }
-        if (off < 1e-16) break;
-    }
-    // pinv (n x m) = sum_j v_j (1/s_j) u_j^H, u_j = a_j / s_j
-    std::vector<cd> P((size_t)n * m, cmk(0, 0));
-    for (int j = 0; j < n; ++j) {
-        cd *aj = col(A, m, j);
-        double s2 = 0;
-        for (int i = 0; i < m; ++i) s2 += cabs2(aj[i]);
-        double s = std::sqrt(s2);
-        if (!(s > thr)) continue;
-        cd *vj = col(V, n, j);
-        for (int i = 0; i < m; ++i) {
-            cd u = cscale(cconj(aj[i]), 1.0 / (s * s));  // conj(u_i)/s
-            for (int r = 0; r < n; ++r) P[(size_t)i * n + r] = cadd(P[(size_t)i * n + r], cmul(vj[r], u));
-        }
-    }
-    return P;
-}
-
 static bool is_smooth(int L) {
     int r = L;
     for (int p : {2, 3, 5, 7})

@@ -156,7 +156,7 @@ void build_near_rows(const HostGeometry &g, NearRows &nr);
 
 // SVD pseudo-inverse (one-sided Jacobi), singular values <= thr dropped.
 // A is m x n column-major; returns n x m column-major.
-std::vector<cd> pinv_jacobi(const std::vector<cd> &A, int m, int n, double thr);
+std::vector<cd> pinv_jacobi(const std::vector<cd> &A, int m, int n, double thr, bool wide = true);
 
 // Smallest 2,3,5,7-smooth length >= n, and its radix list (largest first).
 int smooth_length(int n);
