@@ -790,11 +790,15 @@ __global__ void k_retire(KrylovDims d, const int *__restrict__ col, SlotState *_
 //    load).
 //  * The tiles of a row chunk run together on one XCD (xcd_remap): its rows of mat and X
 //    come into that L2 once, not into all eight.
-// 129,744 rows, 336 x 336: 3.49 ms (33.6 TFLOP/s) before, 2.27 ms (51.6) now.
+// 129,744 rows, 336 x 336: 3.49 ms (33.6 TFLOP/s) before, 2.26 ms (51.9) now.
+//  * Two waves per SIMD at most, also where the registers let three or four in: the row
+//    chunks make two for each SIMD, and with room for more some got three and some one,
+//    as the kernel before had left them (91,422 rows, 320 x 259: 1,297 us or 1,617, now
+//    always 1,289).
 typedef double v4d __attribute__((ext_vector_type(4)));
 
 template <int TA, int TB>
-__global__ __launch_bounds__(64, 2) void k_tgemm(const cd *__restrict__ A, const cd *__restrict__ X, long long n,
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_tgemm(const cd *__restrict__ A, const cd *__restrict__ X, long long n,
                                                  int na, int nx, int ta, int tx, long long chunk,
                                                  cd *__restrict__ part) {
     const int lane = threadIdx.x, kk = lane >> 4, ii = lane & 15;
@@ -881,12 +885,23 @@ __global__ __launch_bounds__(64, 2) void k_tgemm(const cd *__restrict__ A, const
             }
 }
 
-__global__ void k_tgemm_reduce(const cd *__restrict__ part, int nz, size_t tot, cd *__restrict__ T) {
-    for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < tot; e += (size_t)gridDim.x * blockDim.x) {
-        cd a = cmk(0, 0);
-        for (int z = 0; z < nz; ++z) a = cadd(a, part[(size_t)z * tot + e]);
-        T[e] = a;
-    }
+// T = sum of the chunks' parts: 16 neighbouring elements by 16 shares of the chunks per
+// workgroup.  One thread per element adds the up to a thousand parts of a tall narrow
+// product one after the other: 64,935 rows, 21 x 57 took 286 us in all, now 47.
+__global__ __launch_bounds__(256) void k_tgemm_reduce(const cd *__restrict__ part, int nz, size_t tot,
+                                                      cd *__restrict__ T) {
+    __shared__ cd sm[16][16];
+    const int c = threadIdx.x & 15, share = threadIdx.x >> 4;
+    const size_t e = blockIdx.x * (size_t)16 + c;
+    cd a = cmk(0, 0);
+    if (e < tot)
+#pragma unroll 8
+        for (int z = share; z < nz; z += 16) a = cadd(a, part[(size_t)z * tot + e]);
+    sm[share][c] = a;
+    __syncthreads();
+    if (share || e >= tot) return;
+    for (int k = 1; k < 16; ++k) a = cadd(a, sm[k][c]);
+    T[e] = a;
 }
 
 // restart batch: columns slot[j] (j < cap, -1 none) of X (n x B) into the
@@ -1059,15 +1074,18 @@ void launch_tgemm(const cd *mat, const cd *X, long long n, int na, int nx, cd *T
                   hipStream_t s) {
     // tiles of 48 where that pads less than 32 (a larger tile reads its operands
     // fewer times); row chunks (multiples of 4 rows) so that two waves run on each of the
-    // 1024 SIMDs, limited by the partial-sum workspace and to 64 rows at least (a
-    // chunk is a serial chain: 576 rows, 6 x 6 in two chunks took 67 us)
+    // 1024 SIMDs, limited by the partial-sum workspace and to 32 rows at least (a
+    // chunk is a serial chain: 576 rows, 6 x 6 in two chunks took 67 us, 1,157 rows,
+    // 12 x 4 in chunks of 64 rows 27 us and of 32 rows 22); beyond 512 chunks the
+    // sum of the parts costs more than the shorter chains give (63,487 rows, 8 x 14:
+    // 44 us with 992 chunks, 58 with 1,984), so there 64 rows
     auto pick = [](int m) { return (m + 47) / 48 * 48 <= (m + 31) / 32 * 32 ? 3 : 2; };
     const int ba = pick(na), bx = pick(nx);
     const int ta = (na + 16 * ba - 1) / (16 * ba), tx = (nx + 16 * bx - 1) / (16 * bx);
     const size_t tot = (size_t)na * nx;
     long long nz = std::max<long long>(1, 2048 / ((long long)ta * tx));
     nz = std::min<long long>(nz, std::max<long long>(1, (long long)(work_elems / tot)));
-    nz = std::min<long long>(nz, std::max<long long>(1, n / 64));
+    nz = std::min<long long>(nz, std::max<long long>(1, std::max(n / 64, std::min(n / 32, 512LL))));
     long long chunk = (n + nz - 1) / nz;
     chunk = (chunk + 3) / 4 * 4;
     nz = (n + chunk - 1) / chunk;
@@ -1075,7 +1093,7 @@ void launch_tgemm(const cd *mat, const cd *X, long long n, int na, int nx, cd *T
     auto kern = ba == 3 ? (bx == 3 ? &k_tgemm<3, 3> : &k_tgemm<3, 2>) : (bx == 3 ? &k_tgemm<2, 3> : &k_tgemm<2, 2>);
     hipLaunchKernelGGL(kern, grid, dim3(64), 0, s, mat, X, n, na, nx, ta, tx, chunk, work);
     HIP_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(k_tgemm_reduce, dim3(256), dim3(256), 0, s, work, (int)nz, tot, T);
+    hipLaunchKernelGGL(k_tgemm_reduce, dim3((unsigned)((tot + 15) / 16)), dim3(256), 0, s, work, (int)nz, tot, T);
     HIP_CHECK(hipGetLastError());
 }
 

@@ -79,3 +79,28 @@ def test_project_noalloc_matches_project():
     for b in bufs:
         b.free()
     op.close()
+
+
+# one row; chunks of fewer than four rows at the end; the first shapes with 512 chunks of
+# 32 rows and with chunks of 64; parts that fill the shares of the sum unevenly; tiles
+# of 32 and 48 with a remainder.  Sums of up to 40,000 products: 1e-12.
+@pytest.mark.parametrize('n,na,nx', [(1, 1, 1), (31, 3, 2), (67, 1, 17), (1157, 12, 4), (16385, 5, 3), (32801, 4, 7),
+                                     (40001, 3, 2), (4099, 49, 65), (2050, 33, 97)])
+def test_project_shapes(n, na, nx):
+    from scadyn_amd import native
+    c, e, p, k = sphere_case(n_cells=5)
+    op = native.Operator(c, e, p, k)
+    hip = _hip()
+    rng = np.random.default_rng(12)
+    print(f'[no-alloc] {n} rows, {na} x {nx}', flush=True)
+    mat = rng.standard_normal((n, na)) + 1j * rng.standard_normal((n, na))
+    X = rng.standard_normal((n, nx)) + 1j * rng.standard_normal((n, nx))
+    mat_d, X_d, T_d = (DeviceBuffer(hip, 16 * m) for m in (n * na, n * nx, na * nx))
+    mat_d.put(mat)
+    X_d.put(X)
+    T_d.put(np.full((na, nx), np.nan + 0j))
+    op.project_noalloc(n, na, nx, mat_d.p.value, X_d.p.value, T_d.p.value)
+    assert rel(T_d.get(np.empty((na, nx), np.complex128)), mat.conj().T @ X) < 1e-12
+    for b in (mat_d, X_d, T_d):
+        b.free()
+    op.close()
