@@ -476,7 +476,7 @@ HD void line_reg_phase(int phase, const C *__restrict__ in, C *__restrict__ out,
 }
 
 // smallest compiled radix bound covering a pass (instances 12, 14, 16, 18 and
-// 20: complex128 takes 106, 124, 139, 158 and 174 VGPRs, i.e. 4, 4, 3, 3 and 2
+// 20: complex128 takes 102, 124, 136, 156 and 170 VGPRs, i.e. 4, 4, 3, 3 and 2
 // waves per SIMD)
 HD int reg_rmax(const LinePass &p) {
     const int r = p.rad[0] > p.rad[1] ? p.rad[0] : p.rad[1];
