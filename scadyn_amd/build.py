@@ -104,13 +104,15 @@ SELFTEST = os.path.join(OBJDIR, 'fft_selftest')
 SELFTESTS = {'fft': ('fft_selftest.hip', SELFTEST), 'bmgs': ('bmgs_selftest.hip', os.path.join(OBJDIR, 'bmgs_selftest')),
              'gather': ('gather_selftest.hip', os.path.join(OBJDIR, 'gather_selftest')),
              'mgsb': ('mgsb_selftest.hip', os.path.join(OBJDIR, 'mgsb_selftest')),
+             'fft_inst': ('fft_inst_selftest.hip', os.path.join(OBJDIR, 'fft_inst_selftest')),
              'pinv': ('pinv_selftest.hip', os.path.join(OBJDIR, 'pinv_selftest'))}
 
 
 def build_selftest(verbose=False, which='fft'):
     """Host self-tests of kernel code (CPU only, AddressSanitizer on the host
     code): 'fft' the register FFT stages (links the library for the pass
-    planner), 'bmgs' the block Gram-Schmidt bodies, 'gather' the LDS-staged
+    planner), 'fft_inst' its compiled instances at the planner's widths, 'bmgs' the block
+    Gram-Schmidt bodies, 'gather' the LDS-staged
     per-cube gather, 'pinv' the pseudo-inverse (from the library)."""
     hipcc = os.environ.get('HIPCC', '/opt/rocm/bin/hipcc')
     os.makedirs(OBJDIR, exist_ok=True)

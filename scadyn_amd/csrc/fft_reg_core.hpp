@@ -349,13 +349,15 @@ HD void conv_compute(C *v, const C *lds, const C *tw, const C *__restrict__ fg, 
         const int gy = (int)(xy / (unsigned)ci.Lx), gx = (int)(xy - (unsigned)gy * (unsigned)ci.Lx);
         const int kx = imin(gx, ci.Lx - gx), ky = imin(gy, ci.Ly - gy);
         // row min(k, Lz - k) of the octant as the smaller of two running byte
-        // offsets, in 32 bits (the octant is checked to stay below 2^32 bytes)
-        const unsigned zs = (unsigned)(ci.Hy * ci.Hx) * (unsigned)sizeof(C);
-        const unsigned f0 = (unsigned)(ky * ci.Hx + kx) * (unsigned)sizeof(C), step = (unsigned)LR * zs;
-        unsigned up = f0 + (unsigned)j * zs, down = f0 + (unsigned)(ci.Lz - j) * zs;
+        // offsets; the larger starts at nearly twice the octant's size.  In 32 bits
+        // where both fit (conv_near32), which the SH >= 0 instances require
+        typedef typename std::conditional<(SH >= 0), unsigned, size_t>::type Off;
+        const Off zs = (Off)ci.Hy * (Off)ci.Hx * (Off)sizeof(C);
+        const Off f0 = (Off)((Off)ky * (Off)ci.Hx + (Off)kx) * (Off)sizeof(C), step = (Off)LR * zs;
+        Off up = f0 + (Off)j * zs, down = f0 + (Off)(ci.Lz - j) * zs;
         sfor<0, R>([&](auto rr) {
             constexpr int r = CV(rr);
-            const unsigned f = up < down ? up : down;
+            const Off f = up < down ? up : down;
             v[r] = cmul(v[r], *reinterpret_cast<const C *>(reinterpret_cast<const char *>(fg) + f));
             up += step;
             down -= step;
@@ -481,6 +483,23 @@ HD void line_reg_phase(int phase, const C *__restrict__ in, C *__restrict__ out,
 HD int reg_rmax(const LinePass &p) {
     const int r = p.rad[0] > p.rad[1] ? p.rad[0] : p.rad[1];
     return r <= 12 ? 12 : (r <= 14 ? 14 : (r <= 16 ? 16 : (r <= 18 ? 18 : 20)));
+}
+
+// true when the convolution's running offsets into the octant of FFT(G) stay in
+// 32 bits: the largest is below (Lz + 1) planes of Hx Hy elements
+HD bool conv_near32(const ConvInfo &ci, size_t elem) {
+    return (double)ci.Hx * (double)ci.Hy * ((double)ci.Lz + 1.0) * (double)elem <= 4294967296.0;
+}
+
+// The instance for a pass: log2 of its tile width where one is compiled for that
+// width (those the planner chooses on all but the narrowest batches) and every
+// offset it keeps in 32 bits fits: a wave's lanes span 64 / ti items of a line,
+// and the convolution walks the octant.  Else -1: any width, 64-bit offsets.
+HD int reg_shift(const LinePass &p, const ConvInfo &ci, int mode, size_t elem) {
+    if ((double)(64 / p.ti) * (double)p.inner * (double)elem >= 4294967296.0) return -1;
+    if (mode == 1 && !conv_near32(ci, elem)) return -1;
+    const int sh = log2_pow2(p.ti), s0 = mode == 1 ? 3 : (elem == 16 ? 3 : 4);
+    return sh == s0 || sh == s0 + 1 ? sh : -1;
 }
 
 }  // namespace regfft

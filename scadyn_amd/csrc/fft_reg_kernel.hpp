@@ -80,15 +80,10 @@ void launch_line_reg(const LinePass &p, const C *in, C *out, const C *tw, int si
     const size_t lds = line_pass_lds(p, sizeof(C));
     if (p.threads > reg_max_threads(sizeof(C))) fail(SCADYN_ERR_UNSUPPORTED, "FFT tile exceeds the thread bound");
     if (lds > 65536) fail(SCADYN_ERR_UNSUPPORTED, "FFT tile exceeds 64 KiB of LDS");
-    if (mode == 1 && (double)ci.Hx * ci.Hy * (ci.Lz / 2 + 1) * sizeof(C) >= 4294967296.0)
-        fail(SCADYN_ERR_UNSUPPORTED, "FFT of the Green's function too large");
     const dim3 grid((unsigned)blocks), block(p.threads);
     const int rm = reg_rmax(p);
-    // the widths the planner chooses on all but the narrowest batches; a wave's
-    // lanes span 64 / ti items of a line
     constexpr int S0 = sizeof(C) == 16 ? 3 : 4;
-    const bool near32 = (double)(64 / p.ti) * (double)p.inner * sizeof(C) < 4294967296.0;
-    const int sh = near32 ? log2_pow2(p.ti) : -1;
+    const int sh = reg_shift(p, ci, mode, sizeof(C));
 #define GO(M, S) launch_sh<M, C, S>(rm, grid, block, lds, s, in, out, p, tw, sign, fg, ci)
     if (mode == 0) {
         if (sh == S0)
