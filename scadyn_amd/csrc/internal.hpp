@@ -48,6 +48,13 @@ __host__ __device__ inline long long xcd_remap(long long b, long long G) {
     return x < tall ? x * per + j : tall * per + (x - tall) * (per - 1) + j;
 }
 
+// Workgroups for tot items, bs to a workgroup: capped, the kernels launched with it
+// stride over the rest.  A launch holds less than 2^32 threads.
+inline unsigned grid_for(long long tot, int bs) {
+    const long long g = (tot + bs - 1) / bs;
+    return (unsigned)(g < 1 ? 1 : (g < (1LL << 20) ? g : 1LL << 20));
+}
+
 __host__ __device__ inline cd cmk(double r, double i) { return make_double2(r, i); }
 __host__ __device__ inline cd cadd(cd a, cd b) { return make_double2(a.x + b.x, a.y + b.y); }
 __host__ __device__ inline cd csub(cd a, cd b) { return make_double2(a.x - b.x, a.y - b.y); }

@@ -10,6 +10,7 @@
 
 #include "matvec.hpp"
 #include "gather_core.hpp"
+#include "scatter_core.hpp"
 
 namespace scadyn {
 
@@ -32,57 +33,20 @@ __device__ inline C group_sum(C v) {
     return v;
 }
 
-// scatter (sparse_T_matmul, src/sparse.f90:13-43, + vec2arr2): node p sums the
-// stencil weights of the tets of the <= 8 cubes whose box holds p
-template <typename C, int SB>
-__global__ __launch_bounds__(256) void k_scatter_narrow(const C *__restrict__ xin,
-                                                        const long long *__restrict__ in_off, int B,
-                                                        const int *__restrict__ cube_start,
-                                                        const C *__restrict__ S4, int Nx, int Ny, int Nz, int ncx,
-                                                        int ncy, int ncz, C *__restrict__ grid) {
-    // at most 16 groups: a node has about 20 tets, and with few slots a wave then
-    // takes several nodes
-    constexpr int G = 64 / SB < 16 ? 64 / SB : 16, NODES = 64 / (SB * G);
-    const int lane = threadIdx.x & 63, b = lane & (SB - 1), g = (lane / SB) % G;
-    const long long p = ((long long)blockIdx.x * 4 + (threadIdx.x >> 6)) * NODES + lane / (SB * G);
-    if (p >= (long long)Nx * Ny * Nz) return;  // a node's lanes leave together
-    const int px = (int)(p % Nx), py = (int)((p / Nx) % Ny), pz = (int)(p / ((long long)Nx * Ny));
-    const int bl = b < B ? b : B - 1;  // idle lanes load the last slot and store nothing
-    const C *xb = xin + in_off[bl] + bl;
-    C a0 = Prec<C>::zero(), a1 = a0, a2 = a0, a3 = a0;
-    // cubes c with 2c <= p <= 2c+2 per axis; those of one x line hold consecutive tets
-    const int cx0 = max(0, (px - 1) / 2), cx1 = min(ncx - 1, px / 2);
-    const int cy0 = max(0, (py - 1) / 2), cy1 = min(ncy - 1, py / 2);
-    const int cz0 = max(0, (pz - 1) / 2), cz1 = min(ncz - 1, pz / 2);
-    for (int cz = cz0; cz <= cz1; ++cz)
-        for (int cy = cy0; cy <= cy1; ++cy) {
-            const int line = ncx * (cy + ncy * cz);
-            const int t1 = cx1 >= cx0 ? cube_start[line + cx1 + 1] : 0, ts = cx1 >= cx0 ? cube_start[line + cx1] : 0;
-            const int j = 3 * (py - 2 * cy) + 9 * (pz - 2 * cz);
-            for (int t = (cx1 >= cx0 ? cube_start[line + cx0] : 0) + g; t < t1; t += G) {
-                const int jt = j + px - 2 * (t < ts ? cx0 : cx1);
-                const C *s = S4 + ((size_t)t * 27 + jt) * 4;
-                const C x0 = xb[(size_t)(3 * t) * B], x1 = xb[(size_t)(3 * t + 1) * B],
-                        x2 = xb[(size_t)(3 * t + 2) * B];
-                const C s0 = s[0];
-                cfma(a0, s0, x0);
-                cfma(a1, s0, x1);
-                cfma(a2, s0, x2);
-                cfma(a3, s[1], x0);
-                cfma(a3, s[2], x1);
-                cfma(a3, s[3], x2);
-            }
-        }
-    a0 = group_sum<C, SB, SB * G>(a0);
-    a1 = group_sum<C, SB, SB * G>(a1);
-    a2 = group_sum<C, SB, SB * G>(a2);
-    a3 = group_sum<C, SB, SB * G>(a3);
-    if (g == 0 && b < B) {
-        C *gp = grid + (size_t)p * 4 * B + b;
-        gp[0] = a0;
-        gp[(size_t)B] = a1;
-        gp[(size_t)2 * B] = a2;
-        gp[(size_t)3 * B] = a3;
+// scatter (scatter_core.hpp); the launch caps the grid, a workgroup strides over nodes
+template <typename C, int SB, int G>
+__global__ __launch_bounds__(score::THREADS) void k_scatter_narrow(score::ScatterArgs<C> s) {
+    constexpr int PER = score::nodes_per_group<SB, G>();
+    const int b = threadIdx.x & (SB - 1), g = (threadIdx.x / SB) % G;
+    const int bl = b < s.B ? b : s.B - 1;  // idle lanes load the last slot and store nothing
+    const long long nodes = (long long)s.Nx * s.Ny * s.Nz;
+    // a node's lanes leave together
+    for (long long p = (long long)blockIdx.x * PER + threadIdx.x / (SB * G); p < nodes; p += (long long)gridDim.x * PER) {
+        C a[4];
+        score::node_share<C, G>(s, p, bl, g, a);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) a[c] = group_sum<C, SB, SB * G>(a[c]);
+        if (g == 0 && b < s.B) score::write_node(s, p, b, a);
     }
 }
 
@@ -516,11 +480,6 @@ __global__ __launch_bounds__(64, 3) void k_gather_mf(gcore::GatherArgs<cf> g) {
 // costs more than it saves from 8: 24,708 tets 259 against 142), then row groups.
 constexpr int SCATTER_NARROW = 24, GATHER_NARROW = 4;
 
-static unsigned grid_for(long long tot, int bs) {
-    long long g = (tot + bs - 1) / bs;
-    return (unsigned)std::min<long long>(std::max<long long>(g, 1), 1LL << 20);
-}
-
 // f(integral constant SB): the lanes' slots of a narrow batch of B
 template <typename F>
 static void narrow_slots(int B, F &&f) {
@@ -545,12 +504,13 @@ void launch_scatter(const MatvecArgs<C> &a, hipStream_t s) {
         hipLaunchKernelGGL((k_scatter_blk_w64<C>), dim3(grid_for(nw, 4)), dim3(256), 0, s, a.xin, a.in_off, a.B,
                            a.cube_start, a.S4, a.Nx, a.Ny, a.Nz, a.ncx, a.ncy, a.ncz, a.grid_in);
     } else {
-        const long long nodes = (long long)a.Nx * a.Ny * a.Nz;
+        const score::ScatterArgs<C> sa = {a.xin, a.in_off, a.B,   a.cube_start, a.S4,  a.Nx,
+                                          a.Ny,  a.Nz,     a.ncx, a.ncy,        a.ncz, a.grid_in};
         narrow_slots(a.B, [&](auto sb) {
-            constexpr int SB = decltype(sb)::value, per = SB < 4 ? 16 / SB : 4;  // nodes per workgroup
-            hipLaunchKernelGGL((k_scatter_narrow<C, SB>), dim3((unsigned)((nodes + per - 1) / per)), dim3(256), 0, s,
-                               a.xin, a.in_off, a.B, a.cube_start, a.S4, a.Nx, a.Ny, a.Nz, a.ncx, a.ncy, a.ncz,
-                               a.grid_in);
+            constexpr int SB = decltype(sb)::value, G = 64 / SB < 16 ? 64 / SB : 16;
+            hipLaunchKernelGGL((k_scatter_narrow<C, SB, G>),
+                               dim3(grid_for((long long)a.Nx * a.Ny * a.Nz, score::nodes_per_group<SB, G>())),
+                               dim3(score::THREADS), 0, s, sa);
         });
     }
     HIP_CHECK(hipGetLastError());
