@@ -11,6 +11,7 @@
 //                  src/mie.f90:408-496)
 #include <cmath>
 
+#include "pairs_core.hpp"
 #include "setup.hpp"
 
 namespace scadyn {
@@ -487,30 +488,12 @@ __global__ void k_fg_octant(const cd *__restrict__ F, cd *__restrict__ fg, int L
 // of the pair and entry lists.  At 43,248 tets (6.4 M entries) an operator is
 // set up in 33 ms; with the pairs pushed, counted and sorted one by one on the
 // host, and the lists copied over, it took 110 ms, at 369,390 tets 222 ms.
-__device__ inline int near_cube(int c, int o, const GridDesc &g) {
-    const int x = c % g.ncx + o % 3 - 1, y = (c / g.ncx) % g.ncy + (o / 3) % 3 - 1, z = c / (g.ncx * g.ncy) + o / 9 - 1;
-    if (x < 0 || x >= g.ncx || y < 0 || y >= g.ncy || z < 0 || z >= g.ncz) return -1;
-    return x + g.ncx * (y + g.ncy * z);
-}
-// first tet of [b, e) whose reference id is >= id
-__device__ inline int first_from(const int *__restrict__ perm, int b, int e, int id) {
-    while (b < e) {
-        const int m = (b + e) >> 1;
-        if (perm[m] < id)
-            b = m + 1;
-        else
-            e = m;
-    }
-    return b;
-}
 __global__ __launch_bounds__(64) void k_pair_count(const int *__restrict__ cs, const int *__restrict__ perm, GridDesc g,
                                                    uint32_t *__restrict__ tot) {
     const int c = blockIdx.x, t0 = cs[c], n = cs[c + 1] - t0;
-    int sum = 0;
-    for (int s = threadIdx.x; s < 27 * n; s += 64) {
-        const int nc = near_cube(c, s / n, g);
-        if (nc >= 0) sum += cs[nc + 1] - first_from(perm, cs[nc], cs[nc + 1], perm[t0 + s % n]);
-    }
+    int sum = 0, b;
+    for (int s = threadIdx.x; s < 27 * n; s += 64)
+        sum += pairs::kept(cs, perm, pairs::near_cube(c, s / n, g), t0 + s % n, b);
     for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
     if (threadIdx.x == 0) tot[c] = (uint32_t)sum;
 }
@@ -543,12 +526,8 @@ __global__ __launch_bounds__(64) void k_pair_fill(const int *__restrict__ cs, co
     uint32_t run = base[c];
     for (int s0 = 0; s0 < 27 * n; s0 += 64) {
         const int s = s0 + lane, o = s / max(n, 1), T = t0 + s % max(n, 1);
-        int b = 0, cnt = 0;
-        const int nc = s < 27 * n ? near_cube(c, o, g) : -1;
-        if (nc >= 0) {
-            b = first_from(perm, cs[nc], cs[nc + 1], perm[T]);
-            cnt = cs[nc + 1] - b;
-        }
+        int b;
+        const int cnt = pairs::kept(cs, perm, s < 27 * n ? pairs::near_cube(c, o, g) : -1, T, b);
         int inc = cnt;
         for (int d = 1; d < 64; d <<= 1) {
             const int v = __shfl_up(inc, d, 64);
@@ -569,28 +548,7 @@ __global__ __launch_bounds__(64) void k_row_fill(const int *__restrict__ cs, con
                                                  const int64_t *__restrict__ row_start,
                                                  const uint32_t *__restrict__ pos, int *__restrict__ ent_col,
                                                  uint32_t *__restrict__ ent_blk) {
-    const int c = blockIdx.x, t0 = cs[c], t1 = cs[c + 1], n = t1 - t0;
-    if (n == 0) return;
-    int col = 0;  // entries of the near cubes before o
-    for (int o = 0; o < 27; ++o) {
-        const int nc = near_cube(c, o, g);
-        if (nc < 0) continue;
-        const int b0 = cs[nc], b1 = cs[nc + 1], m = b1 - b0;
-        for (int l = threadIdx.x; l < n * m; l += 64) {
-            const int T = t0 + l / m, B = b0 + l % m;
-            uint32_t blk;
-            if (perm[B] >= perm[T])
-                blk = pos[(size_t)27 * t0 + (size_t)o * n + (T - t0)] + (uint32_t)(B - first_from(perm, b0, b1, perm[T]));
-            else
-                blk = (pos[(size_t)27 * b0 + (size_t)(26 - o) * m + (B - b0)] +
-                       (uint32_t)(T - first_from(perm, t0, t1, perm[B]))) |
-                      BLK_TRANSPOSE;
-            const int64_t r = row_start[T] + col + l % m;
-            ent_col[r] = B;
-            ent_blk[r] = blk;
-        }
-        col += m;
-    }
+    pairs::fill_rows(cs, perm, g, row_start, pos, ent_col, ent_blk, blockIdx.x, threadIdx.x);
 }
 
 // ---- near-zone G between box nodes for the 27 cube offsets ---------------------
