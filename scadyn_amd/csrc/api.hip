@@ -778,22 +778,14 @@ static void h2d_sync(void *dst, const void *src, size_t bytes, hipStream_t s) {
     HIP_CHECK(hipStreamSynchronize(s));
 }
 
-static int auto_batch(scadyn_operator *op, int ncols) {
-    if (op->opts.batch > 0) return std::min(op->opts.batch, std::max(ncols, 1));
-    // an existing workspace that holds enough slots is reused (no reallocation)
-    if (op->ws && op->ws->m == op->opts.maxit && op->ws->B >= std::min(ncols, 64)) return op->ws->B;
-    size_t free_b = 0, total_b = 0;
-    HIP_CHECK(hipMemGetInfo(&free_b, &total_b));
-    size_t per = slot_bytes(op, op->opts.maxit);
-    size_t cap = (size_t)(0.75 * (double)free_b) / std::max<size_t>(per, 1);
-    if (cap == 0) fail(SCADYN_ERR_MEMORY, "not enough device memory for one RHS slot");
-    // Above 64 columns, equal generations of at most 128 slots.  A step costs about
-    // one part per slot (transforms, Krylov sweeps; idle slots too) and half a part
-    // per lane of the 64-slot chunks that the scatter and gather run, so take the
-    // split with the least of that over all generations, the fewest where two are
-    // equal: 70 columns run as one batch of 70 rather than as 64 and 6 (the
-    // 43,248-tet FP64 bar: 126 ms instead of 163; the 24,708-tet mixed bar 167 instead of
-    // 237).
+// Slots for ncols columns where at most cap fit: up to 64 columns one batch; above,
+// equal generations of at most 128 slots.  A step costs about one part per slot
+// (transforms, Krylov sweeps; idle slots too) and half a part per lane of the
+// 64-slot chunks that the scatter and gather run, so take the split with the least
+// of that over all generations, the fewest where two are equal: 70 columns run as
+// one batch of 70 rather than as 64 and 6 (the 43,248-tet FP64 bar: 126 ms instead of
+// 163; the 24,708-tet mixed bar 167 instead of 237).
+static int batch_width(int ncols, size_t cap) {
     int B = std::min(64, ncols);
     if (ncols > 64) {
         long long best = -1;
@@ -807,9 +799,21 @@ static int auto_batch(scadyn_operator *op, int ncols) {
             }
         }
     }
+    return (int)std::min<size_t>((size_t)B, cap);
+}
+
+static int auto_batch(scadyn_operator *op, int ncols) {
+    if (op->opts.batch > 0) return std::min(op->opts.batch, std::max(ncols, 1));
+    // an existing workspace that holds enough slots is reused (no reallocation)
+    if (op->ws && op->ws->m == op->opts.maxit && op->ws->B >= std::min(ncols, 64)) return op->ws->B;
+    size_t free_b = 0, total_b = 0;
+    HIP_CHECK(hipMemGetInfo(&free_b, &total_b));
+    size_t per = slot_bytes(op, op->opts.maxit);
+    size_t cap = (size_t)(0.75 * (double)free_b) / std::max<size_t>(per, 1);
+    if (cap == 0) fail(SCADYN_ERR_MEMORY, "not enough device memory for one RHS slot");
+    int B = batch_width(ncols, cap);
     // memory, not the column count, limits the batch
     const bool capped = cap < (size_t)std::min(ncols, 128);
-    B = (int)std::min<size_t>((size_t)B, cap);
     // a memory-capped batch: round down to a width whose last 64-slot chunk holds
     // at least 48 slots
     if (capped && B > 64 && B % 64 != 0 && B % 64 < 48) B -= B % 64;
@@ -2018,7 +2022,8 @@ int scadyn_footprint(const scadyn_mesh *mesh, const scadyn_opts *opts, int32_t n
     NearRows rows;
     build_near_rows(g, rows);
     const int ncol = 2 * ((nmax + 1) * (nmax + 1) - 1);
-    const int B = o.batch > 0 ? std::min(o.batch, ncol) : std::min(ncol, 64);
+    // the width that the solve takes where memory does not limit it
+    const int B = o.batch > 0 ? std::min(o.batch, ncol) : batch_width(ncol, SIZE_MAX);
     *bytes = (int64_t)footprint_of(g, rows.P, o, nmax, B).peak();
     ABI_CATCH
 }
