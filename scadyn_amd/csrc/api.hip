@@ -165,6 +165,7 @@ struct Workspace {
     int *col = nullptr, *ret = nullptr, *flag = nullptr;
     cd *cc = nullptr, *hprev = nullptr;
     int nwg = 0;
+    size_t bytes() const { return mem.bytes + mv.mem.bytes + (rs ? rs->mem.bytes : 0); }
 };
 
 }  // namespace scadyn
@@ -778,13 +779,18 @@ static void h2d_sync(void *dst, const void *src, size_t bytes, hipStream_t s) {
     HIP_CHECK(hipStreamSynchronize(s));
 }
 
+// Cost of ncols columns in generations of B slots.  A step costs about one part per
+// slot (transforms, Krylov sweeps; idle slots too) and half a part per lane of the
+// 64-slot chunks that the scatter and gather run.
+static long long batch_cost(int ncols, int B) {
+    return (long long)((ncols + B - 1) / B) * (B + 32 * ((B + 63) / 64));
+}
+
 // Slots for ncols columns where at most cap fit: up to 64 columns one batch; above,
-// equal generations of at most 128 slots.  A step costs about one part per slot
-// (transforms, Krylov sweeps; idle slots too) and half a part per lane of the
-// 64-slot chunks that the scatter and gather run, so take the split with the least
-// of that over all generations, the fewest where two are equal: 70 columns run as
-// one batch of 70 rather than as 64 and 6 (the 43,248-tet FP64 bar: 126 ms instead of
-// 163; the 24,708-tet mixed bar 167 instead of 237).
+// the equal generations of at most 128 slots that cost least, the fewest where two
+// are equal: 70 columns run as one batch of 70 rather than as 64 and 6 (the
+// 43,248-tet FP64 bar: 126 ms instead of 163; the 24,708-tet mixed bar 167 instead of
+// 237).
 static int batch_width(int ncols, size_t cap) {
     int B = std::min(64, ncols);
     if (ncols > 64) {
@@ -792,7 +798,7 @@ static int batch_width(int ncols, size_t cap) {
         for (int gen = (ncols + 127) / 128; gen <= (ncols + 31) / 32; ++gen) {
             const int Bg = (ncols + gen - 1) / gen;
             if ((size_t)Bg > cap) continue;
-            const long long cost = (long long)gen * (Bg + 32 * ((Bg + 63) / 64));
+            const long long cost = batch_cost(ncols, Bg);
             if (best < 0 || cost < best) {
                 best = cost;
                 B = Bg;
@@ -804,10 +810,17 @@ static int batch_width(int ncols, size_t cap) {
 
 static int auto_batch(scadyn_operator *op, int ncols) {
     if (op->opts.batch > 0) return std::min(op->opts.batch, std::max(ncols, 1));
-    // an existing workspace that holds enough slots is reused (no reallocation)
-    if (op->ws && op->ws->m == op->opts.maxit && op->ws->B >= std::min(ncols, 64)) return op->ws->B;
+    // An existing workspace that holds enough slots is reused (no reallocation).
+    // Above 64 columns only where it holds them all or its generations cost no more
+    // than a sixteenth above the rule's: the width of the call before (64 from a
+    // product of 64 vectors, say) would else run 70 columns as 64 and 6 again.
+    const int have = op->ws && op->ws->m == op->opts.maxit ? op->ws->B : 0;
+    if (have >= std::min(ncols, 64) &&
+        (have >= ncols || 16 * batch_cost(ncols, have) <= 17 * batch_cost(ncols, batch_width(ncols, SIZE_MAX))))
+        return have;
     size_t free_b = 0, total_b = 0;
     HIP_CHECK(hipMemGetInfo(&free_b, &total_b));
+    if (op->ws) free_b += op->ws->bytes();  // goes before the new one is made
     size_t per = slot_bytes(op, op->opts.maxit);
     size_t cap = (size_t)(0.75 * (double)free_b) / std::max<size_t>(per, 1);
     if (cap == 0) fail(SCADYN_ERR_MEMORY, "not enough device memory for one RHS slot");

@@ -2,9 +2,10 @@
 takes.  The width by its rule, written out: up to 64 columns one batch, above the
 equal generations of at most 128 slots with the least sum of slots and half the lanes
 of their 64-slot chunks, the fewest where two are equal."""
+import numpy as np
 import pytest
 
-from helpers import sphere_case
+from helpers import rel, sphere_case
 
 
 def width(ncols):
@@ -50,3 +51,27 @@ def test_solve_takes_that_width(nmax):
     op.tmatrix(nmax)
     assert op.info()['batch'] == width(columns(nmax))
     op.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('first,nmax,slots', [(64, 5, 70),   # 64 and 6 would cost 1.4 times one batch of 70
+                                              (64, 7, 64),   # two batches of 64 within 2% of one of 126
+                                              (100, 5, 100), # holds them all
+                                              (64, 4, 64)])
+def test_width_does_not_depend_on_the_call_before(first, nmax, slots):
+    """A workspace of `first` slots, from a product, then a T-matrix."""
+    from scadyn_amd import native
+    c, e, p, k = sphere_case()
+    print(f'[batch-width] {columns(nmax)} columns after a product of {first}', flush=True)
+    op = native.Operator(c, e, p, k)
+    op.matvec(np.ones((first, 3 * e.shape[0]), complex))
+    assert op.info()['batch'] == first
+    T, it = op.tmatrix(nmax)
+    assert op.info()['batch'] == slots
+    fresh = native.Operator(c, e, p, k)
+    Tf, itf = fresh.tmatrix(nmax)
+    assert np.array_equal(it, itf)
+    for a, b in zip(T, Tf):
+        assert rel(a, b) < 1e-9
+    op.close()
+    fresh.close()
