@@ -14,15 +14,15 @@
 
 namespace scadyn {
 
-// ---- narrow batches (fewer than 32 slots) --------------------------------------
-// One wave per grid node (or several, scatter) or tet (gather): the lanes are SB
-// slots (a power of two >= B) x 64 / SB groups that share the sum's terms, combined at the
-// end by a fixed exchange over the groups.  A few slots leave nothing to hide a
+// ---- narrow batches (up to 32 slots) -------------------------------------------
+// One wave per tet (gather) or a few nodes (scatter): the lanes are SB slots (a power
+// of two >= B) x groups that share the sum's terms, combined at the end by a fixed
+// exchange over the groups.  A few slots leave nothing to hide a
 // serial chain of loads behind, so what bounds these kernels is the number of
 // dependent rounds: 160 near tets and 27 nodes per row, about 20 tets per node,
 // divided by the groups.  With one thread per (row, slot), which walked them all,
-// 1,680 tets x 1 vector took 164 us (gather) and 29 us (scatter), now 13 and 11;
-// 24,708 tets x 1 206 and 37, now 95 and 26.
+// 1,680 tets x 1 vector took 164 us (gather) and 29 us (scatter), now 13 and 10;
+// 24,708 tets x 1 206 and 37, now 95 and 21.
 template <typename C, int SB, int END = 64>
 __device__ inline C group_sum(C v) {
 #pragma unroll
@@ -47,6 +47,20 @@ __global__ __launch_bounds__(score::THREADS) void k_scatter_narrow(score::Scatte
 #pragma unroll
         for (int c = 0; c < 4; ++c) a[c] = group_sum<C, SB, SB * G>(a[c]);
         if (g == 0 && b < s.B) score::write_node(s, p, b, a);
+    }
+}
+
+// one thread per (node, slot), the node's tets in order
+template <typename C>
+__global__ __launch_bounds__(score::THREADS) void k_scatter_flat(score::ScatterArgs<C> s) {
+    const long long tot = (long long)s.Nx * s.Ny * s.Nz * s.B;
+    for (long long e = blockIdx.x * (long long)score::THREADS + threadIdx.x; e < tot;
+         e += (long long)gridDim.x * score::THREADS) {
+        const long long p = e / s.B;
+        const int b = (int)(e - p * s.B);
+        C a[4];
+        score::node_share<C, 1>(s, p, b, 0, a);
+        score::write_node(s, p, b, a);
     }
 }
 
@@ -473,12 +487,10 @@ __global__ __launch_bounds__(64, 3) void k_gather_mf(gcore::GatherArgs<cf> g) {
     }
 }
 
-// Widths, us per launch in complex128 (complex64 orders them alike).  Scatter: the
-// narrow kernel to 24 slots (24,708 tets: 16 slots 85 against 115 in a 64-slot
-// chunk, 24 slots 126 and 128; 43,248 tets, 24 slots 206 and 198).  Gather: one tet a
+// Widths, us per launch in complex128 (complex64 orders them alike).  Gather: one tet a
 // wave to 4 slots (1,680 tets x 3: 18; it reads every block by single lanes, which
 // costs more than it saves from 8: 24,708 tets 259 against 142), then row groups.
-constexpr int SCATTER_NARROW = 24, GATHER_NARROW = 4;
+constexpr int GATHER_NARROW = 4;
 
 // f(integral constant SB): the lanes' slots of a narrow batch of B
 template <typename F>
@@ -499,18 +511,36 @@ static void narrow_slots(int B, F &&f) {
 
 template <typename C>
 void launch_scatter(const MatvecArgs<C> &a, hipStream_t s) {
-    if (a.B > SCATTER_NARROW) {
+    const long long nodes = (long long)a.Nx * a.Ny * a.Nz;
+    const score::ScatterArgs<C> sa = {a.xin, a.in_off, a.B,   a.cube_start, a.S4,  a.Nx,
+                                      a.Ny,  a.Nz,     a.ncx, a.ncy,        a.ncz, a.grid_in};
+    const score::Kernel kern = score::pick_kernel(a.B, nodes);
+    if (kern == score::BLOCKS) {
         const long long nw = (long long)((a.Nx + 1) / 2) * ((a.Ny + 1) / 2) * ((a.Nz + 1) / 2) * ((a.B + 63) / 64);
         hipLaunchKernelGGL((k_scatter_blk_w64<C>), dim3(grid_for(nw, 4)), dim3(256), 0, s, a.xin, a.in_off, a.B,
                            a.cube_start, a.S4, a.Nx, a.Ny, a.Nz, a.ncx, a.ncy, a.ncz, a.grid_in);
+    } else if (kern == score::FLAT) {
+        hipLaunchKernelGGL((k_scatter_flat<C>), dim3(grid_for(nodes * a.B, score::THREADS)), dim3(score::THREADS), 0, s,
+                           sa);
     } else {
-        const score::ScatterArgs<C> sa = {a.xin, a.in_off, a.B,   a.cube_start, a.S4,  a.Nx,
-                                          a.Ny,  a.Nz,     a.ncx, a.ncy,        a.ncz, a.grid_in};
         narrow_slots(a.B, [&](auto sb) {
-            constexpr int SB = decltype(sb)::value, G = 64 / SB < 16 ? 64 / SB : 16;
-            hipLaunchKernelGGL((k_scatter_narrow<C, SB, G>),
-                               dim3(grid_for((long long)a.Nx * a.Ny * a.Nz, score::nodes_per_group<SB, G>())),
-                               dim3(score::THREADS), 0, s, sa);
+            constexpr int SB = decltype(sb)::value;
+            const int groups = score::pick_groups<SB>(nodes);
+            auto go = [&](auto gg) {
+                constexpr int G = decltype(gg)::value;
+                if constexpr (SB * G <= 64)
+                    hipLaunchKernelGGL((k_scatter_narrow<C, SB, G>),
+                                       dim3(grid_for(nodes, score::nodes_per_group<SB, G>())), dim3(score::THREADS), 0,
+                                       s, sa);
+            };
+            if (groups == 16)
+                go(std::integral_constant<int, 16>{});
+            else if (groups == 8)
+                go(std::integral_constant<int, 8>{});
+            else if (groups == 4)
+                go(std::integral_constant<int, 4>{});
+            else
+                go(std::integral_constant<int, 2>{});
         });
     }
     HIP_CHECK(hipGetLastError());

@@ -30,6 +30,38 @@ constexpr int nodes_per_group() {
     return THREADS / (SB * G);
 }
 
+// Which kernel takes a batch of B on a grid of so many nodes.  Few nodes: as many lane
+// groups as fit share each node's tets, to keep the chip busy.  Many: they only add
+// exchanges, about eight lanes to a node are best; and lanes past B idle, so that
+// one thread per (node, slot) wins for widths well below SB.  From 25 slots the
+// node blocks of 64-slot chunks.
+// us per launch in complex128 (complex64 orders them alike), by grid nodes:
+//   3 slots: 16, 8, 4, 2 groups, 99 k nodes 73, 42, 32, 33; 614 k 510, 303, 215, 205;
+//     thread per slot 47 and 233
+//   5 slots: 8, 4, 2 groups, 50 k 39, 30, 32; 149 k 120, 85, 83; 614 k 531, 372, 335;
+//     thread per slot 36, 86 and 306
+//   9 slots: 4, 2 groups, 50 k 46, 48; 149 k 141, 133; 614 k 639, 578; thread per slot
+//     41, 118 and 456
+//   12 slots: 2 groups, 149 k 140, 360 k 328, 614 k 606; thread per slot 142, 375, 565
+//   20 slots: 2 groups, 149 k 207, 614 k 942; thread per slot 200 and 840
+//   24 slots: 2 groups, 149 k 208, 360 k 508, 614 k 981; thread per slot 219, 547, 922
+//   25 slots: 64-slot chunk, 149 k 193; thread per slot 235
+enum Kernel { NARROW, FLAT, BLOCKS };
+inline Kernel pick_kernel(int B, long long nodes) {
+    if (B > 24) return BLOCKS;
+    if (nodes >= 1LL << 17 && (B == 9 || B == 10 || (B >= 17 && B <= 20))) return FLAT;
+    if (nodes >= 3LL << 17 && (B == 5 || B == 11 || B == 12 || (B >= 21 && B <= 24))) return FLAT;
+    return NARROW;
+}
+// lane groups of the narrow kernel
+template <int SB>
+inline int pick_groups(long long nodes) {
+    if (nodes < 1LL << 15 || SB == 32) return 64 / SB < 16 ? 64 / SB : 16;
+    if (SB <= 2) return 8 / SB;
+    if (SB == 4) return nodes < 1LL << 19 ? 4 : 2;
+    return nodes < 1LL << 16 ? 4 : 2;
+}
+
 // group g's share of the sums of node p, slot b
 template <typename C, int G>
 SC_HD void node_share(const ScatterArgs<C> &s, long long p, int b, int g, C *a) {

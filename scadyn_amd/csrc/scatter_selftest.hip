@@ -62,6 +62,17 @@ static void emulate(const ScatterArgs<C> &s, unsigned nwg) {
                 }
 }
 
+// one thread per (node, slot)
+template <typename C>
+static void emulate_flat(const ScatterArgs<C> &s) {
+    for (long long p = 0; p < (long long)s.Nx * s.Ny * s.Nz; ++p)
+        for (int b = 0; b < s.B; ++b) {
+            C a[4];
+            node_share<C, 1>(s, p, b, 0, a);
+            write_node(s, p, b, a);
+        }
+}
+
 template <typename C>
 static double error(const Data<C> &d) {
     const ScatterArgs<C> &s = d.a;
@@ -109,6 +120,32 @@ static void one(int B, std::mt19937_64 &rng) {
         }
     }
 }
+template <typename C>
+static void flat(int B, std::mt19937_64 &rng) {
+    Data<C> d;
+    make(d, 3, 2, 4, B, rng);
+    emulate_flat(d.a);
+    ++cases;
+    const double e = error(d);
+    if (!(e < (sizeof(C) == 16 ? 1e-14 : 2e-6))) {
+        ++failures;
+        std::printf("%s B=%d, thread per slot: rel.err %.2e\n", sizeof(C) == 16 ? "c128" : "c64", B, e);
+    }
+}
+
+// the rule's groups fit a wave, and its kernels are those compiled
+template <int SB>
+static void picks() {
+    for (long long nodes = 1; nodes < 1LL << 40; nodes = nodes * 3 / 2 + 1) {
+        const int g = pick_groups<SB>(nodes);
+        ++cases;
+        if (SB * g > 64 || (g != 2 && g != 4 && g != 8 && g != 16)) {
+            ++failures;
+            std::printf("SB=%d, %lld nodes: %d groups\n", SB, nodes, g);
+        }
+    }
+}
+
 template <int SB, int G>
 static void both(int B, std::mt19937_64 &rng) {
     one<cd, SB, G>(B, rng);
@@ -137,6 +174,8 @@ int main() {
     for (int B : {5, 8}) both<8, 8>(B, rng), both<8, 4>(B, rng), both<8, 2>(B, rng);
     for (int B : {9, 16}) both<16, 4>(B, rng), both<16, 2>(B, rng);
     for (int B : {17, 24}) both<32, 2>(B, rng);
+    for (int B : {5, 12, 24}) flat<cd>(B, rng), flat<cf>(B, rng);
+    picks<1>(), picks<2>(), picks<4>(), picks<8>(), picks<16>(), picks<32>();
     for (long long nodes : {1LL, 15LL, 17LL, (1LL << 26) - 1, (1LL << 26) + 1, 1LL << 28, (1LL << 28) + 5, 1LL << 33})
         for (int per : {4, 8, 16, 32}) launch(nodes, per);
     std::printf("%d cases, %d failures\n", cases, failures);
