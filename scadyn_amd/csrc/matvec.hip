@@ -131,6 +131,73 @@ __global__ __launch_bounds__(256) void k_gather_narrow(
     }
 }
 
+// the same with one thread per (row, slot), the row's terms in order
+template <typename C>
+__global__ __launch_bounds__(256) void k_gather_flat(
+    const C *__restrict__ grid, const C *__restrict__ xin, const long long *__restrict__ in_off, int B,
+    int N, const int *__restrict__ tet_cube, const C *__restrict__ S4, int Nx, int Ny, int ncx, int ncy,
+    const int64_t *__restrict__ row_start, const int *__restrict__ ent_col,
+    const uint32_t *__restrict__ ent_blk, const cf *__restrict__ blocks, double k2,
+    const int *__restrict__ slot_active, cd *__restrict__ y) {
+    const long long tot = (long long)N * B;
+    for (long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x; e < tot;
+         e += (long long)gridDim.x * blockDim.x) {
+        const int b = (int)(e % B);
+        const int t = (int)(e / B);
+        cd *yo = y + (size_t)(3 * t) * B + b;
+        if (slot_active && !slot_active[b]) continue;  // inactive slots are not written
+        const int c = tet_cube[t];
+        const int cx = c % ncx, cy = (c / ncx) % ncy, cz = c / (ncx * ncy);
+        const size_t base = (size_t)(2 * cx) + (size_t)Nx * ((size_t)(2 * cy) + (size_t)Ny * (2 * cz));
+        const C *s = S4 + (size_t)t * 108;
+        C Y0 = Prec<C>::zero(), Y1 = Y0, Y2 = Y0, Z0 = Y0, Z1 = Y0, Z2 = Y0;
+        for (int jz = 0; jz < 3; ++jz)
+            for (int jy = 0; jy < 3; ++jy)
+                for (int jx = 0; jx < 3; ++jx) {
+                    const int j = jx + 3 * jy + 9 * jz;
+                    const size_t node = base + jx + (size_t)Nx * (jy + (size_t)Ny * jz);
+                    const C *g = grid + node * 4 * B + b;
+                    const C g0 = g[0], g1 = g[(size_t)B], g2 = g[(size_t)2 * B], g3 = g[(size_t)3 * B];
+                    const C *sj = s + j * 4;
+                    cfma(Y0, sj[0], g0);
+                    cfma(Y1, sj[0], g1);
+                    cfma(Y2, sj[0], g2);
+                    cfma(Z0, sj[1], g3);
+                    cfma(Z1, sj[2], g3);
+                    cfma(Z2, sj[3], g3);
+                }
+        // near zone
+        const C *xb = xin + in_off[b] + b;
+        C n0 = Prec<C>::zero(), n1 = n0, n2 = n0;
+        for (int64_t q = row_start[t]; q < row_start[t + 1]; ++q) {
+            const int col = ent_col[q];
+            const uint32_t eb = ent_blk[q];
+            const cf *a = blocks + (size_t)(eb & 0x7fffffffu) * 9;
+            const C x0 = Prec<C>::from(xb[(size_t)(3 * col) * B]),
+                    x1 = Prec<C>::from(xb[(size_t)(3 * col + 1) * B]),
+                    x2 = Prec<C>::from(xb[(size_t)(3 * col + 2) * B]);
+            C m[9];
+#pragma unroll
+            for (int i = 0; i < 9; ++i) m[i] = Prec<C>::from(a[i]);
+            if (eb & 0x80000000u) {
+                // transpose: y_i += sum_j A(j,i) x_j ; A(i,j) at i + 3j
+                cfma(n0, m[0], x0); cfma(n0, m[1], x1); cfma(n0, m[2], x2);
+                cfma(n1, m[3], x0); cfma(n1, m[4], x1); cfma(n1, m[5], x2);
+                cfma(n2, m[6], x0); cfma(n2, m[7], x1); cfma(n2, m[8], x2);
+            } else {
+                cfma(n0, m[0], x0); cfma(n0, m[3], x1); cfma(n0, m[6], x2);
+                cfma(n1, m[1], x0); cfma(n1, m[4], x1); cfma(n1, m[7], x2);
+                cfma(n2, m[2], x0); cfma(n2, m[5], x1); cfma(n2, m[8], x2);
+            }
+        }
+        typedef typename Prec<C>::real R;
+        const R kk = (R)k2;
+        yo[0] = Prec<cd>::from(cadd(n0, csub(Z0, cscale(Y0, kk))));
+        yo[(size_t)B] = Prec<cd>::from(cadd(n1, csub(Z1, cscale(Y1, kk))));
+        yo[(size_t)2 * B] = Prec<cd>::from(cadd(n2, csub(Z2, cscale(Y2, kk))));
+    }
+}
+
 // ---- on-chip reuse variants (slots in chunks of 64) --------------------------
 // Scatter, one wave per 2x2x2 block of grid nodes (2a..2a+1, 2b..2b+1, 2c..2c+1),
 // ceil(N/2) blocks per axis:
@@ -312,7 +379,7 @@ __global__ __launch_bounds__(64, 3) void k_gather_lds(gcore::GatherArgs<C> g) {
     }
 }
 
-// complex128, 5 to 32 slots: three rows at a time, the columns shared by the lane
+// complex128, up to 32 slots (up to 4 on large meshes): three rows at a time, the columns shared by the lane
 // groups (24,708 tets x 7: 153 us against 231 with the rows shared; complex64 keeps
 // the order of its sums)
 template <typename C, int NT, int VC, int SB>
@@ -487,10 +554,25 @@ __global__ __launch_bounds__(64, 3) void k_gather_mf(gcore::GatherArgs<cf> g) {
     }
 }
 
-// Widths, us per launch in complex128 (complex64 orders them alike).  Gather: one tet a
-// wave to 4 slots (1,680 tets x 3: 18; it reads every block by single lanes, which
-// costs more than it saves from 8: 24,708 tets 259 against 142), then row groups.
-constexpr int GATHER_NARROW = 4;
+// Gather kernels by width and mesh, us per launch at N tets.
+//  * One tet a wave to 4 slots: it reads every block by single lanes, which costs more
+//    than it saves once the chip is full, so in complex128 only on small meshes
+//    (1,680 tets x 3: 17 us against 30 with k_gather_cols; 12.7 k 74 and 62; 201 k
+//    1,415 and 911; thread per slot 155, 161, 1,360).  Complex64 keeps it: another
+//    order of its sums can move a mixed solve's iteration counts.
+//  * Complex64 of 5 to 8 slots: row groups leave lanes idle (six of eight lane groups
+//    have a row, and five of eight lanes a slot); on large meshes one thread per slot
+//    is faster (5 slots: 24.7 k 179 us in groups, 179 by threads; 98 k 814 and 728;
+//    201 k 1,536 and 1,357; 8 slots: 98 k 825 and 815; 201 k 1,557 and 1,498).
+//  * Else row groups.
+enum GatherKernel { GATHER_NARROW, GATHER_FLAT, GATHER_GROUPS };
+template <typename C>
+static GatherKernel pick_gather(int B, int N) {
+    const bool wide = sizeof(C) == 16;
+    if (B <= 4) return wide && N >= 8192 ? GATHER_GROUPS : GATHER_NARROW;
+    if (!wide && B <= 8 && N >= (B <= 6 ? 1 << 16 : 3 << 16)) return GATHER_FLAT;
+    return GATHER_GROUPS;
+}
 
 // f(integral constant SB): the lanes' slots of a narrow batch of B
 template <typename F>
@@ -548,10 +630,11 @@ void launch_scatter(const MatvecArgs<C> &a, hipStream_t s) {
 
 template <typename C>
 void launch_gather_near(const MatvecArgs<C> &a, hipStream_t s) {
-    if (a.B <= GATHER_NARROW) {
+    const GatherKernel kern = pick_gather<C>(a.B, a.N);
+    if (kern == GATHER_NARROW) {
         narrow_slots(a.B, [&](auto sb) {
             constexpr int SB = decltype(sb)::value;
-            if constexpr (SB <= GATHER_NARROW)
+            if constexpr (SB <= 4)
                 hipLaunchKernelGGL((k_gather_narrow<C, SB>), dim3((unsigned)((a.N + 3) / 4)), dim3(256), 0, s,
                                    a.grid_out, a.xin, a.in_off, a.B, a.N, a.tet_cube, a.S4, a.Nx, a.Ny, a.ncx, a.ncy,
                                    a.row_start, a.ent_col, a.ent_blk, a.blocks, a.k2, a.slot_active, a.y);
@@ -559,6 +642,14 @@ void launch_gather_near(const MatvecArgs<C> &a, hipStream_t s) {
         HIP_CHECK(hipGetLastError());
         return;
     }
+    if constexpr (std::is_same<C, cf>::value)
+        if (kern == GATHER_FLAT) {
+            hipLaunchKernelGGL((k_gather_flat<C>), dim3(grid_for((long long)a.N * a.B, 256)), dim3(256), 0, s,
+                               a.grid_out, a.xin, a.in_off, a.B, a.N, a.tet_cube, a.S4, a.Nx, a.Ny, a.ncx, a.ncy,
+                               a.row_start, a.ent_col, a.ent_blk, a.blocks, a.k2, a.slot_active, a.y);
+            HIP_CHECK(hipGetLastError());
+            return;
+        }
     gcore::GatherArgs<C> g = {a.grid_out, a.xin,     a.in_off,    a.B,      a.ne_cubes,
                                     a.n_ne,     a.cube_start, a.S4,      a.Nx,     a.Ny,
                                     a.ncx,      a.ncy,       a.ncz,       a.row_start, a.ent_blk,
@@ -584,8 +675,12 @@ void launch_gather_near(const MatvecArgs<C> &a, hipStream_t s) {
                 cols(std::integral_constant<int, 32>{});
             else if (a.B > 8)
                 cols(std::integral_constant<int, 16>{});
-            else
+            else if (a.B > 4)
                 cols(std::integral_constant<int, 8>{});
+            else if (a.B > 2)
+                cols(std::integral_constant<int, 4>{});
+            else
+                cols(std::integral_constant<int, 2>{});
             HIP_CHECK(hipGetLastError());
             return;
         }

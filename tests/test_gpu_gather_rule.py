@@ -1,0 +1,29 @@
+"""The gather's rule on width and mesh: batches of 1 to 9 vectors on meshes of 6.7
+thousand to 0.2 million tets, on both sides of each line of the rule, against other
+kernels of the same sums: complex128 against the vectors in a batch of 33, 1e-13;
+complex64 against complex64 in that batch, 2e-6, as the other widths."""
+import numpy as np
+import pytest
+
+from helpers import rel, sphere_case
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize('n_cells,lo,hi', [(12, 4096, 8192), (14, 8192, 1 << 16), (30, 1 << 16, 3 << 16),
+                                           (40, 3 << 16, 1 << 18)])
+def test_gather_widths(n_cells, lo, hi):
+    from scadyn_amd import native
+    c, e, param, k = sphere_case(n_cells=n_cells)
+    assert lo <= e.shape[0] < hi
+    print(f'[gather-rule] {e.shape[0]} tets', flush=True)
+    a = native.Operator(c, e, param, k, precision=native.PREC_MIXED)
+    x = np.random.default_rng(6).standard_normal((2, 33, 3 * e.shape[0]))
+    x = x[0] + 1j * x[1]
+    for prec, tol in ((native.PREC_FP64, 1e-13), (native.PREC_MIXED, 2e-6)):
+        ref = a.matvec(x, precision=prec)
+        for wide in (1, 2, 3, 4, 5, 6, 7, 8, 9):
+            y = a.matvec(x[:wide], precision=prec)
+            for r in range(wide):
+                assert rel(y[r], ref[r]) < tol
+    a.close()
