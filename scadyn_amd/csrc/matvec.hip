@@ -657,7 +657,8 @@ void launch_gather_near(const MatvecArgs<C> &a, hipStream_t s) {
     g.groups = a.groups;
     g.n_groups = a.n_groups;
     if constexpr (std::is_same<C, cf>::value) {
-        if (a.gather_kernel == 1) {
+        // half full chunks at least: it costs the same for 8 slots as for 64
+        if (a.gather_kernel == 1 && (a.B % 64 == 0 || a.B % 64 >= 32)) {
             hipLaunchKernelGGL((k_gather_mf<gcore::GATHER_GT, gcore::GATHER_VC>), dim3(grid_for((long long)a.n_ne * ((a.B + 63) / 64), 1)),
                                dim3(64), 0, s, g);
             HIP_CHECK(hipGetLastError());

@@ -27,3 +27,19 @@ def test_gather_widths(n_cells, lo, hi):
             for r in range(wide):
                 assert rel(y[r], ref[r]) < tol
     a.close()
+
+
+@pytest.mark.parametrize('wide', [8, 31, 70])
+def test_matrix_core_gather_needs_half_a_chunk(wide):
+    """gather_kernel = 1 on widths whose last 64-slot chunk is less than half full: the
+    vector kernel, hence its bits."""
+    from scadyn_amd import native
+    c, e, param, k = sphere_case(n_cells=8)
+    print(f'[gather-rule] matrix cores, {wide} vectors', flush=True)
+    a = native.Operator(c, e, param, k, precision=native.PREC_MIXED)
+    b = native.Operator(c, e, param, k, precision=native.PREC_MIXED, gather_kernel=1)
+    x = np.random.default_rng(8).standard_normal((2, wide, 3 * e.shape[0]))
+    x = x[0] + 1j * x[1]
+    assert np.array_equal(a.matvec(x, precision=native.PREC_MIXED), b.matvec(x, precision=native.PREC_MIXED))
+    a.close()
+    b.close()
