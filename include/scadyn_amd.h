@@ -98,7 +98,8 @@ typedef struct scadyn_opts {
                             2 + 2/mgs_block vectors of HBM traffic per coefficient      */
     int32_t gather_kernel; /* complex64 gather + near zone: 0 vector FMA (default), 1 the near-zone
                               product on the matrix cores (v_mfma_f32_16x16x4f32; batches whose last
-                              64-slot chunk is at least half full; measured about 2x slower, its operand set-up costs as much as the FMAs it replaces) */
+                              64-slot chunk is at least half full; measured about 2x slower, its
+                              operand set-up costs as much as the FMAs it replaces) */
     int32_t basis;       /* mixed precision with the blocked MGS (ortho 0, mgs_block > 1):
                             storage of the Krylov basis.  SCADYN_BASIS_AUTO (binary16 for
                             systems of 2^20 to 2^26 rows, else complex64),

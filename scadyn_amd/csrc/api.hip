@@ -540,25 +540,14 @@ static void make_matvec_space(scadyn_operator *op, int B, MatvecSpace &ms) {
     ms.grid1 = ms.mem.alloc<cd>(gsz);
     ms.in_off = ms.mem.alloc<long long>(B);
     ms.active = ms.mem.alloc<int>(B);
-    // Tile widths of the register kernel.  Transforms: 256 bytes of columns (16
-    // complex128, 32 complex64), half where that takes more than 64 KiB of LDS.
-    // Convolutions: 16 columns, 8 beyond 48 KiB; they are bound by instructions
-    // and latency, not by the width of their accesses, and more workgroups fit.
-    // Measured over lengths 24 to 270 and batches 3 to 64, widths 4 to 32: the rule
-    // is within 3% of the fastest width (convolution of 210 points, 64 slots,
-    // complex128: 8 columns 10.9 ms, 16 11.8; of 160 points 8 5.2, 16 4.6;
-    // complex64, 160 points: 16 2.7, 32 2.6; 105 points: 16 0.78, 32 0.85).
-    // Timing every width on the batch's own grids, as was done before, cost 45 ms of
-    // a 225 ms bar (43,248 tets, FP64).
-    const size_t budget = 64 * 1024, conv_budget = 48 * 1024;
     const bool reg = op->opts.fft_kernel == 0;
     for (int pr = 0; pr < 2; ++pr) {
         const size_t el = pr == 0 ? sizeof(cd) : sizeof(cf);
-        make_line_pass(ms.pass[pr][0], Lx, Nx, Lx, nb, (long long)Ny * Nz, budget, el, reg);
-        make_line_pass(ms.pass[pr][1], Ly, Ny, Ly, (long long)Lx * nb, Nz, budget, el, reg);
-        make_line_pass(ms.pass[pr][2], Lz, Nz, Nz, (long long)Ly * Lx * nb, 1, conv_budget, el, reg, 16);
-        make_line_pass(ms.pass[pr][3], Ly, Ly, Ny, (long long)Lx * nb, Nz, budget, el, reg);
-        make_line_pass(ms.pass[pr][4], Lx, Lx, Nx, nb, (long long)Ny * Nz, budget, el, reg);
+        plan_transform(ms.pass[pr][0], Lx, Nx, Lx, nb, (long long)Ny * Nz, el, reg);
+        plan_transform(ms.pass[pr][1], Ly, Ny, Ly, (long long)Lx * nb, Nz, el, reg);
+        plan_conv(ms.pass[pr][2], Lz, Nz, (long long)Ly * Lx * nb, el, reg);
+        plan_transform(ms.pass[pr][3], Ly, Ly, Ny, (long long)Lx * nb, Nz, el, reg);
+        plan_transform(ms.pass[pr][4], Lx, Lx, Nx, nb, (long long)Ny * Nz, el, reg);
     }
 }
 

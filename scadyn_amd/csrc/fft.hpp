@@ -44,9 +44,14 @@ struct ConvInfo {
 };
 
 // allow_reg: use the two-stage register kernel when L = R1 R2 with both
-// radices in the register set; want: its tile width (0: 256 bytes of columns)
+// radices in the register set; want: its tile width (0: 256 bytes of columns), soft:
+// LDS bytes beyond which it is narrowed (fft.hip)
 void make_line_pass(LinePass &p, int L, int n_in, int n_out, long long inner, long long outer, size_t lds_budget,
-                    size_t elem, bool allow_reg = true, int want = 0);
+                    size_t elem, bool allow_reg = true, int want = 0, size_t soft = 0);
+// the matvec's passes: a transform, and the fused z convolution of n points padded to L
+void plan_transform(LinePass &p, int L, int n_in, int n_out, long long inner, long long outer, size_t elem,
+                    bool allow_reg);
+void plan_conv(LinePass &p, int L, int n, long long inner, size_t elem, bool allow_reg);
 bool reg_radix_ok(int r);
 template <typename C>
 void launch_line_reg(const LinePass &p, const C *in, C *out, const C *tw, int sign, const C *fg, const ConvInfo &ci,

@@ -104,17 +104,35 @@ static void planned(int L, long long inner, std::mt19937_64 &rng) {
     for (int sign = -1; sign <= 1; sign += 2) {
         const int n_in = sign < 0 ? L / 2 + 1 : L, n_out = sign < 0 ? L : L / 2 + 1;
         LinePass p;
-        make_line_pass(p, L, n_in, n_out, inner, 2, 64 * 1024, sizeof(C), true);
+        plan_transform(p, L, n_in, n_out, inner, 2, sizeof(C), true);
         const int sh = reg_shift(p, ConvInfo(), 0, sizeof(C));
         std::vector<C> in((size_t)2 * n_in * inner), a((size_t)2 * n_out * inner), b(a.size());
         fill(in, rng);
         run<0, C>(sh, p, in.data(), a.data(), tw.data(), sign, nullptr, ConvInfo());
         run<0, C>(-1, p, in.data(), b.data(), tw.data(), sign, nullptr, ConvInfo());
         same_bits(sign < 0 ? "fwd" : "inv", p, sh, a, b);
+        // and the widest tiles against the definition
+        if (inner < 64) continue;
+        std::vector<cl> w(L);
+        for (int q = 0; q < L; ++q) w[q] = std::polar(1.0L, sign * 2.0L * PI_L * q / L);
+        long double num = 0, den = 0;
+        for (int c = 0; c < inner; c += 7)
+            for (int k = 0; k < n_out; ++k) {
+                cl r = 0;
+                for (int n = 0; n < n_in; ++n) r += cl(in[(size_t)n * inner + c].x, in[(size_t)n * inner + c].y) * w[(n * k) % L];
+                const C o = a[(size_t)k * inner + c];
+                num += std::norm(cl(o.x, o.y) - r);
+                den += std::norm(r);
+            }
+        ++cases;
+        if (!(std::sqrt(num / den) < (sizeof(C) == 16 ? 1e-14 : 2e-6))) {
+            ++failures;
+            std::printf("%d points, %d columns: rel.err %.2Le\n", L, p.ti, std::sqrt(num / den));
+        }
     }
     const int Nz = L / 2;
     LinePass p;
-    make_line_pass(p, L, Nz, Nz, inner, 1, 48 * 1024, sizeof(C), true, 16);
+    plan_conv(p, L, Nz, inner, sizeof(C), true);
     ConvInfo ci;
     ci.Lx = (int)inner, ci.Ly = 1, ci.Lz = L, ci.Hx = (int)inner / 2 + 1, ci.Hy = 1, ci.nb = 1;
     const int sh = reg_shift(p, ci, 1, sizeof(C));
@@ -126,6 +144,41 @@ static void planned(int L, long long inner, std::mt19937_64 &rng) {
     same_bits("conv", p, sh, a, b);
 }
 
+// the planner's widths: {length, columns, complex128 transform, complex64 transform,
+// complex128 convolution, complex64 convolution}
+static void widths() {
+    const int want[][6] = {
+        {105, 1 << 20, 16, 32, 16, 16}, {160, 1 << 20, 16, 32, 16, 16}, {168, 1 << 20, 16, 32, 16, 16},
+        {210, 1 << 20, 16, 32, 8, 16},  // 16 columns of complex128 exceed 48 KiB
+        {270, 1 << 20, 8, 16, 8, 16},   // and here 64 KiB, as do 32 of complex64
+        {360, 1 << 20, 8, 16, 8, 16},  {400, 1 << 20, 8, 16, 8, 16},  // not below 128 bytes
+        {20, 1 << 20, 32, 32, 32, 32}, {75, 1 << 20, 32, 32, 32, 32}, // five thread rows: twice as wide
+        {20, 16, 16, 16, 16, 16},                                     // the inner extent bounds it
+        {168, 4, 4, 4, 4, 4},          {168, 8, 8, 8, 8, 8},
+        {168, 12, 4, 8, 4, 8},         {168, 20, 8, 8, 8, 8}, // a quarter of the columns beyond the extent
+        {168, 48, 16, 16, 16, 16},     {168, 36, 16, 16, 16, 16}, {168, 28, 16, 16, 16, 16}};
+    for (auto &q : want) {
+        LinePass p[4];
+        plan_transform(p[0], q[0], q[0] / 2, q[0], q[1], 3, 16, true);
+        plan_transform(p[1], q[0], q[0] / 2, q[0], q[1], 3, 8, true);
+        plan_conv(p[2], q[0], q[0] / 2, q[1], 16, true);
+        plan_conv(p[3], q[0], q[0] / 2, q[1], 8, true);
+        for (int i = 0; i < 4; ++i) {
+            ++cases;
+            if (p[i].ti != q[2 + i] || !p[i].reg || line_pass_lds(p[i], i % 2 ? 8 : 16) > 64 * 1024 ||
+                p[i].threads > reg_max_threads(i % 2 ? 8 : 16)) {
+                ++failures;
+                std::printf("%d points, %d columns, plan %d: %d columns a tile, not %d\n", q[0], q[1], i, p[i].ti, q[2 + i]);
+            }
+        }
+        // the Stockham kernel: two buffers of 64 columns at most in 64 KiB, transform and convolution alike
+        plan_transform(p[0], q[0], q[0] / 2, q[0], q[1], 1, 16, false);
+        plan_conv(p[2], q[0], q[0] / 2, q[1], 16, false);
+        ++cases;
+        if (p[0].ti != p[2].ti || p[0].reg || p[2].reg) ++failures, std::printf("%d points: Stockham widths %d, %d\n", q[0], p[0].ti, p[2].ti);
+    }
+}
+
 // The tile of the columns around (Lx / 2, Ly / 2), the octant's last row, of a grid
 // Lx x Ly x Lz.  16 columns, 4 to a grid point.
 template <typename C>
@@ -133,7 +186,7 @@ static void wide(int Lx, int Ly, int Lz, std::mt19937_64 &rng, double tol) {
     const int Nz = Lz / 2, nb = 4;
     const long long inner = 16;
     LinePass p;
-    make_line_pass(p, Lz, Nz, Nz, inner, 1, 64 * 1024, sizeof(C), true, 16);
+    plan_conv(p, Lz, Nz, inner, sizeof(C), true);
     ConvInfo ci;
     ci.Lx = Lx, ci.Ly = Ly, ci.Lz = Lz, ci.Hx = Lx / 2 + 1, ci.Hy = Ly / 2 + 1, ci.nb = nb;
     const size_t zs = (size_t)ci.Hx * ci.Hy, bytes = zs * (Lz / 2 + 1) * sizeof(C);
@@ -190,6 +243,7 @@ static void wide(int Lx, int Ly, int Lz, std::mt19937_64 &rng, double tol) {
 
 int main() {
     std::mt19937_64 rng(77);
+    widths();
     for (int L : {20, 24, 35, 75, 90, 105, 112, 160, 168, 210, 270, 360, 400})
         for (long long inner : {4, 12, 16, 20, 33, 64}) {
             planned<cd>(L, inner, rng);

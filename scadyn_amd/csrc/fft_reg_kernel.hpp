@@ -21,7 +21,10 @@ __device__ inline void wave_base(size_t &base, unsigned &lane) {
     base = b;
 }
 
-// SH: log2 of the tile width, with 32-bit lane offsets; -1: any width, 64-bit addresses
+// SH: log2 of the tile width, with 32-bit lane offsets; -1: any width, 64-bit addresses.
+// RMAX, the largest radix compiled in, sets the registers and so the waves per SIMD, of
+// the any-width instance too: narrow batches run it on the x passes (105 points, 1
+// vector, complex128: 18 us with radices up to 20 compiled in, 13 with up to 16)
 template <int MODE, typename C, int RMAX, int SH>
 __global__ __launch_bounds__(sizeof(C) <= 8 ? 1024 : 512) void k_line_reg(const C *__restrict__ in,
                                                                           C *__restrict__ out, LinePass p,
@@ -53,17 +56,13 @@ __global__ __launch_bounds__(sizeof(C) <= 8 ? 1024 : 512) void k_line_reg(const 
 template <int MODE, typename C, int SH>
 static void launch_sh(int rm, dim3 grid, dim3 block, size_t lds, hipStream_t s, const C *in, C *out,
                       const LinePass &p, const C *tw, int sign, const C *fg, const ConvInfo &ci) {
-    if constexpr (SH < 0) {
-        hipLaunchKernelGGL((k_line_reg<MODE, C, 20, SH>), grid, block, lds, s, in, out, p, tw, sign, fg, ci);
-    } else {
-        switch (rm) {
-#define INST(R)                                                                                                  \
-    case R:                                                                                                      \
-        hipLaunchKernelGGL((k_line_reg<MODE, C, R, SH>), grid, block, lds, s, in, out, p, tw, sign, fg, ci);     \
+    switch (rm) {
+#define INST(R)                                                                                              \
+    case R:                                                                                                  \
+        hipLaunchKernelGGL((k_line_reg<MODE, C, R, SH>), grid, block, lds, s, in, out, p, tw, sign, fg, ci); \
         break;
-            INST(12) INST(14) INST(16) INST(18) INST(20)
+        INST(12) INST(14) INST(16) INST(18) INST(20)
 #undef INST
-        }
     }
 }
 

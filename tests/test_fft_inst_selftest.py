@@ -1,7 +1,8 @@
 """The compiled instances of the register line FFT (fixed tile width, 32-bit lane
 offsets), run on the CPU (host build with AddressSanitizer) as the launcher picks
 them: bit for bit against the 64-bit instance, and the fused convolution with
-octants of FFT(G) around and beyond 2 and 4 GiB against a direct long-double DFT.
+octants of FFT(G) around and beyond 2 and 4 GiB against a direct long-double DFT;
+and the planner's tile widths.
 
 Tolerances (relative Frobenius): 1e-14 complex128, 2e-6 complex64, as for the
 stages themselves."""
