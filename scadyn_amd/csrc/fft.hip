@@ -268,14 +268,16 @@ size_t line_pass_lds(const LinePass &p, size_t elem) {
 
 // Register-kernel tile width: the largest power of two <= want that fits the inner
 // extent, the LDS budget and the kernel's thread bound; narrower beyond soft bytes of
-// LDS (0: none) where that keeps 128 bytes of columns.  Then
+// LDS (0: none), down to 8 columns.  Then
 //  * twice as wide where more than a quarter of its threads have no point (five
 //    thread rows of 16 columns are 80 of 128): transforms of 20 points, 24 vectors,
-//    complex128 284 us with 16 columns, 242 with 32; convolution of 20 points,
-//    complex64 1,081 and 907, of 75 points, 64 vectors 540 and 487;
+//    complex128 286 us with 16 columns, 244 with 32; convolution of 20 points,
+//    complex64 1,112 and 941, of 75 points, 64 vectors, complex128 1,084 and 907;
 //  * half as wide where a quarter of its columns lie beyond the inner extent, down to
-//    64 bytes: 168 points, 5 vectors (20 columns) complex128 133 us with 16, 116 with
-//    8; 3 vectors (12) 84 with 8, 74 with 4.
+//    4 complex128 or 16 complex64 columns: 168 points, 5 vectors (20 columns),
+//    complex128 137 us with 16, 106 with 8; 3 vectors (12) 83 with 8, 74 with 4;
+//    complex64, 5 vectors 68 with 16 and 77 with 8, 12 vectors (48) 124 with 32, 110
+//    with 16.
 static int reg_tile(int L, int rows, long long inner, size_t lds_budget, size_t elem, int want, size_t soft) {
     auto lds = [&](int ti) { return elem * ((size_t)L + (size_t)L * ti); };
     auto fits = [&](int ti, size_t budget) {
@@ -285,9 +287,10 @@ static int reg_tile(int L, int rows, long long inner, size_t lds_budget, size_t 
     int ti = want;
     while (ti > 1 && !fits(ti, lds_budget)) ti /= 2;
     if (soft)
-        while (ti * elem > 128 && lds(ti) > soft) ti /= 2;
+        while (ti > 8 && lds(ti) > soft) ti /= 2;
     if (4 * ti * rows < 3 * ((ti * rows + 63) / 64 * 64) && fits(2 * ti, soft ? soft : lds_budget)) ti *= 2;
-    while (ti * elem > 64 && 3 * padded(ti) >= 4 * padded(ti / 2)) ti /= 2;
+    const int least = elem >= 16 ? 4 : 16;
+    while (ti > least && 3 * padded(ti) >= 4 * padded(ti / 2)) ti /= 2;
     return ti;
 }
 
@@ -340,11 +343,11 @@ void make_line_pass(LinePass &p, int L, int n_in, int n_out, long long inner, lo
 
 // Tile widths of the register kernel.  Transforms: 256 bytes of columns (16
 // complex128, 32 complex64), half where that takes more than 64 KiB of LDS.
-// Convolutions: 16 columns, fewer beyond 48 KiB but not below 128 bytes; they are
-// bound by instructions and latency, not by the width of their accesses, and more
-// workgroups fit (210 points, 64 vectors, complex128: 8 columns 10.9 ms, 16 11.8; 160
-// points 8 5.2, 16 4.6; complex64, 160 points: 16 2.7, 32 2.6; 105 points: 16 0.78, 32
-// 0.85; 360 points complex128: 4 0.83, 8 0.76).  Timing every width on the batch's
+// Convolutions: 16 columns, 8 beyond 48 KiB; they are bound by instructions and
+// latency, not by the width of their accesses, and more workgroups fit (210 points,
+// 64 vectors, complex128: 8 columns 10.9 ms, 16 11.8; 160 points 8 5.2, 16 4.6; 360
+// points 4 0.83, 8 0.76; complex64, 160 points: 16 2.7, 32 2.6; 105 points: 16 0.78,
+// 32 0.85; 400 points: 8 0.38, 16 0.41).  Timing every width on the batch's
 // own grids instead cost 45 ms of a 225 ms bar (43,248 tets, FP64).
 constexpr size_t LDS_BYTES = 64 * 1024, CONV_LDS_BYTES = 48 * 1024;
 constexpr int CONV_COLUMNS = 16;

@@ -151,11 +151,11 @@ static void widths() {
         {105, 1 << 20, 16, 32, 16, 16}, {160, 1 << 20, 16, 32, 16, 16}, {168, 1 << 20, 16, 32, 16, 16},
         {210, 1 << 20, 16, 32, 8, 16},  // 16 columns of complex128 exceed 48 KiB
         {270, 1 << 20, 8, 16, 8, 16},   // and here 64 KiB, as do 32 of complex64
-        {360, 1 << 20, 8, 16, 8, 16},  {400, 1 << 20, 8, 16, 8, 16},  // not below 128 bytes
+        {360, 1 << 20, 8, 16, 8, 16},  {400, 1 << 20, 8, 16, 8, 8},   // not below 8 columns
         {20, 1 << 20, 32, 32, 32, 32}, {75, 1 << 20, 32, 32, 32, 32}, // five thread rows: twice as wide
         {20, 16, 16, 16, 16, 16},                                     // the inner extent bounds it
         {168, 4, 4, 4, 4, 4},          {168, 8, 8, 8, 8, 8},
-        {168, 12, 4, 8, 4, 8},         {168, 20, 8, 8, 8, 8}, // a quarter of the columns beyond the extent
+        {168, 12, 4, 8, 4, 8},         {168, 20, 8, 16, 8, 16}, // a quarter of the columns beyond the extent
         {168, 48, 16, 16, 16, 16},     {168, 36, 16, 16, 16, 16}, {168, 28, 16, 16, 16, 16}};
     for (auto &q : want) {
         LinePass p[4];
