@@ -105,6 +105,7 @@ SELFTESTS = {'fft': ('fft_selftest.hip', SELFTEST), 'bmgs': ('bmgs_selftest.hip'
              'gather': ('gather_selftest.hip', os.path.join(OBJDIR, 'gather_selftest')),
              'mgsb': ('mgsb_selftest.hip', os.path.join(OBJDIR, 'mgsb_selftest')),
              'fft_inst': ('fft_inst_selftest.hip', os.path.join(OBJDIR, 'fft_inst_selftest')),
+             'gather_rows': ('gather_rows_selftest.hip', os.path.join(OBJDIR, 'gather_rows_selftest')),
              'scatter': ('scatter_selftest.hip', os.path.join(OBJDIR, 'scatter_selftest')),
              'pairs': ('pairs_selftest.hip', os.path.join(OBJDIR, 'pairs_selftest')),
              'pinv': ('pinv_selftest.hip', os.path.join(OBJDIR, 'pinv_selftest'))}
@@ -113,10 +114,11 @@ SELFTESTS = {'fft': ('fft_selftest.hip', SELFTEST), 'bmgs': ('bmgs_selftest.hip'
 def build_selftest(verbose=False, which='fft'):
     """Host self-tests of kernel code (CPU only, AddressSanitizer on the host
     code): 'fft' the register FFT stages (links the library for the pass
-    planner), 'fft_inst' its compiled instances at the planner's widths, 'bmgs' the block
-    Gram-Schmidt bodies, 'scatter' the narrow scatter, 'pairs' the near-zone pair and
-    row lists, 'gather' the LDS-staged
-    per-cube gather, 'pinv' the pseudo-inverse (from the library)."""
+    planner), 'fft_inst' its compiled instances at the planner's widths, 'bmgs'
+    and 'mgsb' the block Gram-Schmidt bodies, 'scatter' the narrow scatter,
+    'pairs' the near-zone pair and row lists, 'gather' the gather's staging and
+    its matrix-core pass, 'gather_rows' its row-group kernels, 'pinv' the
+    pseudo-inverse (from the library)."""
     hipcc = os.environ.get('HIPCC', '/opt/rocm/bin/hipcc')
     os.makedirs(OBJDIR, exist_ok=True)
     src, exe = SELFTESTS[which]

@@ -425,13 +425,7 @@ static void create_operator(scadyn_operator *op, const scadyn_mesh &mesh, const 
         for (const auto &kc : key) ne.push_back(kc.second);
         op->n_ne_cubes = (int)ne.size();
         std::vector<int2> groups;
-        for (int c : ne) {
-            const int t0 = g.cube_start[c], n = g.cube_start[c + 1] - t0, k = (n + gcore::ROW_GT - 1) / gcore::ROW_GT;
-            for (int q = 0; q < k; ++q) {  // equal parts
-                const int a = t0 + (int)((long long)n * q / k), b = t0 + (int)((long long)n * (q + 1) / k);
-                groups.push_back(make_int2(c, 8 * a + (b - a)));
-            }
-        }
+        for (int c : ne) gcore::add_row_groups(groups, c, g.cube_start[c], g.cube_start[c + 1] - g.cube_start[c]);
         op->n_groups = (int)groups.size();
         op->d_groups = M.upload(groups, s);
         if (!ne.empty()) op->d_ne_cubes = M.upload(ne, s);

@@ -1,11 +1,12 @@
-// Gather + near zone with LDS-staged operands, one wave per (non-empty cube,
-// 64-slot chunk): the per-lane steps, host+device so that the host self-test
-// runs the same code on the CPU.
+// Gather + near zone with LDS-staged operands: the per-lane steps, host+device so that
+// the host self-tests run the same code on the CPU.  The vector kernels take a row
+// group (a few tets of a cube) and a chunk of slots per wave, the matrix-core kernel a
+// non-empty cube and 64 slots; chunk_part, the near part of one slot a lane, is left
+// to the self-test of the latter's staging.
 //
-//  * grid part: the S* records of up to GT tets of the cube (contiguous, 108
-//    complex each) are copied to the staging buffer with coalesced loads, then
-//    read as wave-uniform broadcasts while each lane streams its slot's 27 box
-//    nodes (gather, src/sparse.f90:47-77, and Y2 - k^2 Y,
+//  * grid part: the S* records of the rows' tets (contiguous, 108 complex each) are
+//    copied to the staging buffer with coalesced loads, then read from there while
+//    each lane streams its slots' 27 box nodes (gather, src/sparse.f90:47-77, and Y2 - k^2 Y,
 //    src/gmres_module.f90:148-153);
 //  * near part (matmul_Acorr_const, src/sparse_mat.f90:96-123): for each x line of
 //    near cubes, in chunks of VC column tets, lane (u, v) = (lane / VC, lane % VC)
@@ -117,6 +118,15 @@ GC_HD Item group_item(const GatherArgs<C> &g, int i) {
     it.t0 = q.y >> 3;
     it.t1 = it.t0 + (q.y & 7);
     return it;
+}
+
+// the row groups of cube c, tets t0 .. t0 + n - 1: equal parts of at most ROW_GT rows
+inline void add_row_groups(std::vector<int2> &out, int c, int t0, int n) {
+    const int k = (n + ROW_GT - 1) / ROW_GT;
+    for (int q = 0; q < k; ++q) {
+        const int a = t0 + (int)((long long)n * q / k), b = t0 + (int)((long long)n * (q + 1) / k);
+        out.push_back(make_int2(c, 8 * a + (b - a)));
+    }
 }
 
 // stage the S* records of tets tp .. tp+nt-1 (lane's share)
@@ -257,8 +267,9 @@ GC_HD void write_out(const GatherArgs<C> &g, const Item &it, int tp, C (*acc)[3]
 // when all lanes read one address: with one slot per lane and one row at a time the
 // block reads alone took the CU's LDS as long as the FMAs took its four SIMDs, and
 // every block was widened to complex128 once per wave and slot chunk.  A row's sum
-// still runs node by node and column by column, as the reference's loops do: the
-// complex64 product keeps its rounding, whatever the batch width.
+// still runs node by node and column by column, as the reference's loops do: in these
+// kernels the complex64 product keeps its rounding, whatever the batch width (up to 4
+// slots, and 5 to 8 on large meshes, run others: k_gather_narrow and k_gather_flat).
 template <int SB, int NS>
 struct Slots {
     int s[NS];    // slot used for loads
@@ -358,6 +369,23 @@ GC_HD void chunk_rows(const GatherArgs<C> &g, const long long *off, int v0, int 
 #pragma unroll
                     for (int i = 0; i < NS; ++i) cfma(acc[u][r][i], a, x[c][i]);
                 }
+        }
+    }
+}
+
+// the lane's rows to y
+template <typename C, int NT, int SB, int NS>
+GC_HD void write_rows(const GatherArgs<C> &g, const Item &it, const Slots<SB, NS> &sl, C (*acc)[3][NS]) {
+#pragma unroll
+    for (int i = 0; i < NS; ++i) {
+        if (!sl.ok[i] || (g.slot_active && !g.slot_active[sl.s[i]])) continue;  // inactive slots are not written
+#pragma unroll
+        for (int u = 0; u < NT; ++u) {
+            const int row = sl.grp * NT + u;
+            if (row >= it.t1 - it.t0) continue;
+            cd *yo = g.y + (size_t)(3 * (it.t0 + row)) * g.B + sl.s[i];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) yo[(size_t)c * g.B] = Prec<cd>::from(acc[u][c][i]);
         }
     }
 }

@@ -300,8 +300,8 @@ __global__ __launch_bounds__(256) void k_scatter_blk_w64(const C *__restrict__ x
 }
 
 // Gather + near zone with the per-tet operands staged in LDS, one 64-thread
-// workgroup per (row group of a cube, 64-slot chunk); the steps are in
-// gather_core.hpp (shared with the host self-test).  Staging keeps many
+// workgroup per (row group of a cube, chunk of slots); the steps are in
+// gather_core.hpp (shared with the host self-test of the row groups).  Staging keeps many
 // operand fetches in flight (wave-uniform operands read through scalar loads
 // would wait on each other).
 template <typename C, int NT, int VC, int SB, int NS>
@@ -342,18 +342,7 @@ __device__ __forceinline__ void gather_pass(const gcore::GatherArgs<C> &g, const
             q += nv;
         }
     });
-#pragma unroll
-    for (int i = 0; i < NS; ++i) {
-        if (!sl.ok[i] || (g.slot_active && !g.slot_active[sl.s[i]])) continue;  // inactive slots are not written
-#pragma unroll
-        for (int u = 0; u < NT; ++u) {
-            const int row = sl.grp * NT + u;
-            if (row >= rows) continue;
-            cd *yo = g.y + (size_t)(3 * (it.t0 + row)) * g.B + sl.s[i];
-#pragma unroll
-            for (int c = 0; c < 3; ++c) yo[(size_t)c * g.B] = Prec<cd>::from(acc[u][c][i]);
-        }
-    }
+    write_rows<C, NT, SB, NS>(g, it, sl, acc);
 }
 
 template <typename C, int VC, int SB, int NS>
