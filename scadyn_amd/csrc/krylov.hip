@@ -1078,7 +1078,7 @@ void launch_tgemm(const cd *mat, const cd *X, long long n, int na, int nx, cd *T
     // chunk is a serial chain: 576 rows, 6 x 6 in two chunks took 67 us, 1,157 rows,
     // 12 x 4 in chunks of 64 rows 27 us and of 32 rows 22); beyond 512 chunks the
     // sum of the parts costs more than the shorter chains give (63,487 rows, 8 x 14:
-    // 44 us with 992 chunks, 58 with 1,984), so there 64 rows
+    // 44 us in 934 chunks of 68 rows, 58 in 1,984 of 32), so there 64 rows
     auto pick = [](int m) { return (m + 47) / 48 * 48 <= (m + 31) / 32 * 32 ? 3 : 2; };
     const int ba = pick(na), bx = pick(nx);
     const int ta = (na + 16 * ba - 1) / (16 * ba), tx = (nx + 16 * bx - 1) / (16 * bx);

@@ -26,8 +26,9 @@ void launch_pg_table(cd *Gtab, const GridDesc &gd, double k, hipStream_t s);
 // Near-zone pairs in the reference's storage order (src/precorrection.f90:182-258:
 // test cube, near cube, test tet, basis tet with reference id >= the test
 // tet's): internal ids PT[p], PB[p] and cube offset PO[p] = (dx+1) + 3(dy+1) +
-// 9(dz+1).  self[t]: the block of tet t with itself.  With ent_blk also the block id (| BLK_TRANSPOSE) and column tet of
-// every row entry.  pos (27 N) and tot (N_cubes + 1) are scratch.
+// 9(dz+1).  self[t]: the block of tet t with itself.  With ent_blk also the block id
+// (| BLK_TRANSPOSE) and column tet of every row entry.  pos (27 N) and tot (N_cubes)
+// are scratch.
 void launch_near_pairs(const int *cube_start, const int *perm, const int64_t *row_start, const GridDesc &gd,
                        uint32_t *pos, uint32_t *tot, int *PT, int *PB, uint8_t *PO, uint32_t *self,
                        int *ent_col, uint32_t *ent_blk, hipStream_t s);

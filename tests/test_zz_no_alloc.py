@@ -104,3 +104,9 @@ def test_project_shapes(n, na, nx):
     for b in (mat_d, X_d, T_d):
         b.free()
     op.close()
+
+
+# chunks of exactly 32 and 64 rows, the most of each: 512
+@pytest.mark.parametrize('n,na,nx', [(16384, 5, 3), (32768, 4, 7)])
+def test_project_whole_chunks(n, na, nx):
+    test_project_shapes(n, na, nx)
