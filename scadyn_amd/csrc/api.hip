@@ -194,7 +194,8 @@ struct scadyn_operator {
     int *d_ent_col = nullptr;
     uint32_t *d_ent_blk = nullptr;
     long long nblocks = 0;
-    std::unique_ptr<Workspace> ws;
+    // shared with a live job (ColumnSolver::hold): other calls then take one of their own
+    std::shared_ptr<Workspace> ws;
     Profiler prof;
     int32_t last_outer_rounds = 0;
     // times the reference's re-orthogonalisation test (src/gmres_module.f90:251)
@@ -547,8 +548,9 @@ static void make_matvec_space(scadyn_operator *op, int B, MatvecSpace &ms) {
 
 static Workspace &workspace(scadyn_operator *op, int B) {
     const int m = op->opts.maxit;
-    if (op->ws && op->ws->B == B && op->ws->m == m) return *op->ws;
-    op->ws.reset(new Workspace());
+    if (op->ws && op->ws.use_count() == 1 && op->ws->B == B && op->ws->m == m) return *op->ws;
+    op->ws.reset();  // its memory goes before the new one's is taken
+    op->ws = std::make_shared<Workspace>();
     Workspace &w = *op->ws;
     w.B = B;
     w.m = m;
@@ -797,13 +799,14 @@ static int auto_batch(scadyn_operator *op, int ncols) {
     // Above 64 columns only where it holds them all or its generations cost no more
     // than a sixteenth above the rule's: the width of the call before (64 from a
     // product of 64 vectors, say) would else run 70 columns as 64 and 6 again.
-    const int have = op->ws && op->ws->m == op->opts.maxit ? op->ws->B : 0;
+    const bool own = op->ws && op->ws.use_count() == 1;
+    const int have = own && op->ws->m == op->opts.maxit ? op->ws->B : 0;
     if (have >= std::min(ncols, 64) &&
         (have >= ncols || 16 * batch_cost(ncols, have) <= 17 * batch_cost(ncols, batch_width(ncols, SIZE_MAX))))
         return have;
     size_t free_b = 0, total_b = 0;
     HIP_CHECK(hipMemGetInfo(&free_b, &total_b));
-    if (op->ws) free_b += op->ws->bytes();  // goes before the new one is made
+    if (own) free_b += op->ws->bytes();  // goes before the new one is made
     size_t per = slot_bytes(op, op->opts.maxit);
     size_t cap = (size_t)(0.75 * (double)free_b) / std::max<size_t>(per, 1);
     if (cap == 0) fail(SCADYN_ERR_MEMORY, "not enough device memory for one RHS slot");
@@ -882,6 +885,7 @@ struct ColumnSolver {
     cd *dst = nullptr;
     int32_t *iters = nullptr;
     Workspace *w = nullptr;
+    std::shared_ptr<Workspace> hold;  // w, until the last column is finished
     KrylovDims d;
     int B = 0;
     Pinned<SlotState> hs;
@@ -912,6 +916,7 @@ struct ColumnSolver {
         spec = sp;
         B = auto_batch(op, (int)cols.size());
         w = &workspace(op, B);
+        hold = op->ws;
         // a complex64 or binary16 basis serves only the mixed-precision blocked-MGS solve
         if ((w->Vf || w->Vh) && (spec.prec != SCADYN_PREC_MIXED || spec.ortho != 0 || spec.mgs_block <= 1))
             fail(SCADYN_ERR_ARG, "solve settings do not match the operator's reduced-precision Krylov basis");
@@ -1258,6 +1263,7 @@ struct TmatJob {
         nfail += cs->nfail;
         rounds = cs->max_cycles;
         finished = true;
+        cs->hold.reset();
     }
 
     // i k^3 mat^H X: ncol x ns, row-major (i, j), on the host
