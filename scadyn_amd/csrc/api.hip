@@ -36,9 +36,11 @@ struct DevMem {
         if (n == 0) n = 1;
         void *p = nullptr;
         hipError_t e = hipMalloc(&p, n * sizeof(T));
-        if (e != hipSuccess)
+        if (e != hipSuccess) {
+            (void)hipGetLastError();  // reported here, not by the next launch's check
             fail(SCADYN_ERR_MEMORY, "hipMalloc of " + std::to_string(n * sizeof(T)) + " bytes failed: " +
                                         hipGetErrorString(e));
+        }
         ptrs.push_back(p);
         bytes += n * sizeof(T);
         return (T *)p;
@@ -308,9 +310,9 @@ static void make_fp32_copies(scadyn_operator *op) {
     if (op->d_S4f) return;
     DevMem &M = op->mem;
     const size_t nS = (size_t)op->g.N * 108, nF = (size_t)op->Hh[0] * op->Hh[1] * op->Hh[2];
-    op->d_S4f = M.alloc<cf>(nS);
+    cf *S4f = M.alloc<cf>(nS);
     op->d_fgf = M.alloc<cf>(nF);
-    hipLaunchKernelGGL(k_to_f32, dim3(1024), dim3(256), 0, op->s, op->d_S4, op->d_S4f, nS);
+    hipLaunchKernelGGL(k_to_f32, dim3(1024), dim3(256), 0, op->s, op->d_S4, S4f, nS);
     hipLaunchKernelGGL(k_to_f32, dim3(1024), dim3(256), 0, op->s, op->d_fg, op->d_fgf, nF);
     HIP_CHECK(hipGetLastError());
     std::vector<cf> tw;
@@ -320,6 +322,7 @@ static void make_fp32_copies(scadyn_operator *op) {
     }
     op->d_twf = M.upload(tw, op->s);
     HIP_CHECK(hipStreamSynchronize(op->s));
+    op->d_S4f = S4f;  // only when complete
 }
 
 // Morton code of cube coordinates (bits of x, y, z interleaved, 21 per axis)
@@ -550,8 +553,8 @@ static Workspace &workspace(scadyn_operator *op, int B) {
     const int m = op->opts.maxit;
     if (op->ws && op->ws.use_count() == 1 && op->ws->B == B && op->ws->m == m) return *op->ws;
     op->ws.reset();  // its memory goes before the new one's is taken
-    op->ws = std::make_shared<Workspace>();
-    Workspace &w = *op->ws;
+    const std::shared_ptr<Workspace> made = std::make_shared<Workspace>();
+    Workspace &w = *made;
     w.B = B;
     w.m = m;
     w.n = 3LL * op->g.N;
@@ -605,6 +608,7 @@ static Workspace &workspace(scadyn_operator *op, int B) {
     w.hprev = w.mem.alloc<cd>((size_t)B * (m + 1));
     w.col = w.mem.alloc<int>(B);
     w.ret = w.mem.alloc<int>(B);
+    op->ws = made;  // only when complete: an allocation above may have failed
     return w;
 }
 
@@ -614,13 +618,14 @@ static void h2d_sync(void *dst, const void *src, size_t bytes, hipStream_t s);
 static void restart_space(scadyn_operator *op, Workspace &w) {
     if (w.rs) return;
     w.rs_cap = std::min(w.B, 8);
-    w.rs.reset(new MatvecSpace());
-    make_matvec_space(op, w.rs_cap, *w.rs);
+    std::unique_ptr<MatvecSpace> rs(new MatvecSpace());
+    make_matvec_space(op, w.rs_cap, *rs);
     w.rx = w.mem.alloc<cd>((size_t)w.n * w.rs_cap);
     w.ry = w.mem.alloc<cd>((size_t)w.n * w.rs_cap);
     w.rslot = w.mem.alloc<int>(w.rs_cap);
     std::vector<long long> off(w.rs_cap, 0);
-    h2d_sync(w.rs->in_off, off.data(), sizeof(long long) * w.rs_cap, op->s);
+    h2d_sync(rs->in_off, off.data(), sizeof(long long) * w.rs_cap, op->s);
+    w.rs = std::move(rs);  // only when complete
 }
 
 struct ProfScope {
