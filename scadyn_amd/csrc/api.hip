@@ -483,10 +483,13 @@ static void create_operator(scadyn_operator *op, const scadyn_mesh &mesh, const 
             }
         }
         std::vector<cd> WW = pinv_jacobi(W, 98, 27, 1e-6);
+        // the sample points behind it: the operator's own, others may be in the making
+        for (int i = 0; i < 98 * 3; i += 2) WW.push_back(cmk(Psph[i], Psph[i + 1]));
         cd *d_WW = M.upload(WW, s);
-        upload_tables(Psph.data(), s);
+        upload_tables(s);
         op->d_S4 = M.alloc<cd>((size_t)N * 108);
-        launch_projection(op->d_tcoord, op->d_vol, op->d_tet_cube, gd, k, d_WW, op->d_S4, N, s);
+        launch_projection(op->d_tcoord, op->d_vol, op->d_tet_cube, gd, k, d_WW, (const double *)(d_WW + 98 * 27),
+                          op->d_S4, N, s);
         HIP_CHECK(hipStreamSynchronize(s));
         M.release(d_WW);
     }

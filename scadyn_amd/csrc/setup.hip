@@ -20,7 +20,6 @@ __constant__ double c_tet24_p[24 * 3];
 __constant__ double c_tet24_w[24];
 __constant__ double c_tri7_p[7 * 2];
 __constant__ double c_tri7_w[7];
-__constant__ double c_cube98[98 * 3];  // 2*box_delta * sample points
 
 static const double PI_D = 3.141592653589793;
 
@@ -72,7 +71,9 @@ const double *host_tet24_w() { return h_tet24_w; }
 const double *host_tri7_p() { return h_tri7_p; }
 const double *host_tri7_w() { return h_tri7_w; }
 
-void upload_tables(const double *cube98_scaled, hipStream_t s) {
+// the quadrature rules: the same bytes for every operator, so that operators made in
+// several threads may write them while others read
+void upload_tables(hipStream_t s) {
     HIP_CHECK(hipMemcpyToSymbolAsync(HIP_SYMBOL(c_tet24_p), h_tet24_p, sizeof(h_tet24_p), 0,
                                      hipMemcpyHostToDevice, s));
     HIP_CHECK(hipMemcpyToSymbolAsync(HIP_SYMBOL(c_tet24_w), h_tet24_w, sizeof(h_tet24_w), 0,
@@ -80,8 +81,6 @@ void upload_tables(const double *cube98_scaled, hipStream_t s) {
     HIP_CHECK(hipMemcpyToSymbolAsync(HIP_SYMBOL(c_tri7_p), h_tri7_p, sizeof(h_tri7_p), 0,
                                      hipMemcpyHostToDevice, s));
     HIP_CHECK(hipMemcpyToSymbolAsync(HIP_SYMBOL(c_tri7_w), h_tri7_w, sizeof(h_tri7_w), 0,
-                                     hipMemcpyHostToDevice, s));
-    HIP_CHECK(hipMemcpyToSymbolAsync(HIP_SYMBOL(c_cube98), cube98_scaled, 98 * 3 * sizeof(double), 0,
                                      hipMemcpyHostToDevice, s));
 }
 
@@ -408,6 +407,7 @@ __global__ __launch_bounds__(128) void k_projection(const double *__restrict__ t
                                                     const double *__restrict__ vol,
                                                     const int *__restrict__ tet_cube, GridDesc gd,
                                                     double k, const cd *__restrict__ WW,
+                                                    const double *__restrict__ cube98,
                                                     cd *__restrict__ S4, int N) {
     __shared__ cd Q[4][98];
     const int t = blockIdx.x;
@@ -420,7 +420,7 @@ __global__ __launch_bounds__(128) void k_projection(const double *__restrict__ t
     v3 cp = mk3(node1.x + gd.box_delta / 2.0, node1.y + gd.box_delta / 2.0, node1.z + gd.box_delta / 2.0);
     const double v = vol[t];
     for (int m = threadIdx.x; m < 98; m += blockDim.x) {
-        v3 test = add3(mk3(c_cube98[3 * m], c_cube98[3 * m + 1], c_cube98[3 * m + 2]), cp);
+        v3 test = add3(mk3(cube98[3 * m], cube98[3 * m + 1], cube98[3 * m + 2]), cp);
         // 1-point tet rule: centroid, weight W0*6*vol
         v3 pb = tet_point(tc, 0.25, 0.25, 0.25);
         double wb = 1.666666666666667e-01 * 6.0 * v;
@@ -1038,8 +1038,8 @@ __global__ void k_vswf(const double *__restrict__ tcoord, const double *__restri
 
 // ---- launchers -----------------------------------------------------------------
 void launch_projection(const double *tcoord, const double *vol, const int *tet_cube, const GridDesc &gd,
-                       double k, const cd *WW, cd *S4, int N, hipStream_t s) {
-    hipLaunchKernelGGL(k_projection, dim3(N), dim3(128), 0, s, tcoord, vol, tet_cube, gd, k, WW, S4, N);
+                       double k, const cd *WW, const double *cube98, cd *S4, int N, hipStream_t s) {
+    hipLaunchKernelGGL(k_projection, dim3(N), dim3(128), 0, s, tcoord, vol, tet_cube, gd, k, WW, cube98, S4, N);
     HIP_CHECK(hipGetLastError());
 }
 void launch_green_grid(cd *A, const GridDesc &gd, int Lx, int Ly, int Lz, double k, hipStream_t s) {

@@ -12,14 +12,15 @@ struct GridDesc {
     int ncx, ncy, ncz;
 };
 
-void upload_tables(const double *cube98_scaled, hipStream_t s);
+void upload_tables(hipStream_t s);
 const double *host_tet24_p();
 const double *host_tet24_w();
 const double *host_tri7_p();
 const double *host_tri7_w();
 
+// cube98: the 98 sample points, times 2 box_delta
 void launch_projection(const double *tcoord, const double *vol, const int *tet_cube, const GridDesc &gd,
-                       double k, const cd *WW, cd *S4, int N, hipStream_t s);
+                       double k, const cd *WW, const double *cube98, cd *S4, int N, hipStream_t s);
 void launch_green_grid(cd *A, const GridDesc &gd, int Lx, int Ly, int Lz, double k, hipStream_t s);
 void launch_fg_octant(const cd *F, cd *fg, int Lx, int Ly, int Lz, hipStream_t s);
 void launch_pg_table(cd *Gtab, const GridDesc &gd, double k, hipStream_t s);
