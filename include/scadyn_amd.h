@@ -126,6 +126,8 @@ const char *scadyn_last_error(void);
  * complex arrays, nm = nmax(nmax+2), returned already scaled by i k^3
  * (src/T_matrix.f90:270-275).  iters (optional, length 2*nm) receives
  * the GMRES iteration count of each column.
+ * A bar's large blocks of device memory are kept for up to a second for the
+ * next bar, at most a quarter of the card.
  */
 int scadyn_tmat_solve(const scadyn_mesh *mesh, const scadyn_opts *opts,
                       double k, int32_t nmax,

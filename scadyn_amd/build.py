@@ -107,6 +107,7 @@ SELFTESTS = {'fft': ('fft_selftest.hip', SELFTEST), 'bmgs': ('bmgs_selftest.hip'
              'fft_inst': ('fft_inst_selftest.hip', os.path.join(OBJDIR, 'fft_inst_selftest')),
              'gather_rows': ('gather_rows_selftest.hip', os.path.join(OBJDIR, 'gather_rows_selftest')),
              'scatter': ('scatter_selftest.hip', os.path.join(OBJDIR, 'scatter_selftest')),
+             'devpool': ('devpool_selftest.hip', os.path.join(OBJDIR, 'devpool_selftest')),
              'pairs': ('pairs_selftest.hip', os.path.join(OBJDIR, 'pairs_selftest')),
              'pinv': ('pinv_selftest.hip', os.path.join(OBJDIR, 'pinv_selftest'))}
 
@@ -117,8 +118,8 @@ def build_selftest(verbose=False, which='fft'):
     planner), 'fft_inst' its compiled instances at the planner's widths, 'bmgs'
     and 'mgsb' the block Gram-Schmidt bodies, 'scatter' the narrow scatter,
     'pairs' the near-zone pair and row lists, 'gather' the gather's staging and
-    its matrix-core pass, 'gather_rows' its row-group kernels, 'pinv' the
-    pseudo-inverse (from the library)."""
+    its matrix-core pass, 'gather_rows' its row-group kernels, 'devpool'
+    the device-memory pool, 'pinv' the pseudo-inverse (from the library)."""
     hipcc = os.environ.get('HIPCC', '/opt/rocm/bin/hipcc')
     os.makedirs(OBJDIR, exist_ok=True)
     src, exe = SELFTESTS[which]

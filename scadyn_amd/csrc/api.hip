@@ -13,6 +13,7 @@
 #include <mutex>
 #include <thread>
 
+#include "devpool.hpp"
 #include "fft.hpp"
 #include "gather_core.hpp"
 #include "internal.hpp"
@@ -28,22 +29,57 @@ void set_error(int, const std::string &msg) { g_err = msg; }
 void fail(int code, const std::string &msg) { throw Error{code, msg}; }
 
 // ---------------------------------------------------------------- device memory
+static void free_on(int device, void *p) {
+    (void)hipSetDevice(device);
+    (void)hipFree(p);
+}
+static DevicePool &pool() {
+    static DevicePool p(free_on, 1.0);
+    return p;
+}
+constexpr size_t POOL_LEAST = (size_t)32 << 20;  // smaller blocks are freed at once
+// the bar that this thread runs: its blocks go to the pool (DevMem)
+static thread_local bool t_bar = false;
+struct BarScope {
+    BarScope() { t_bar = true; }
+    ~BarScope() { t_bar = false; }
+};
+
+// free device memory, what the pool keeps included: an allocation that fails
+// without it gives it back
+static size_t free_memory() {
+    int device = 0;
+    size_t free_b = 0, total_b = 0;
+    HIP_CHECK(hipGetDevice(&device));
+    HIP_CHECK(hipMemGetInfo(&free_b, &total_b));
+    return free_b + pool().kept(device);
+}
+
 struct DevMem {
-    std::vector<void *> ptrs;
+    struct Block {
+        void *p;
+        size_t size;
+    };
+    std::vector<Block> blocks;
     size_t bytes = 0;
+    int device = 0;
+    const bool bar = t_bar;
     template <class T>
     T *alloc(size_t n) {
         if (n == 0) n = 1;
-        void *p = nullptr;
-        hipError_t e = hipMalloc(&p, n * sizeof(T));
+        const size_t want = n * sizeof(T);
+        Block b = {nullptr, want};
+        HIP_CHECK(hipGetDevice(&device));
+        if (bar && want >= POOL_LEAST) b.p = pool().take(device, want, &b.size);
+        hipError_t e = b.p ? hipSuccess : hipMalloc(&b.p, want);
+        if (e != hipSuccess && pool().trim(device)) e = hipMalloc(&b.p, want);
         if (e != hipSuccess) {
             (void)hipGetLastError();  // reported here, not by the next launch's check
-            fail(SCADYN_ERR_MEMORY, "hipMalloc of " + std::to_string(n * sizeof(T)) + " bytes failed: " +
-                                        hipGetErrorString(e));
+            fail(SCADYN_ERR_MEMORY, "hipMalloc of " + std::to_string(want) + " bytes failed: " + hipGetErrorString(e));
         }
-        ptrs.push_back(p);
-        bytes += n * sizeof(T);
-        return (T *)p;
+        blocks.push_back(b);
+        bytes += want;
+        return (T *)b.p;
     }
     template <class T>
     T *upload(const std::vector<T> &v, hipStream_t s) {
@@ -56,15 +92,28 @@ struct DevMem {
         return p;
     }
     void release(void *p) {
-        auto it = std::find(ptrs.begin(), ptrs.end(), p);
-        if (it != ptrs.end()) {
+        auto it = std::find_if(blocks.begin(), blocks.end(), [&](const Block &b) { return b.p == p; });
+        if (it != blocks.end()) {
             (void)hipFree(p);
-            ptrs.erase(it);
+            blocks.erase(it);
         }
     }
     void clear() {
-        for (void *p : ptrs) (void)hipFree(p);
-        ptrs.clear();
+        bool keep = false;
+        size_t total_b = 0;
+        for (const Block &b : blocks) keep |= bar && b.size >= POOL_LEAST;
+        if (keep) {
+            size_t free_b = 0;
+            // as a free does, wait for whatever still uses the blocks
+            keep = hipSetDevice(device) == hipSuccess && hipDeviceSynchronize() == hipSuccess &&
+                   hipMemGetInfo(&free_b, &total_b) == hipSuccess;
+        }
+        for (const Block &b : blocks)
+            if (keep && b.size >= POOL_LEAST)
+                pool().keep(device, b.p, b.size, total_b / 4);  // at most a quarter of the card
+            else
+                (void)hipFree(b.p);
+        blocks.clear();
         bytes = 0;
     }
     ~DevMem() { clear(); }
@@ -812,8 +861,7 @@ static int auto_batch(scadyn_operator *op, int ncols) {
     if (have >= std::min(ncols, 64) &&
         (have >= ncols || 16 * batch_cost(ncols, have) <= 17 * batch_cost(ncols, batch_width(ncols, SIZE_MAX))))
         return have;
-    size_t free_b = 0, total_b = 0;
-    HIP_CHECK(hipMemGetInfo(&free_b, &total_b));
+    size_t free_b = free_memory();
     if (own) free_b += op->ws->bytes();  // goes before the new one is made
     size_t per = slot_bytes(op, op->opts.maxit);
     size_t cap = (size_t)(0.75 * (double)free_b) / std::max<size_t>(per, 1);
@@ -1972,6 +2020,7 @@ void scadyn_tjob_destroy(scadyn_tjob *j) {
 
 int scadyn_tmat_solve(const scadyn_mesh *mesh, const scadyn_opts *opts, double k, int32_t nmax, double *Taa,
                       double *Tab, double *Tba, double *Tbb, int32_t *iters) {
+    const BarScope bar;
     scadyn_operator *op = nullptr;
     int rc = scadyn_op_create(mesh, opts, k, &op);
     if (rc) return rc;
@@ -2049,9 +2098,7 @@ int scadyn_server_create(const scadyn_server_opts *so, scadyn_server **out) {
     if (budget == 0 && sv->host_only) fail(SCADYN_ERR_ARG, "a host-only server needs an explicit hbm_budget");
     if (budget == 0) {
         HIP_CHECK(hipSetDevice(sv->device));
-        size_t fr = 0, tot = 0;
-        HIP_CHECK(hipMemGetInfo(&fr, &tot));
-        budget = (size_t)(0.8 * (double)fr);
+        budget = (size_t)(0.8 * (double)free_memory());
     }
     sv->budget = budget;
     sv->t0 = std::chrono::steady_clock::now();
