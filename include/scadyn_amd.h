@@ -126,8 +126,6 @@ const char *scadyn_last_error(void);
  * complex arrays, nm = nmax(nmax+2), returned already scaled by i k^3
  * (src/T_matrix.f90:270-275).  iters (optional, length 2*nm) receives
  * the GMRES iteration count of each column.
- * A bar's large blocks of device memory are kept for up to a second for the
- * next bar, at most a quarter of the card.
  */
 int scadyn_tmat_solve(const scadyn_mesh *mesh, const scadyn_opts *opts,
                       double k, int32_t nmax,
@@ -143,6 +141,8 @@ typedef struct scadyn_operator scadyn_operator;
  * src/precorrection.f90:131-264). */
 int scadyn_op_create(const scadyn_mesh *mesh, const scadyn_opts *opts, double k,
                      scadyn_operator **out);
+/* Large blocks of device memory that an operator or a call frees are kept for up
+ * to a second for the next one, at most a quarter of the card. */
 void scadyn_op_destroy(scadyn_operator *op);
 
 /* Sizes: info[0..15] = N_tet, Nx, Ny, Nz, N_cubes, N_tet_cube, n_blocks,

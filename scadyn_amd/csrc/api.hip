@@ -38,12 +38,9 @@ static DevicePool &pool() {
     return p;
 }
 constexpr size_t POOL_LEAST = (size_t)32 << 20;  // smaller blocks are freed at once
-// the bar that this thread runs: its blocks go to the pool (DevMem)
-static thread_local bool t_bar = false;
-struct BarScope {
-    BarScope() { t_bar = true; }
-    ~BarScope() { t_bar = false; }
-};
+// blocks that this thread's objects free go to the pool; not those of the request
+// loop, whose memory budget is its own
+static thread_local bool t_keep = true;
 
 // free device memory, what the pool keeps included: an allocation that fails
 // without it gives it back
@@ -63,14 +60,14 @@ struct DevMem {
     std::vector<Block> blocks;
     size_t bytes = 0;
     int device = 0;
-    const bool bar = t_bar;
+    const bool keeps = t_keep;
     template <class T>
     T *alloc(size_t n) {
         if (n == 0) n = 1;
         const size_t want = n * sizeof(T);
         Block b = {nullptr, want};
         HIP_CHECK(hipGetDevice(&device));
-        if (bar && want >= POOL_LEAST) b.p = pool().take(device, want, &b.size);
+        if (keeps && want >= POOL_LEAST) b.p = pool().take(device, want, &b.size);
         hipError_t e = b.p ? hipSuccess : hipMalloc(&b.p, want);
         if (e != hipSuccess && pool().trim(device)) e = hipMalloc(&b.p, want);
         if (e != hipSuccess) {
@@ -101,7 +98,7 @@ struct DevMem {
     void clear() {
         bool keep = false;
         size_t total_b = 0;
-        for (const Block &b : blocks) keep |= bar && b.size >= POOL_LEAST;
+        for (const Block &b : blocks) keep |= keeps && b.size >= POOL_LEAST;
         if (keep) {
             size_t free_b = 0;
             // as a free does, wait for whatever still uses the blocks
@@ -1505,6 +1502,7 @@ static void stamp(scadyn_server *sv, Request *r, int i) {
 }  // namespace scadyn
 
 void scadyn_server::run() {
+    t_keep = false;
     using namespace scadyn;
     if (!host_only) (void)hipSetDevice(device);
     for (;;) {
@@ -2020,7 +2018,6 @@ void scadyn_tjob_destroy(scadyn_tjob *j) {
 
 int scadyn_tmat_solve(const scadyn_mesh *mesh, const scadyn_opts *opts, double k, int32_t nmax, double *Taa,
                       double *Tab, double *Tba, double *Tbb, int32_t *iters) {
-    const BarScope bar;
     scadyn_operator *op = nullptr;
     int rc = scadyn_op_create(mesh, opts, k, &op);
     if (rc) return rc;

@@ -1,13 +1,13 @@
-// Device memory kept between the operators of consecutive bars (host code; the
-// allocator behind it is passed in, so that the host self-test runs it on the CPU).
+// Device memory kept between the calls of consecutive bars (host code; the allocator
+// behind it is passed in, so that the host self-test runs it on the CPU).
 //
-// A bar (scadyn_tmat_solve) makes an operator and frees it: 14 GB in 120 ms at 43,248
-// tets, FP64, nmax 5.  The driver wipes freed device memory at about 36 GB/s here; bars
-// that follow one another faster build up a backlog, for which an allocation then
-// waits up to seconds.  Bars of one mesh in a row, FP64, ms, mean (longest): 43,248
-// tets, nmax 5 384 (4,187) with every block freed, 119 (128) with the large ones kept;
-// 103 k, nmax 6 1,176 (5,387) and 306 (307); 201 k, nmax 6 2,219 (6,391) and 601
-// (1,189), though its blocks exceed the limit.
+// A bar makes an operator and frees it: 14 GB in 120 ms at 43,248 tets, FP64, nmax 5.
+// The driver wipes freed device memory at about 36 GB/s here; bars that follow one
+// another faster build up a backlog, for which an allocation then waits up to
+// seconds.  Bars of one mesh in a row, FP64, ms, mean (longest): 43,248 tets, nmax 5
+// 384 (4,187) with every block freed, 119 (128) with the large ones kept; 103 k, nmax 6
+// 1,176 (5,387) and 306 (307); 201 k, nmax 6 2,219 (6,391) and 601 (1,189), though its
+// blocks exceed the limit.
 //
 //  * Bounded: at most `limit` bytes a device; the blocks kept longest go first.
 //  * Given back: a thread frees what no call took for `idle` seconds; a failed

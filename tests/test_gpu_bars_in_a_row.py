@@ -65,3 +65,23 @@ def test_same_results_and_memory_given_back():
     assert free_bytes() < free - (1 << 28)
     time.sleep(2.5)
     assert free_bytes() > free - (1 << 26)
+    op = native.Operator(*a[:4], **o)
+    T = op.tmatrix(a[4])
+    op.close()
+    assert same(T, first[0])
+    assert free_bytes() < free - (1 << 28)
+    time.sleep(2.5)
+    assert free_bytes() > free - (1 << 26)
+
+
+def test_the_request_loop_keeps_nothing():
+    from scadyn_amd import native
+    a, o = bars()[0]
+    sv = native.Server()
+    sv.wait(sv.submit(*a, **o))
+    time.sleep(2.5)
+    free = free_bytes()
+    sv.wait(sv.submit(*a, **o))
+    time.sleep(0.2)  # the worker retires the request
+    assert free_bytes() > free - (1 << 26)
+    sv.close()
