@@ -115,8 +115,9 @@ private:
                 continue;
             }
             // blocks are in the order of their times
-            if (Clock::now() < blocks_.front().until) {
-                cv_.wait_until(lk, blocks_.front().until);
+            const Clock::time_point until = blocks_.front().until;  // the list may move meanwhile
+            if (Clock::now() < until) {
+                cv_.wait_until(lk, until);
                 continue;
             }
             const Block b = blocks_.front();

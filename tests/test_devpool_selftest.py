@@ -18,3 +18,15 @@ def test_device_pool():
     r = subprocess.run([exe], capture_output=True, text=True, env=env, timeout=600)
     assert r.returncode == 0, r.stdout[-4000:] + r.stderr[-4000:]
     assert ' 0 failures' in r.stdout
+
+
+def test_device_pool_built_by_the_host_compiler(tmp_path):
+    """It optimises less away: reads that the device compiler drops stay and are checked."""
+    src = os.path.join(build.CSRC, build.SELFTESTS['devpool'][0])
+    exe = str(tmp_path / 'devpool_selftest')
+    cmd = ['g++', '-x', 'c++', '-std=c++17', '-g', '-O1', '-fsanitize=address', '-pthread', '-o', exe, src]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-4000:]
+    env = dict(os.environ, ASAN_OPTIONS='detect_leaks=0')
+    r = subprocess.run([exe], capture_output=True, text=True, env=env, timeout=600)
+    assert r.returncode == 0, r.stdout[-4000:] + r.stderr[-4000:]
