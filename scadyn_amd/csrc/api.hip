@@ -33,10 +33,7 @@ static void free_on(int device, void *p) {
     (void)hipSetDevice(device);
     (void)hipFree(p);
 }
-static DevicePool &pool() {
-    static DevicePool p(free_on, 1.0);
-    return p;
-}
+static DevicePool &pool() { return process_pool(free_on, 1.0); }
 constexpr size_t POOL_LEAST = (size_t)32 << 20;  // smaller blocks are freed at once
 // blocks that this thread's objects free go to the pool; not those of the request
 // loop, whose memory budget is its own

@@ -24,14 +24,21 @@
 #include <thread>
 #include <vector>
 
+#include <unistd.h>
+
 namespace scadyn {
 
 class DevicePool {
 public:
     typedef void (*Free)(int device, void *p);
     DevicePool(Free f, double idle_s) : free_(f), idle_(std::chrono::duration_cast<Clock::duration>(std::chrono::duration<double>(idle_s))) {}
-    // at the process's end the driver takes the memory back
-    ~DevicePool() {
+    ~DevicePool() { stop(); }
+
+    // Ends the thread; from then on blocks are freed at once.  What is still kept the
+    // driver takes back at the process's end.  A forked child has no such thread:
+    // nothing to wait for.
+    void stop() {
+        if (reaper_.joinable() && pid_ != getpid()) return;
         {
             std::lock_guard<std::mutex> lk(mu_);
             stop_ = true;
@@ -55,11 +62,12 @@ public:
         return p;
     }
 
-    // keeps an idle block; what exceeds the limit is freed
+    // keeps an idle block; what exceeds the limit is freed, all of it after stop()
     void keep(int device, void *p, size_t size, size_t limit) {
         std::vector<Block> out;
         {
             std::lock_guard<std::mutex> lk(mu_);
+            if (stop_) limit = 0;
             blocks_.push_back({device, p, size, Clock::now() + idle_});
             size_t sum = 0;
             for (const Block &b : blocks_) sum += b.device == device ? b.size : 0;
@@ -72,7 +80,10 @@ public:
                 out.push_back(blocks_[i]);
                 blocks_.erase(blocks_.begin() + (long)i);
             }
-            if (!reaper_.joinable()) reaper_ = std::thread([this] { reap(); });
+            if (!stop_ && !reaper_.joinable()) {
+                pid_ = getpid();
+                reaper_ = std::thread([this] { reap(); });
+            }
         }
         cv_.notify_all();
         for (const Block &b : out) free_(b.device, b.p);
@@ -134,7 +145,19 @@ private:
     std::condition_variable cv_;
     std::vector<Block> blocks_;
     std::thread reaper_;
+    pid_t pid_ = 0;  // the process that the thread runs in
     bool stop_ = false;
 };
+
+// The process's pool.  Its thread ends before the driver's own clean-up (statics made
+// first go last); the object stays, since objects that end later may still free
+// memory and since a forked child could not destroy what its parent's thread waits on.
+inline DevicePool &process_pool(DevicePool::Free f, double idle_s) {
+    static DevicePool *const pool = new DevicePool(f, idle_s);
+    static struct End {
+        ~End() { pool->stop(); }
+    } end;
+    return *pool;
+}
 
 }  // namespace scadyn

@@ -1,7 +1,8 @@
 // Host self-test of the device-memory pool (devpool.hpp) over a stand-in allocator:
 // which block is taken, the limit, devices apart, memory given back after the idle
-// time and on trim, and threads that take and keep at once (no block ever has two
-// owners, every block is freed once).
+// time and on trim, threads that take and keep at once (no block ever has two
+// owners, every block is freed once), a forked child that ends, and objects freed
+// after the pool's end.
 //
 // Exit status 0 when all of it holds.
 #include <atomic>
@@ -10,6 +11,10 @@
 #include <map>
 #include <random>
 #include <set>
+
+#include <csignal>
+#include <sys/wait.h>
+#include <unistd.h>
 
 #include "devpool.hpp"
 
@@ -33,7 +38,42 @@ static size_t freed(void *p) {
 }
 static void *at(size_t i) { return (void *)(i * 64 + 64); }
 
+// a user's static object that frees its memory after the pool's end: the child's exit
+// status is 3 where that memory was freed
+static struct Late {
+    bool armed = false;
+    ~Late() {
+        if (!armed) return;
+        process_pool(fake_free, 60.0).keep(0, at(21), 100, 1000);
+        _exit(freed(at(21)) == 1 ? 3 : 4);
+    }
+} g_late;
+
+// exit status of a child that runs f and ends as programs do; -1 where it hangs
+template <class F>
+static int child(F f) {
+    std::fflush(stdout);
+    const pid_t p = fork();
+    if (p == 0) {
+        f();
+        std::exit(0);
+    }
+    for (int i = 0; i < 200; ++i) {
+        int st = 0;
+        if (waitpid(p, &st, WNOHANG) == p) return WIFEXITED(st) ? WEXITSTATUS(st) : -2;
+        std::this_thread::sleep_for(std::chrono::milliseconds(50));
+    }
+    (void)kill(p, SIGKILL);
+    (void)waitpid(p, nullptr, 0);
+    return -1;
+}
+
 int main() {
+    expect(child([] {
+               process_pool(fake_free, 60.0).keep(0, at(20), 100, 1000);
+               g_late.armed = true;
+           }) == 3,
+           "an object freed after the pool's end");
     {
         DevicePool pool(fake_free, 60.0);
         size_t size = 0;
@@ -105,6 +145,9 @@ int main() {
         expect(twice == 0, "one owner at a time, none freed before");
         expect(once, "each block freed once");
     }
+    process_pool(fake_free, 60.0).keep(0, at(22), 100, 1000);
+    std::this_thread::sleep_for(std::chrono::milliseconds(50));  // its thread waits
+    expect(child([] {}) == 0, "a forked child ends");
     std::printf("%d cases, %d failures\n", cases, failures);
     return failures != 0;
 }
