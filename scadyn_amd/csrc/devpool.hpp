@@ -20,6 +20,7 @@
 #include <chrono>
 #include <condition_variable>
 #include <cstddef>
+#include <exception>
 #include <mutex>
 #include <thread>
 #include <vector>
@@ -62,11 +63,19 @@ public:
         return p;
     }
 
-    // keeps an idle block; what exceeds the limit is freed, all of it after stop()
-    void keep(int device, void *p, size_t size, size_t limit) {
+    // keeps an idle block; what exceeds the limit is freed, all of it after stop() or
+    // where the thread or the list's memory cannot be had (never throws: objects call it
+    // as they end)
+    void keep(int device, void *p, size_t size, size_t limit) noexcept {
         std::vector<Block> out;
-        {
+        try {
             std::lock_guard<std::mutex> lk(mu_);
+            if (!stop_ && !reaper_.joinable()) {
+                pid_ = getpid();
+                reaper_ = std::thread([this] { reap(); });
+            }
+            blocks_.reserve(blocks_.size() + 1);
+            out.reserve(blocks_.size() + 1);
             if (stop_) limit = 0;
             blocks_.push_back({device, p, size, Clock::now() + idle_});
             size_t sum = 0;
@@ -80,10 +89,9 @@ public:
                 out.push_back(blocks_[i]);
                 blocks_.erase(blocks_.begin() + (long)i);
             }
-            if (!stop_ && !reaper_.joinable()) {
-                pid_ = getpid();
-                reaper_ = std::thread([this] { reap(); });
-            }
+        } catch (const std::exception &) {  // before the block was listed
+            free_(device, p);
+            return;
         }
         cv_.notify_all();
         for (const Block &b : out) free_(b.device, b.p);

@@ -1,8 +1,8 @@
 // Host self-test of the device-memory pool (devpool.hpp) over a stand-in allocator:
 // which block is taken, the limit, devices apart, memory given back after the idle
 // time and on trim, threads that take and keep at once (no block ever has two
-// owners, every block is freed once), a forked child that ends, and objects freed
-// after the pool's end.
+// owners, every block is freed once), a forked child that ends, objects freed
+// after the pool's end, and a pool that cannot have its thread.
 //
 // Exit status 0 when all of it holds.
 #include <atomic>
@@ -13,6 +13,7 @@
 #include <set>
 
 #include <csignal>
+#include <pthread.h>
 #include <sys/wait.h>
 #include <unistd.h>
 
@@ -144,6 +145,20 @@ int main() {
         for (size_t i = 1000; i < next; ++i) once &= freed(at(i)) == 1;
         expect(twice == 0, "one owner at a time, none freed before");
         expect(once, "each block freed once");
+    }
+    {
+        // threads' default stack larger than the address space: none can be made
+        pthread_attr_t was, huge;
+        (void)pthread_getattr_default_np(&was);
+        pthread_attr_init(&huge);
+        const bool set = pthread_attr_setstacksize(&huge, (size_t)1 << 50) == 0 && pthread_setattr_default_np(&huge) == 0;
+        expect(set, "a stack size that no thread gets");
+        DevicePool pool(fake_free, 60.0);
+        if (set) pool.keep(0, at(23), 100, 1000);
+        (void)pthread_setattr_default_np(&was);
+        expect(freed(at(23)) == 1 && pool.kept(0) == 0, "freed at once without a thread");
+        pool.keep(0, at(24), 100, 1000);
+        expect(freed(at(24)) == 0 && pool.kept(0) == 100, "kept once there is one");
     }
     process_pool(fake_free, 60.0).keep(0, at(22), 100, 1000);
     std::this_thread::sleep_for(std::chrono::milliseconds(50));  // its thread waits
