@@ -30,8 +30,13 @@ void fail(int code, const std::string &msg) { throw Error{code, msg}; }
 
 // ---------------------------------------------------------------- device memory
 static void free_on(int device, void *p) {
+    // relaxed: in the default mode a free by the pool's thread would invalidate a
+    // capture that another thread of the program has under way, and fail
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool set = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
     (void)hipSetDevice(device);
     (void)hipFree(p);
+    if (set) (void)hipThreadExchangeStreamCaptureMode(&mode);
 }
 static DevicePool &pool() { return process_pool(free_on, 1.0); }
 constexpr size_t POOL_LEAST = (size_t)32 << 20;  // smaller blocks are freed at once
