@@ -645,9 +645,14 @@ static Workspace &workspace(scadyn_operator *op, int B) {
         // row-sweep workgroups of the Krylov kernels: up to 2048 (8 waves per
         // SIMD), each sweeping at least 16 row groups, except that small systems
         // spread over up to 1024 workgroups: a sweep is a chain of dependent row groups
-        // (5,472 tets, 3 slots: 12 workgroups of 16 groups 30.2 us, 194 of one 20.5)
+        // (5,472 tets, 3 slots: 12 workgroups of 16 groups 30.2 us, 194 of one 20.5).
+        // Up to 256 where a pass leaves 21 (6 vectors) or 36 (8) partial sums a slot and
+        // workgroup, which one workgroup per slot adds: solves of 25,344 tets, 3 slots,
+        // 8 vectors 7.6 ms with 16 groups at least, 9.2 in up to 1024 workgroups,
+        // 5.6 in 256; 103,536 tets, 1 slot 16.5, 21.5, 11.3
         const long long rw = 256 / std::min(B, 256), groups = (w.n + rw - 1) / rw;
-        w.nwg = (int)std::max(std::min(groups, 1024LL), std::min(2048LL, (groups + 15) / 16));
+        const long long spread = op->opts.mgs_block > 4 ? 256 : 1024;
+        w.nwg = (int)std::max(std::min(groups, spread), std::min(2048LL, (groups + 15) / 16));
     }
     w.nrm2 = w.mem.alloc<double>(B);
     w.nav2 = w.mem.alloc<double>(B);
