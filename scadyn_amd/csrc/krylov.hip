@@ -1078,8 +1078,11 @@ void launch_tgemm(const cd *mat, const cd *X, long long n, int na, int nx, cd *T
     // chunk is a serial chain: 576 rows, 6 x 6 in two chunks took 67 us, 1,157 rows,
     // 12 x 4 in chunks of 64 rows 27 us and of 32 rows 22); beyond 512 chunks the
     // sum of the parts costs more than the shorter chains give (63,487 rows, 8 x 14:
-    // 44 us in 934 chunks of 68 rows, 58 in 1,984 of 32), so there 64 rows
-    auto pick = [](int m) { return (m + 47) / 48 * 48 <= (m + 31) / 32 * 32 ? 3 : 2; };
+    // 44 us in 934 chunks of 68 rows, 58 in 1,984 of 32), so there 64 rows.  Fewer than
+    // 64 rows are one chunk: tiles of 32, whose chain is shorter, where there is a SIMD
+    // for each (63 rows, 96 x 96: 33 us with tiles of 48, 27 with tiles of 32)
+    const bool narrow = n < 64 && (long long)((na + 31) / 32) * ((nx + 31) / 32) <= 1024;
+    auto pick = [&](int m) { return !narrow && (m + 47) / 48 * 48 <= (m + 31) / 32 * 32 ? 3 : 2; };
     const int ba = pick(na), bx = pick(nx);
     const int ta = (na + 16 * ba - 1) / (16 * ba), tx = (nx + 16 * bx - 1) / (16 * bx);
     const size_t tot = (size_t)na * nx;
@@ -1091,8 +1094,10 @@ void launch_tgemm(const cd *mat, const cd *X, long long n, int na, int nx, cd *T
     nz = (n + chunk - 1) / chunk;
     const dim3 grid((unsigned)(ta * tx * nz));
     auto kern = ba == 3 ? (bx == 3 ? &k_tgemm<3, 3> : &k_tgemm<3, 2>) : (bx == 3 ? &k_tgemm<2, 3> : &k_tgemm<2, 2>);
-    hipLaunchKernelGGL(kern, grid, dim3(64), 0, s, mat, X, n, na, nx, ta, tx, chunk, work);
+    // a single chunk (few rows or a wide T) is the result itself
+    hipLaunchKernelGGL(kern, grid, dim3(64), 0, s, mat, X, n, na, nx, ta, tx, chunk, nz == 1 ? T : work);
     HIP_CHECK(hipGetLastError());
+    if (nz == 1) return;
     hipLaunchKernelGGL(k_tgemm_reduce, dim3((unsigned)((tot + 15) / 16)), dim3(256), 0, s, work, (int)nz, tot, T);
     HIP_CHECK(hipGetLastError());
 }

@@ -110,3 +110,10 @@ def test_project_shapes(n, na, nx):
 @pytest.mark.parametrize('n,na,nx', [(16384, 5, 3), (32768, 4, 7)])
 def test_project_whole_chunks(n, na, nx):
     test_project_shapes(n, na, nx)
+
+
+# one chunk of rows, whose products are the result itself: tiles of both sizes, fewer
+# than four rows and a remainder
+@pytest.mark.parametrize('n,na,nx', [(63, 65, 129), (50, 70, 33), (3, 31, 140)])
+def test_project_one_chunk(n, na, nx):
+    test_project_shapes(n, na, nx)
