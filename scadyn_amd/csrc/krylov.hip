@@ -1080,7 +1080,7 @@ void launch_tgemm(const cd *mat, const cd *X, long long n, int na, int nx, cd *T
     // sum of the parts costs more than the shorter chains give (63,487 rows, 8 x 14:
     // 44 us in 934 chunks of 68 rows, 58 in 1,984 of 32), so there 64 rows.  Fewer than
     // 64 rows are one chunk: tiles of 32, whose chain is shorter, where there is a SIMD
-    // for each (63 rows, 96 x 96: 33 us with tiles of 48, 27 with tiles of 32)
+    // for each (63 rows, 96 x 96: 33 us with tiles of 48, 23 with tiles of 32)
     const bool narrow = n < 64 && (long long)((na + 31) / 32) * ((nx + 31) / 32) <= 1024;
     auto pick = [&](int m) { return !narrow && (m + 47) / 48 * 48 <= (m + 31) / 32 * 32 ? 3 : 2; };
     const int ba = pick(na), bx = pick(nx);

@@ -553,11 +553,30 @@ __global__ __launch_bounds__(64, 3) void k_gather_mf(gcore::GatherArgs<cf> g) {
 //    have a row, and five of eight lanes a slot); on large meshes one thread per slot
 //    is faster (5 slots: 24.7 k 179 us in groups, 179 by threads; 98 k 814 and 728;
 //    201 k 1,536 and 1,357; 8 slots: 98 k 825 and 815; 201 k 1,557 and 1,498).
+//  * Few rows to a group (fine grids, bodies of many half-empty cubes; the default grid
+//    has five to six): a group costs about the same whatever its rows, so there one
+//    thread per (row, slot) wins, the wider the batch the fewer rows it takes.
+//    43,248 tets, us in groups and by threads: 2.0 rows a group complex128 3 slots 295
+//    and 125, 12 431 and 254, 24 654 and 475; complex64 5 slots 374 and 134, 12 400 and
+//    208, 24 400 and 382; 3.3 rows complex128 5 slots 278 and 260, 8 306 and 351, 17 641
+//    and 525; complex64 5 349 and 221, 12 369 and 329, 16 399 and 430; 55,968 tets, 3.9
+//    rows complex64 5 521 and 368, 9 534 and 489; 103,536 tets, 4.3 rows 8 939 and 822.
+//    Small meshes leave lanes idle either way (5,472 tets, 2 rows, 12 slots 72 and 76).
 //  * Else row groups.
 enum GatherKernel { GATHER_NARROW, GATHER_FLAT, GATHER_GROUPS };
+static bool few_rows(bool wide, int B, int N, int groups) {
+    const double rows = (double)N / std::max(groups, 1);
+    if (B >= 32) return false;
+    if (N < 8192) return wide && B > 16 && rows < 2.5;
+    if (!wide) return B >= 5 && B <= (rows < 2.5 ? 24 : rows < 3.5 ? 12 : rows < 4.0 ? 9 : rows < 4.5 ? 8 : 0);
+    int lanes = 4;
+    while (lanes < B) lanes *= 2;
+    return rows < 2.5 || (rows < 3.5 && B >= 3 && (lanes == 4 || 4 * B <= 3 * lanes));
+}
 template <typename C>
-static GatherKernel pick_gather(int B, int N) {
+static GatherKernel pick_gather(int B, int N, int groups) {
     const bool wide = sizeof(C) == 16;
+    if (few_rows(wide, B, N, groups)) return GATHER_FLAT;
     if (B <= 4) return wide && N >= 8192 ? GATHER_GROUPS : GATHER_NARROW;
     if (!wide && B <= 8 && N >= (B <= 6 ? 1 << 16 : 3 << 16)) return GATHER_FLAT;
     return GATHER_GROUPS;
@@ -619,7 +638,7 @@ void launch_scatter(const MatvecArgs<C> &a, hipStream_t s) {
 
 template <typename C>
 void launch_gather_near(const MatvecArgs<C> &a, hipStream_t s) {
-    const GatherKernel kern = pick_gather<C>(a.B, a.N);
+    const GatherKernel kern = pick_gather<C>(a.B, a.N, a.n_groups);
     if (kern == GATHER_NARROW) {
         narrow_slots(a.B, [&](auto sb) {
             constexpr int SB = decltype(sb)::value;
@@ -631,14 +650,13 @@ void launch_gather_near(const MatvecArgs<C> &a, hipStream_t s) {
         HIP_CHECK(hipGetLastError());
         return;
     }
-    if constexpr (std::is_same<C, cf>::value)
-        if (kern == GATHER_FLAT) {
-            hipLaunchKernelGGL((k_gather_flat<C>), dim3(grid_for((long long)a.N * a.B, 256)), dim3(256), 0, s,
-                               a.grid_out, a.xin, a.in_off, a.B, a.N, a.tet_cube, a.S4, a.Nx, a.Ny, a.ncx, a.ncy,
-                               a.row_start, a.ent_col, a.ent_blk, a.blocks, a.k2, a.slot_active, a.y);
-            HIP_CHECK(hipGetLastError());
-            return;
-        }
+    if (kern == GATHER_FLAT) {
+        hipLaunchKernelGGL((k_gather_flat<C>), dim3(grid_for((long long)a.N * a.B, 256)), dim3(256), 0, s, a.grid_out,
+                           a.xin, a.in_off, a.B, a.N, a.tet_cube, a.S4, a.Nx, a.Ny, a.ncx, a.ncy, a.row_start,
+                           a.ent_col, a.ent_blk, a.blocks, a.k2, a.slot_active, a.y);
+        HIP_CHECK(hipGetLastError());
+        return;
+    }
     gcore::GatherArgs<C> g = {a.grid_out, a.xin,     a.in_off,    a.B,      a.ne_cubes,
                                     a.n_ne,     a.cube_start, a.S4,      a.Nx,     a.Ny,
                                     a.ncx,      a.ncy,       a.ncz,       a.row_start, a.ent_blk,
