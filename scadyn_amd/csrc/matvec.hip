@@ -604,7 +604,7 @@ void launch_scatter(const MatvecArgs<C> &a, hipStream_t s) {
     const long long nodes = (long long)a.Nx * a.Ny * a.Nz;
     const score::ScatterArgs<C> sa = {a.xin, a.in_off, a.B,   a.cube_start, a.S4,  a.Nx,
                                       a.Ny,  a.Nz,     a.ncx, a.ncy,        a.ncz, a.grid_in};
-    const score::Kernel kern = score::pick_kernel(a.B, nodes);
+    const score::Kernel kern = score::pick_kernel(a.B, nodes, a.Nx);
     if (kern == score::BLOCKS) {
         const long long nw = (long long)((a.Nx + 1) / 2) * ((a.Ny + 1) / 2) * ((a.Nz + 1) / 2) * ((a.B + 63) / 64);
         hipLaunchKernelGGL((k_scatter_blk_w64<C>), dim3(grid_for(nw, 4)), dim3(256), 0, s, a.xin, a.in_off, a.B,

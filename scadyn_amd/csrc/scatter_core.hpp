@@ -46,9 +46,16 @@ constexpr int nodes_per_group() {
 //   20 slots: 2 groups, 149 k 207, 614 k 942; thread per slot 200 and 840
 //   24 slots: 2 groups, 149 k 208, 360 k 508, 614 k 981; thread per slot 219, 547, 922
 //   25 slots: 64-slot chunk, 149 k 193; thread per slot 235
+// Lines of a multiple of 32 nodes: the narrow kernel's workgroups of 8 or 16 nodes, and
+// with them the eight XCDs, keep their place along x from line to line, so that some get
+// only the ends of the lines, where a body has few tets.  A thread per (node, slot) does
+// not where the width is no power of two.  64 x 64 x 64 nodes, us narrow and by threads:
+// 3 slots 137 and 114, 5 227 and 148, 7 233 and 183, 12 430 and 234, 24 649 and 412
+// 32 x 32 x 32, 5 slots 32 and 28, 12 48 and 34, 24 75 and 63.
 enum Kernel { NARROW, FLAT, BLOCKS };
-inline Kernel pick_kernel(int B, long long nodes) {
+inline Kernel pick_kernel(int B, long long nodes, int Nx) {
     if (B > 24) return BLOCKS;
+    if (Nx % 32 == 0 && nodes >= 1LL << 15 && B >= 3 && (B & (B - 1)) != 0) return FLAT;
     if (nodes >= 1LL << 17 && (B == 9 || B == 10 || (B >= 17 && B <= 20))) return FLAT;
     if (nodes >= 3LL << 17 && (B == 5 || B == 11 || B == 12 || (B >= 21 && B <= 24))) return FLAT;
     return NARROW;

@@ -38,3 +38,22 @@ def test_scatter_widths(gap, lo, hi):
             assert rel(y[r], one[r]) < 1e-13
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize('n_cells,nx', [(14, 32), (30, 64)])
+def test_scatter_widths_on_lines_of_a_multiple_of_32(n_cells, nx):
+    """The same on a body whose lines have 32 or 64 nodes."""
+    from helpers import sphere_case
+    from scadyn_amd import native
+    case = sphere_case(n_cells=n_cells)
+    a = native.Operator(*case)
+    assert a.info()['Nx'] == nx
+    print(f'[scatter-rule] {nx} nodes along x', flush=True)
+    x = np.random.default_rng(5).standard_normal((2, 25, 3 * case[1].shape[0]))
+    x = x[0] + 1j * x[1]
+    one = np.concatenate([a.matvec(x[r:r + 1]) for r in range(25)])
+    for wide in (2, 3, 4, 5, 7, 8, 11, 12, 15, 16, 23, 24, 25):
+        y = a.matvec(x[:wide])
+        for r in range(wide):
+            assert rel(y[r], one[r]) < 1e-13
+    a.close()
