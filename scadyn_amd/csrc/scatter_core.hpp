@@ -48,9 +48,10 @@ constexpr int nodes_per_group() {
 //   25 slots: 64-slot chunk, 149 k 193; thread per slot 235
 // Lines of a multiple of 32 nodes: the narrow kernel's workgroups of 8 or 16 nodes, and
 // with them the eight XCDs, keep their place along x from line to line, so that some get
-// only the ends of the lines, where a body has few tets.  A thread per (node, slot) does
-// not where the width is no power of two.  64 x 64 x 64 nodes, us narrow and by threads:
-// 3 slots 137 and 114, 5 227 and 148, 7 233 and 183, 12 430 and 234, 24 649 and 412
+// only the ends of the lines, where a body has few tets (shifting them by one a turn
+// took 12 slots below from 430 to 338 us).  A thread per (node, slot) does not where the
+// width is no power of two.  64 x 64 x 64 nodes, complex128, us narrow and by threads:
+// 3 slots 137 and 114, 5 227 and 148, 7 233 and 183, 12 430 and 234, 24 649 and 412;
 // 32 x 32 x 32, 5 slots 32 and 28, 12 48 and 34, 24 75 and 63.
 enum Kernel { NARROW, FLAT, BLOCKS };
 inline Kernel pick_kernel(int B, long long nodes, int Nx) {
